@@ -15,6 +15,7 @@
 
 #include "drr_internal.h"
 #include "epilogue.h"
+#include "fast_march.h"
 #include "jobs.h"
 #include "march.h"
 
@@ -220,7 +221,7 @@ struct drr_batch_s {
 };
 
 template <int M, bool ATTEN, int TW, bool FAST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MarchOcc<M + (ATTEN ? 1 : 0)>::waves)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FAST ? FAST_WAVES : MarchOcc<M + (ATTEN ? 1 : 0)>::waves)))
 void k_batch_march(const JobDev *__restrict__ jobs, const VolDev *__restrict__ vols,
                    const int2 *__restrict__ items, const int *__restrict__ seg, int *counters,
                    SpectrumDev sp, float step, int air, float *__restrict__ I, float *__restrict__ P,
@@ -228,7 +229,12 @@ void k_batch_march(const JobDev *__restrict__ jobs, const VolDev *__restrict__ v
     for_each_tile<TW>(jobs, items, seg, counters, [&](int, const JobDev &J, int udx, int vdx, bool valid) {
         if (!valid) return;
         float ad[M];
-        march_v1<M, ATTEN, FAST>(J.g, vols[J.vol], udx, vdx, step, air, ad);
+        if constexpr (FAST) {
+            __shared__ float acc[M * FAST_LANES];  // each thread its own words
+            march_fast<M, ATTEN>(J.g, vols[J.vol], udx, vdx, step, air, acc + threadIdx.x, ad);
+        } else {
+            march_v1<M, ATTEN>(J.g, vols[J.vol], udx, vdx, step, air, ad);
+        }
         float inten, pp;
         spectral<M>(sp, ad, inten, pp);
         const int64_t pix = (int64_t)vdx * J.g.width + udx;

@@ -168,7 +168,11 @@ __host__ __device__ __forceinline__ uint32_t cell_index_biased(const VolDev &v, 
     const float e2 = __builtin_fmaf(cy, v.b2, cx + v.c2);
     uint32_t bits;
     __builtin_memcpy(&bits, &e2, 4);
+#ifdef __HIP_DEVICE_COMPILE__
+    return __umul24((uint32_t)e1, v.s1) + bits;  // both below 2^24: a full-rate multiply-add
+#else
     return (uint32_t)e1 * v.s1 + bits;
+#endif
 }
 
 inline VolDev vol_to_dev(const drr_volume *v) {

@@ -1,0 +1,348 @@
+// fast_march.h -- the fast single-volume march (DRR_MARCH_FAST), shared by the
+// plain and batched kernels.
+//
+// The samples are those of the exact march (march.h): the same FP32 sequence
+// `alpha += step`, weight 1 except for the ends of the ray; what differs is how
+// their densities are formed and added, so values differ from the exact
+// march's by rounding.  The ray is taken cell by cell.
+//
+// * Along the ray the trilinear density of a cell is a cubic in the distance u
+//   from the middle of the cell's samples, formed from the 8 corner densities,
+//   the fractions there and the ray direction.  The samples sit at u = k inc
+//   about that middle (inc: alpha's exact increment, march.h), so the odd
+//   powers cancel and their sum is n c0 + c2 sum(u^2): a cell costs about 90
+//   vector instructions whatever its number of samples.
+// * The reference adds the samples one by one in FP32, and in a long sum those
+//   roundings are as large as the 1e-5 the fast march promises to stay within
+//   of them (4e-5 on the clinical view where every cell is summed at once).
+//   So a material whose running sum has passed FAST_CLOSED_SUM is added sample
+//   by sample again.  A cell of constant density is the exception: its samples
+//   all round the same way when they are added, so n times what one adds is
+//   what the reference adds, at any size of the sum.
+// * A cell with two labels (nearly every cell on a material boundary) splits
+//   the density by the second label's fraction f, also a cubic: the sum of
+//   density x f has the even moments up to u^6, about the mean of the samples'
+//   FP32 positions, where the exact filter places them (across a metal
+//   boundary the density changes by several g/cm^3 per voxel, and the
+//   positions' rounding shows in the images).  Where a sum is long, each
+//   sample's density and fraction are formed by nested lerps at its position.
+// * A cell with three or more labels takes the exact filter's formulas.
+//
+// Every lane enters its next cell together with the others (one execution of
+// the entry block for the wave); lanes that add one by one do so in loops of
+// their own afterwards.  The materials' sums live in LDS, one word per lane and
+// material: an entry reads and writes the words its labels name, which in
+// registers takes a compare and a select per material and holds the
+// materials' registers and lane masks through the loop.  Nothing depends on
+// the launch or on other lanes, so results are the same from run to run and
+// from kernel to kernel.
+#pragma once
+
+#include "march.h"
+
+namespace drr {
+
+// Running sum (density x step, mm g/cm^3) up to which cells are summed at once:
+// images of clinical views are then within 7.8e-6 of the exact march's (6.4e-6
+// with every sample added singly, 1.2e-5 at 128), at 17.5 ms for 48 mixed views
+// against 24.2 singly.
+constexpr float FAST_CLOSED_SUM = 102.4f;
+// Waves per SIMD of the kernels that march fast: 80 registers hold the entry
+// block (at 8 waves' 64 it spills: 6.1 ms against 5.6 on the clinical view; 7
+// waves: 5.8).
+constexpr int FAST_WAVES = 6;
+
+// Threads per block of the kernels that march fast: the stride of a thread's
+// words in its LDS sums (consecutive lanes in consecutive banks).
+constexpr int FAST_LANES = 256;
+
+// A trilinear interpolant along the ray p(u) = p_m + u r as a cubic in u:
+// value(u) = ((c3 u + c2) u + c1) u + c0, from the lerps along x of the corner
+// pairs (0yz, 1yz) (first corners vYZ, differences xYZ) and the fractions f of
+// p_m against the cell.
+struct Cubic {
+    float c0, c1, c2, c3;
+};
+__device__ __forceinline__ Cubic cell_cubic(float v00, float x00, float v10, float x10, float v01, float x01,
+                                            float v11, float x11, float fx, float fy, float fz, float rx, float ry,
+                                            float rz) {
+    // x: e_yz(u) = A_yz + B_yz u
+    const float A00 = __builtin_fmaf(fx, x00, v00), A10 = __builtin_fmaf(fx, x10, v10);
+    const float A01 = __builtin_fmaf(fx, x01, v01), A11 = __builtin_fmaf(fx, x11, v11);
+    const float B00 = rx * x00, B10 = rx * x10, B01 = rx * x01, B11 = rx * x11;
+    // y: g_z(u) = G_z0 + G_z1 u + G_z2 u^2
+    const float P0 = A10 - A00, Q0 = B10 - B00, P1 = A11 - A01, Q1 = B11 - B01;
+    const float G00 = __builtin_fmaf(fy, P0, A00), G01 = __builtin_fmaf(fy, Q0, __builtin_fmaf(ry, P0, B00));
+    const float G02 = ry * Q0;
+    const float G10 = __builtin_fmaf(fy, P1, A01), G11 = __builtin_fmaf(fy, Q1, __builtin_fmaf(ry, P1, B01));
+    const float G12 = ry * Q1;
+    // z: the cubic
+    const float D0 = G10 - G00, D1 = G11 - G01, D2 = G12 - G02;
+    Cubic k;
+    k.c0 = __builtin_fmaf(fz, D0, G00);
+    k.c1 = __builtin_fmaf(fz, D1, __builtin_fmaf(rz, D0, G01));
+    k.c2 = __builtin_fmaf(fz, D2, __builtin_fmaf(rz, D1, G02));
+    k.c3 = rz * D2;
+    return k;
+}
+
+// Bit 3 of nibble d is set where nibble d of x is nonzero (exact per nibble:
+// the low three bits plus 7 carry into bit 3 and never into the next nibble).
+__device__ __forceinline__ uint32_t nz_nibbles(uint32_t x) {
+    return (((x & 0x77777777u) + 0x77777777u) | x) & 0x88888888u;
+}
+
+// Two-label cells: the corners' indicators of the second label as lerps along x
+// (first corners vYZ, differences xYZ), 0 or 1 and 0 or +-1.
+struct Second {
+    float v00, v10, v01, v11, x00, x10, x01, x11;
+};
+
+// One sample of weight wt by the exact filter's formulas, added to the sums.
+template <int M>
+__device__ __forceinline__ void fast_sample(const Cell &c, float *acc, float fx, float fy, float fz, float wt) {
+    float w[8];
+    weights8(fx, fy, fz, w);
+    const float x = wt * trilerp(c.d0, c.d1, w);
+#pragma unroll 1
+    for (int m = 0; m < M; m++) {
+        const uint32_t xm = c.l0 ^ (0x11111111u * (uint32_t)m);
+        if (((xm - 0x11111111u) & ~xm & 0x88888888u) == 0u) continue;  // no corner has it
+        float sm = 0.0f;
+#pragma unroll
+        for (int d = 0; d < 8; d++) sm += (corner_label(c.l0, c.l1, d) == (uint32_t)m) ? w[d] : 0.0f;
+        acc[FAST_LANES * m] = __builtin_fmaf(x, sm, acc[FAST_LANES * m]);
+    }
+}
+
+// The samples t in [t, tlim) of a stretch over which alpha moves by inc, all of
+// weight 1.  acut: FAST_CLOSED_SUM in units of the sums.
+template <int M>
+__device__ __forceinline__ void fast_run(const VolDev &vol, float *acc, float sx, float sy, float sz, float rix,
+                                         float riy, float riz, float step, float inc, float acut, float alpha, int t,
+                                         int tlim) {
+    // exit distances in steps (reciprocals to 1 ulp are plenty there): per axis
+    // the exit face is reached after fma(-f, j, h) steps with j = 1 / (r inc)
+    // and h = j going up, 0 going down (j = 0, h = +inf where r = 0).  They stay
+    // in registers (an empty asm stops the compiler from forming them again on
+    // every entry).  Where alpha does not move every entry takes one sample.
+    const float iinc = inc > 0.0f ? 1.0f / inc : 0.0f;
+    float jx = rix == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(rix) * iinc;
+    float jy = riy == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(riy) * iinc;
+    float jz = riz == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(riz) * iinc;
+    const float hno = inc > 0.0f ? INFINITY : 0.0f;
+    float hx = rix == 0.0f ? hno : (rix < 0.0f ? 0.0f : jx);
+    float hy = riy == 0.0f ? hno : (riy < 0.0f ? 0.0f : jy);
+    float hz = riz == 0.0f ? hno : (riz < 0.0f ? 0.0f : jz);
+    asm volatile("" : "+v"(jx), "+v"(jy), "+v"(jz), "+v"(hx), "+v"(hy), "+v"(hz));
+    const float inc2_12 = inc * inc * (1.0f / 12.0f);
+    while (t < tlim) {
+        const float alpha0 = alpha;
+        const float px = sample_pos(sx, alpha, rix), py = sample_pos(sy, alpha, riy), pz = sample_pos(sz, alpha, riz);
+        const float bx = floorf(px), by = floorf(py), bz = floorf(pz);
+        Cell c;
+        c.load(vol, bx, by, bz);
+        const float fx = px - bx, fy = py - by, fz = pz - bz;
+        const float nex =
+            fminf(__builtin_fmaf(-fx, jx, hx), fminf(__builtin_fmaf(-fy, jy, hy), __builtin_fmaf(-fz, jz, hz)));
+        // the samples before the exit face, clamped to [1, tlim - t] after the
+        // conversion (which saturates infinities and takes NaN to 0), so every
+        // entry takes at least one sample; one within rounding of the face may
+        // fall to either cell (the density is continuous)
+        int n = min(max((int)ceilf(nex), 1), tlim - t);
+        t += n;
+        const float nf = (float)n;
+        const float um = inc * __builtin_fmaf(0.5f, nf, -0.5f);  // from the entry sample to the middle
+        alpha = __builtin_fmaf(nf, inc, alpha);
+        const float mx = __builtin_fmaf(rix, um, fx), my = __builtin_fmaf(riy, um, fy), mz = __builtin_fmaf(riz, um, fz);
+        // sum of u^2 over the samples
+        const float S2 = inc2_12 * (nf * __builtin_fmaf(nf, nf, -1.0f));
+        const uint32_t l0 = c.l0, la = l0 & 0xfu;
+        float *pa = acc + FAST_LANES * la, *pb = acc;  // sums of the first and second label
+        float cur = *pa, sq = 0.0f;
+        Cubic fc = cell_cubic(c.d0.x, c.d0.y - c.d0.x, c.d0.z, c.d0.w - c.d0.z, c.d1.x, c.d1.y - c.d1.x, c.d1.z,
+                              c.d1.w - c.d1.z, mx, my, mz, rix, riy, riz);
+        bool one = true;  // the samples are to be added one by one
+        bool tw = false, ex = false;  // two labels; three or more
+        Second e;
+        if (c.uni) {
+            const bool flat = (fc.c1 == 0.0f) & (fc.c2 == 0.0f);
+            const float mean = flat ? (cur + fc.c0) - cur : fc.c0;
+            one = !(flat | (cur < acut));
+            if (!one) *pa = cur + __builtin_fmaf(fc.c2, S2, nf * mean);
+        } else {
+            const uint32_t xa = l0 ^ (la * 0x11111111u);  // nonzero nibbles: corners not la
+            const uint32_t lb = (l0 >> (__builtin_ctz(xa) & ~3u)) & 0xfu;
+            const uint32_t xb = l0 ^ (lb * 0x11111111u);
+            const uint32_t na = nz_nibbles(xa), nb = nz_nibbles(xb);  // nb bit set: corner not lb
+            tw = (na & nb) == 0u;
+            ex = !tw;
+            pb = acc + FAST_LANES * lb;
+            sq = *pb;
+            e.v00 = (nb & 0x8u) ? 0.f : 1.f;
+            e.v10 = (nb & 0x800u) ? 0.f : 1.f;
+            e.v01 = (nb & 0x80000u) ? 0.f : 1.f;
+            e.v11 = (nb & 0x8000000u) ? 0.f : 1.f;
+            e.x00 = ((nb & 0x80u) ? 0.f : 1.f) - e.v00;
+            e.x10 = ((nb & 0x8000u) ? 0.f : 1.f) - e.v10;
+            e.x01 = ((nb & 0x800000u) ? 0.f : 1.f) - e.v01;
+            e.x11 = ((nb & 0x80000000u) ? 0.f : 1.f) - e.v11;
+            if (tw & (fmaxf(cur, sq) < acut)) {
+                // The middle's fractions as the mean of the samples' FP32
+                // positions: the exact filter's positions round with the same
+                // sign over many samples, which along a boundary adds up (with
+                // the entry's alone, oblique clinical views came to 2e-5 of the
+                // exact march's, with three samples' to 1.2e-5).
+                float qx = 0.0f, qy = 0.0f, qz = 0.0f, al = alpha0;
+                for (int k = 0;; k += 2) {
+                    const bool in = k < n;
+                    if (__ballot(in) == 0) break;
+                    const float g = in ? 1.0f : 0.0f, g1 = k + 1 < n ? 1.0f : 0.0f, al1 = al + inc;
+                    qx = __builtin_fmaf(g, __builtin_fmaf(al, rix, sx) - (bx + 1.0f), qx);
+                    qy = __builtin_fmaf(g, __builtin_fmaf(al, riy, sy) - (by + 1.0f), qy);
+                    qz = __builtin_fmaf(g, __builtin_fmaf(al, riz, sz) - (bz + 1.0f), qz);
+                    qx = __builtin_fmaf(g1, __builtin_fmaf(al1, rix, sx) - (bx + 1.0f), qx);
+                    qy = __builtin_fmaf(g1, __builtin_fmaf(al1, riy, sy) - (by + 1.0f), qy);
+                    qz = __builtin_fmaf(g1, __builtin_fmaf(al1, riz, sz) - (bz + 1.0f), qz);
+                    al = al1 + inc;
+                }
+                const float rn = __builtin_amdgcn_rcpf(nf);
+                qx *= rn;
+                qy *= rn;
+                qz *= rn;
+                const Cubic g = cell_cubic(e.v00, e.x00, e.v10, e.x10, e.v01, e.x01, e.v11, e.x11, qx, qy, qz, rix,
+                                           riy, riz);
+                fc = cell_cubic(c.d0.x, c.d0.y - c.d0.x, c.d0.z, c.d0.w - c.d0.z, c.d1.x, c.d1.y - c.d1.x, c.d1.z,
+                                c.d1.w - c.d1.z, qx, qy, qz, rix, riy, riz);
+                const float S4 = S2 * (inc2_12 * 0.6f) * __builtin_fmaf(3.0f * nf, nf, -7.0f);
+                const float S6 = S2 * (inc2_12 * inc2_12 * (9.0f / 7.0f)) *
+                                 __builtin_fmaf(nf * nf, __builtin_fmaf(3.0f * nf, nf, -18.0f), 31.0f);
+                const float p2 = __builtin_fmaf(fc.c0, g.c2, __builtin_fmaf(fc.c1, g.c1, fc.c2 * g.c0));
+                const float p4 = __builtin_fmaf(fc.c1, g.c3, __builtin_fmaf(fc.c2, g.c2, fc.c3 * g.c1));
+                const float sum_q = __builtin_fmaf(
+                    nf, fc.c0 * g.c0, __builtin_fmaf(S2, p2, __builtin_fmaf(S4, p4, S6 * (fc.c3 * g.c3))));
+                *pb = sq + sum_q;
+                *pa = cur + (__builtin_fmaf(fc.c2, S2, nf * fc.c0) - sum_q);
+                one = false;
+            }
+        }
+        if (__ballot(one) == 0) continue;
+        if (!one) n = 0;
+        tw = tw & one;
+        if (ex) fc = Cubic{0.0f, 0.0f, 0.0f, 0.0f};
+        // the samples that are added one by one.  The loops' tests are wave votes
+        // and their per-lane choices 0/1 factors: per-lane branches cost scalar
+        // instructions, enough to become the limit in loops this short.
+        if (__ballot(tw) != 0) {
+            // two labels: density and second fraction at the sample's FP32
+            // position, each by nested lerps; the other lanes' cubics beside them
+            float al = alpha0, u = -um;
+            for (int k = 0;; ++k) {
+                const bool in = k < n;
+                if (__ballot(in) == 0) break;
+                const float g = in ? 1.0f : 0.0f;
+                float rho = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(fc.c3, u, fc.c2), u, fc.c1), u, fc.c0);
+                const float fx = __builtin_fmaf(al, rix, sx) - (c.bx + 1.0f);
+                const float fy = __builtin_fmaf(al, riy, sy) - (c.by + 1.0f);
+                const float fz = __builtin_fmaf(al, riz, sz) - (c.bz + 1.0f);
+                const float a00 = __builtin_fmaf(fx, c.d0.y - c.d0.x, c.d0.x);
+                const float a10 = __builtin_fmaf(fx, c.d0.w - c.d0.z, c.d0.z);
+                const float a01 = __builtin_fmaf(fx, c.d1.y - c.d1.x, c.d1.x);
+                const float a11 = __builtin_fmaf(fx, c.d1.w - c.d1.z, c.d1.z);
+                const float b0 = __builtin_fmaf(fy, a10 - a00, a00), b1 = __builtin_fmaf(fy, a11 - a01, a01);
+                const float x = __builtin_fmaf(fz, b1 - b0, b0);
+                const float i00 = __builtin_fmaf(fx, e.x00, e.v00), i10 = __builtin_fmaf(fx, e.x10, e.v10);
+                const float i01 = __builtin_fmaf(fx, e.x01, e.v01), i11 = __builtin_fmaf(fx, e.x11, e.v11);
+                const float j0 = __builtin_fmaf(fy, i10 - i00, i00), j1 = __builtin_fmaf(fy, i11 - i01, i01);
+                const float fq = __builtin_fmaf(fz, j1 - j0, j0);
+                const float xq = x * fq;
+                sq = __builtin_fmaf(g, tw ? xq : 0.0f, sq);
+                rho = tw ? x - xq : rho;
+                cur = __builtin_fmaf(g, rho, cur);
+                al = __builtin_fmaf(g, step, al);
+                u += inc;
+            }
+            if (tw) *pb = sq;
+        } else {
+            float u = -um;
+            for (int k = 0;; ++k) {
+                const bool in = k < n;
+                if (__ballot(in) == 0) break;
+                const float rho = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(fc.c3, u, fc.c2), u, fc.c1), u, fc.c0);
+                cur = __builtin_fmaf(in ? 1.0f : 0.0f, rho, cur);
+                u += inc;
+            }
+        }
+        if (one & !ex) *pa = cur;
+        if (__ballot(ex) != 0) {
+            float al = alpha0;
+            for (int k = 0; __ballot((k < n) & ex) != 0; ++k) {
+                if ((k < n) & ex)
+                    fast_sample<M>(c, acc, __builtin_fmaf(al, rix, sx) - (c.bx + 1.0f),
+                                   __builtin_fmaf(al, riy, sy) - (c.by + 1.0f),
+                                   __builtin_fmaf(al, riz, sz) - (c.bz + 1.0f), 1.0f);
+                al += step;
+            }
+        }
+    }
+}
+
+// The single-volume march (project_kernel.cu:334-584 with NUM_VOLUMES == 1).
+// acc: this thread's sums in LDS, material m at acc[FAST_LANES * m].  On return
+// ad[] holds the final area densities in g/cm^2.
+template <int M, bool ATTEN>
+__device__ __forceinline__ void march_fast(const Geo1 &g, const VolDev &vol, int udx, int vdx, float step, int air,
+                                           float *acc, float (&ad)[M]) {
+    RayV1 r;
+    march_setup_v1(g, udx, vdx, step, r);
+    for (int m = 0; m < M; m++) acc[FAST_LANES * m] = 0.0f;
+    float air_sum = 0.0f;
+    if (ATTEN) air_sum = (float)((double)air_sum + (double)(r.minA / step) * DRR_AIR_DENSITY);
+    const int N = r.N;
+    float alpha = r.minA;
+    int t = 0;
+    if (r.trace) {
+        const float sx = g.s[0], sy = g.s[1], sz = g.s[2];
+        const float rix = r.ri[0], riy = r.ri[1], riz = r.ri[2];
+        skip_steps(N, r.mnv, step, alpha, t);
+        if (ATTEN) {
+            air_steps(t, air_sum);
+            acc[FAST_LANES * air] = air_sum;
+        }
+        // Stretches over which alpha is an exact arithmetic progression (march.h),
+        // ending at the volume's exit or the binade's top; anything else one
+        // sample at a time.
+        const float acut = FAST_CLOSED_SUM / step;
+        while (alpha <= r.mxv && t < N) {
+            if (t == 0 || t == N - 1) {  // weight 0.5
+                const float px = sample_pos(sx, alpha, rix), py = sample_pos(sy, alpha, riy),
+                            pz = sample_pos(sz, alpha, riz);
+                Cell c;
+                c.load(vol, floorf(px), floorf(py), floorf(pz));
+                fast_sample<M>(c, acc, px - c.bx, py - c.by, pz - c.bz, 0.5f);
+                alpha += step;
+                ++t;
+                continue;
+            }
+            const float a0 = alpha;
+            float inc;
+            const int m = stretch(a0, step, r.mxv, N - 1 - t, inc);
+            fast_run<M>(vol, acc, sx, sy, sz, rix, riy, riz, step, inc, acut, alpha, t, t + m);
+            t += m;
+            // the addition after the last sample may leave the binade
+            alpha = __builtin_fmaf((float)(m - 1), inc, a0) + step;
+        }
+        if (ATTEN) air_sum = acc[FAST_LANES * air];
+    }
+    if (ATTEN) {
+        air_steps(N - t, air_sum);
+        air_sum = (float)((double)air_sum + (double)((r.L - r.maxA) / step) * DRR_AIR_DENSITY);
+        acc[FAST_LANES * air] = air_sum;
+    }
+#pragma unroll
+    for (int m = 0; m < M; m++) ad[m] = acc[FAST_LANES * m] * step;
+#pragma unroll
+    for (int m = 0; m < M; m++) ad[m] /= 10.0f;
+}
+
+}  // namespace drr

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include "drr_internal.h"
+#include "fast_march.h"
 #include "march.h"
 
 using namespace drr;
@@ -78,7 +79,7 @@ struct OutDev {
 };
 
 template <int M, bool ATTEN, bool FAST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MarchOcc<M>::waves))) void k_project_v1(Geo1 g, VolDev vol, SpectrumDev sp, float step,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FAST ? FAST_WAVES : MarchOcc<M>::waves))) void k_project_v1(Geo1 g, VolDev vol, SpectrumDev sp, float step,
                                                     int air, OutDev out, int tiles16_x) {
     const int lb = blockIdx.x;
     const int bx = lb % tiles16_x, by = lb / tiles16_x;
@@ -87,7 +88,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MarchOcc<M>
     lane_pixel(bx * 2 + (wave & 1), by * 2 + (wave >> 1), lane, udx, vdx);
     if (udx >= g.width || vdx >= g.height) return;
     float ad[M];
-    march_v1<M, ATTEN, FAST>(g, vol, udx, vdx, step, air, ad);
+    if constexpr (FAST) {
+        __shared__ float acc[M * FAST_LANES];  // each thread its own words
+        march_fast<M, ATTEN>(g, vol, udx, vdx, step, air, acc + threadIdx.x, ad);
+    } else {
+        march_v1<M, ATTEN>(g, vol, udx, vdx, step, air, ad);
+    }
     float I, P;
     spectral<M>(sp, ad, I, P);
     const int64_t npix = (int64_t)g.width * g.height;
