@@ -230,8 +230,8 @@ void k_batch_march(const JobDev *__restrict__ jobs, const VolDev *__restrict__ v
         if (!valid) return;
         float ad[M];
         if constexpr (FAST) {
-            __shared__ float acc[M * FAST_LANES];  // each thread its own words
-            march_fast<M, ATTEN>(J.g, vols[J.vol], udx, vdx, step, air, acc + threadIdx.x, ad);
+            __shared__ float sums[M * LDS_LANES];  // each thread its own words
+            march_fast<M, ATTEN>(J.g, vols[J.vol], udx, vdx, step, air, sums + threadIdx.x, ad);
         } else {
             march_v1<M, ATTEN>(J.g, vols[J.vol], udx, vdx, step, air, ad);
         }
@@ -294,7 +294,7 @@ static void launch_march(const JobTable &t, int M, bool atten, bool fast, int tw
 // Jobs over 2..4 volumes: one 8x8-pixel tile per wave, the literal
 // multi-volume march (march_multi, as drr_project runs such a view).
 template <int V, int M>
-__global__ __launch_bounds__(256) void k_batch_multi(const JobMultiDev *__restrict__ jobs, const int2 *__restrict__ items,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI_WAVES))) void k_batch_multi(const JobMultiDev *__restrict__ jobs, const int2 *__restrict__ items,
                                                      int64_t n_items, SpectrumDev sp, float step, int atten, int air,
                                                      float *__restrict__ I, float *__restrict__ P,
                                                      float *__restrict__ AD) {
@@ -309,7 +309,8 @@ __global__ __launch_bounds__(256) void k_batch_multi(const JobMultiDev *__restri
     lane_pixel(tile % J.tiles_x, tile / J.tiles_x, lane, udx, vdx);
     if (udx >= J.vd.width || vdx >= J.vd.height) return;
     float ad[M];
-    march_multi<V, M>(J.vd, udx, vdx, step, atten, air, ad);
+    __shared__ float sums[M * LDS_LANES];  // each thread its own words
+    march_multi<V, M>(J.vd, udx, vdx, step, atten, air, sums + threadIdx.x, ad);
     float inten, pp;
     spectral<M>(sp, ad, inten, pp);
     const int64_t npix = (int64_t)J.vd.width * J.vd.height;

@@ -52,10 +52,6 @@ constexpr float FAST_CLOSED_SUM = 102.4f;
 // waves: 5.8).
 constexpr int FAST_WAVES = 6;
 
-// Threads per block of the kernels that march fast: the stride of a thread's
-// words in its LDS sums (consecutive lanes in consecutive banks).
-constexpr int FAST_LANES = 256;
-
 // A trilinear interpolant along the ray p(u) = p_m + u r as a cubic in u:
 // value(u) = ((c3 u + c2) u + c1) u + c0, from the lerps along x of the corner
 // pairs (0yz, 1yz) (first corners vYZ, differences xYZ) and the fractions f of
@@ -111,7 +107,7 @@ __device__ __forceinline__ void fast_sample(const Cell &c, float *acc, float fx,
         float sm = 0.0f;
 #pragma unroll
         for (int d = 0; d < 8; d++) sm += (corner_label(c.l0, c.l1, d) == (uint32_t)m) ? w[d] : 0.0f;
-        acc[FAST_LANES * m] = __builtin_fmaf(x, sm, acc[FAST_LANES * m]);
+        acc[LDS_LANES * m] = __builtin_fmaf(x, sm, acc[LDS_LANES * m]);
     }
 }
 
@@ -158,7 +154,7 @@ __device__ __forceinline__ void fast_run(const VolDev &vol, float *acc, float sx
         // sum of u^2 over the samples
         const float S2 = inc2_12 * (nf * __builtin_fmaf(nf, nf, -1.0f));
         const uint32_t l0 = c.l0, la = l0 & 0xfu;
-        float *pa = acc + FAST_LANES * la, *pb = acc;  // sums of the first and second label
+        float *pa = acc + LDS_LANES * la, *pb = acc;  // sums of the first and second label
         float cur = *pa, sq = 0.0f;
         Cubic fc = cell_cubic(c.d0.x, c.d0.y - c.d0.x, c.d0.z, c.d0.w - c.d0.z, c.d1.x, c.d1.y - c.d1.x, c.d1.z,
                               c.d1.w - c.d1.z, mx, my, mz, rix, riy, riz);
@@ -177,7 +173,7 @@ __device__ __forceinline__ void fast_run(const VolDev &vol, float *acc, float sx
             const uint32_t na = nz_nibbles(xa), nb = nz_nibbles(xb);  // nb bit set: corner not lb
             tw = (na & nb) == 0u;
             ex = !tw;
-            pb = acc + FAST_LANES * lb;
+            pb = acc + LDS_LANES * lb;
             sq = *pb;
             e.v00 = (nb & 0x8u) ? 0.f : 1.f;
             e.v10 = (nb & 0x800u) ? 0.f : 1.f;
@@ -288,14 +284,14 @@ __device__ __forceinline__ void fast_run(const VolDev &vol, float *acc, float sx
 }
 
 // The single-volume march (project_kernel.cu:334-584 with NUM_VOLUMES == 1).
-// acc: this thread's sums in LDS, material m at acc[FAST_LANES * m].  On return
+// acc: this thread's sums in LDS, material m at acc[LDS_LANES * m].  On return
 // ad[] holds the final area densities in g/cm^2.
 template <int M, bool ATTEN>
 __device__ __forceinline__ void march_fast(const Geo1 &g, const VolDev &vol, int udx, int vdx, float step, int air,
                                            float *acc, float (&ad)[M]) {
     RayV1 r;
     march_setup_v1(g, udx, vdx, step, r);
-    for (int m = 0; m < M; m++) acc[FAST_LANES * m] = 0.0f;
+    for (int m = 0; m < M; m++) acc[LDS_LANES * m] = 0.0f;
     float air_sum = 0.0f;
     if (ATTEN) air_sum = (float)((double)air_sum + (double)(r.minA / step) * DRR_AIR_DENSITY);
     const int N = r.N;
@@ -307,7 +303,7 @@ __device__ __forceinline__ void march_fast(const Geo1 &g, const VolDev &vol, int
         skip_steps(N, r.mnv, step, alpha, t);
         if (ATTEN) {
             air_steps(t, air_sum);
-            acc[FAST_LANES * air] = air_sum;
+            acc[LDS_LANES * air] = air_sum;
         }
         // Stretches over which alpha is an exact arithmetic progression (march.h),
         // ending at the volume's exit or the binade's top; anything else one
@@ -332,15 +328,15 @@ __device__ __forceinline__ void march_fast(const Geo1 &g, const VolDev &vol, int
             // the addition after the last sample may leave the binade
             alpha = __builtin_fmaf((float)(m - 1), inc, a0) + step;
         }
-        if (ATTEN) air_sum = acc[FAST_LANES * air];
+        if (ATTEN) air_sum = acc[LDS_LANES * air];
     }
     if (ATTEN) {
         air_steps(N - t, air_sum);
         air_sum = (float)((double)air_sum + (double)((r.L - r.maxA) / step) * DRR_AIR_DENSITY);
-        acc[FAST_LANES * air] = air_sum;
+        acc[LDS_LANES * air] = air_sum;
     }
 #pragma unroll
-    for (int m = 0; m < M; m++) ad[m] = acc[FAST_LANES * m] * step;
+    for (int m = 0; m < M; m++) ad[m] = acc[LDS_LANES * m] * step;
 #pragma unroll
     for (int m = 0; m < M; m++) ad[m] /= 10.0f;
 }

@@ -89,8 +89,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FAST ? FAST
     if (udx >= g.width || vdx >= g.height) return;
     float ad[M];
     if constexpr (FAST) {
-        __shared__ float acc[M * FAST_LANES];  // each thread its own words
-        march_fast<M, ATTEN>(g, vol, udx, vdx, step, air, acc + threadIdx.x, ad);
+        __shared__ float sums[M * LDS_LANES];  // each thread its own words
+        march_fast<M, ATTEN>(g, vol, udx, vdx, step, air, sums + threadIdx.x, ad);
     } else {
         march_v1<M, ATTEN>(g, vol, udx, vdx, step, air, ad);
     }
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FAST ? FAST
 }
 
 template <int V, int M>
-__global__ __launch_bounds__(256) void k_project_multi(ViewDev vd, SpectrumDev sp, float step,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI_WAVES))) void k_project_multi(ViewDev vd, SpectrumDev sp, float step,
                                                        int atten, int air, OutDev out,
                                                        int tiles16_x) {
     const int lb = blockIdx.x;
@@ -118,7 +118,8 @@ __global__ __launch_bounds__(256) void k_project_multi(ViewDev vd, SpectrumDev s
     lane_pixel(bx * 2 + (wave & 1), by * 2 + (wave >> 1), lane, udx, vdx);
     if (udx >= vd.width || vdx >= vd.height) return;
     float ad[M];
-    march_multi<V, M>(vd, udx, vdx, step, atten, air, ad);
+    __shared__ float sums[M * LDS_LANES];  // each thread its own words
+    march_multi<V, M>(vd, udx, vdx, step, atten, air, sums + threadIdx.x, ad);
     float I, P;
     spectral<M>(sp, ad, I, P);
     const int64_t npix = (int64_t)vd.width * vd.height;

@@ -17,7 +17,7 @@
 //   * for a single volume the steps before the volume are skipped, with the
 //     alpha the same sequential FP32 `alpha += step` (552) reaches
 //     (skip_steps); the label cache needs no step before the first sample (the
-//     labels a fetch returns depend on the cell alone, see fetch_labels);
+//     labels a fetch returns depend on the cell alone, see Cell);
 //   * a cell whose 8 labels agree sums the weights once instead of per
 //     material; a fused multiply-add with a zero fraction leaves an
 //     accumulator unchanged, so the result is bit-identical to the
@@ -84,38 +84,11 @@ __device__ __forceinline__ float sample_pos(float s, float alpha, float r) {
 typedef const __attribute__((address_space(1))) float gfloat;
 typedef const __attribute__((address_space(1))) uint32_t guint;
 
-// Record of cell `cell` (DRR_CELL_WORDS words, drr_internal.h).
-__device__ __forceinline__ guint *cell_record(const VolDev &v, uint32_t cell) {
-    return (guint *)v.cells + DRR_CELL_WORDS * (size_t)cell;
-}
-
 __device__ __forceinline__ int clamp_cell(float b, int n) {
     // cell index in [-1, n-1]; clamp in float (one v_med3_f32) so that huge
     // values stay defined before the conversion
     const float c = __builtin_amdgcn_fmed3f(b, -1.0f, (float)(n - 1));
     return (int)c;
-}
-
-// Cells of one volume are < 2^31 (checked at upload), so 32-bit indices suffice.
-__device__ __forceinline__ uint32_t cell_index(const VolDev &v, int cx, int cy, int cz) {
-    return ((uint32_t)(cz + 1) * (uint32_t)(v.ny + 1) + (uint32_t)(cy + 1)) * (uint32_t)(v.nx + 1) +
-           (uint32_t)(cx + 1);
-}
-
-// Labels of the 8 corners of the sample at p with base b = floor(p): the
-// reference point-samples L[clamp(floor(p + d))] (project_kernel.cu:421-425).
-// Every p the march forms is fl(q - 1) for an FP32 q (sample_pos), and for
-// such p with |p| < 2^22 the sum p + 1 is exact: for q >= 0.5, q - 1 is exact
-// (Sterbenz, and 1 is a multiple of ulp(q) below 2^24), so fl(p + 1) = q; for
-// p <= -0.5, |p| - 1 is a multiple of ulp(p).  Hence floor(p + d) = b + d.
-// For |p| >= 2^22 the sample is over 2^22 - 16384 voxels outside the volume,
-// where b + 1, b + 2 (and b) all clamp to the same edge voxel.  So the labels
-// are always L[clamp(b + d)], which is exactly the cell record of
-// clamp(b, -1, n-1): l0 = corner labels as nibbles, l1 = common label or ~0.
-__device__ __forceinline__ void fetch_labels(const VolDev &v, uint32_t cell, uint32_t &l0, uint32_t &l1) {
-    guint *r = cell_record(v, cell);
-    l0 = r[8];
-    l1 = r[9];
 }
 
 __device__ __forceinline__ void weights8(float fx, float fy, float fz, float w[8]) {
@@ -132,39 +105,6 @@ __device__ __forceinline__ void weights8(float fx, float fy, float fz, float w[8
 
 __device__ __forceinline__ uint32_t corner_label(uint32_t l0, uint32_t, int d) {
     return (l0 >> (4 * d)) & 0xfu;
-}
-
-// seg[m] = sum over corners (dz, dy, dx order) of w[d] where label == m, for a
-// cell whose labels differ.
-template <int M>
-__device__ __forceinline__ void mixed_fractions(uint32_t l0, uint32_t l1, const float w[8], float seg[M]) {
-#pragma unroll
-    for (int m = 0; m < M; m++) {
-        float s = 0.0f;
-#pragma unroll
-        for (int d = 0; d < 8; d++) s += (corner_label(l0, l1, d) == (uint32_t)m) ? w[d] : 0.0f;
-        seg[m] = s;
-    }
-}
-
-// seg[m] = sum over corners (dz, dy, dx order) of w[d] where label == m.
-template <int M>
-__device__ __forceinline__ void material_fractions(uint32_t l0, uint32_t l1, const float w[8],
-                                                   float seg[M]) {
-    const uint32_t m0 = l1;  // the common label, ~0 if the labels differ
-    if (m0 != 0xffffffffu) {
-        const float ssum = ((((((w[0] + w[1]) + w[2]) + w[3]) + w[4]) + w[5]) + w[6]) + w[7];
-#pragma unroll
-        for (int m = 0; m < M; m++) seg[m] = ((uint32_t)m == m0) ? ssum : 0.0f;
-    } else {
-#pragma unroll
-        for (int m = 0; m < M; m++) {
-            float s = 0.0f;
-#pragma unroll
-            for (int d = 0; d < 8; d++) s += (corner_label(l0, l1, d) == (uint32_t)m) ? w[d] : 0.0f;
-            seg[m] = s;
-        }
-    }
 }
 
 // Density at the sample: corner densities weighted by the same exact FP32
@@ -196,6 +136,17 @@ __device__ __forceinline__ void set_m(float (&a)[M], int idx, float val) {
     for (int m = 0; m < M; m++) a[m] = (m == idx) ? val : a[m];
 }
 
+// Labels of the 8 corners of the sample at p with base b = floor(p): the
+// reference point-samples L[clamp(floor(p + d))] (project_kernel.cu:421-425).
+// Every p the march forms is fl(q - 1) for an FP32 q (sample_pos), and for
+// such p with |p| < 2^22 the sum p + 1 is exact: for q >= 0.5, q - 1 is exact
+// (Sterbenz, and 1 is a multiple of ulp(q) below 2^24), so fl(p + 1) = q; for
+// p <= -0.5, |p| - 1 is a multiple of ulp(p).  Hence floor(p + d) = b + d.
+// For |p| >= 2^22 the sample is over 2^22 - 16384 voxels outside the volume,
+// where b + 1, b + 2 (and b) all clamp to the same edge voxel.  So the labels
+// are always L[clamp(b + d)], which is exactly the cell record of
+// clamp(b, -1, n-1): l0 = corner labels as nibbles, l1 = common label or ~0.
+//
 // Cached trilinear cell of the ray: base, 8 labels, 8 densities and whether
 // the labels agree (l1 = their common label).  Before the first load the base
 // is far from any sample (the fractions p - b test as outside [0, 1)).
@@ -340,7 +291,7 @@ __device__ __forceinline__ void march_v1(const Geo1 &g, const VolDev &vol, int u
         const float sx = g.s[0], sy = g.s[1], sz = g.s[2];
         const float rix = r.ri[0], riy = r.ri[1], riz = r.ri[2];
         // Steps before the volume: only the alpha sequence.  The labels a sample
-        // is split by depend on its cell alone (fetch_labels), so the label
+        // is split by depend on its cell alone (Cell), so the label
         // cache needs no steps before the first sample.
         skip_steps(N, r.mnv, step, alpha, t);
         if (ATTEN) air_steps(t, acc);  // one per step so far
@@ -397,130 +348,313 @@ __device__ __forceinline__ void march_v1(const Geo1 &g, const VolDev &vol, int u
     for (int m = 0; m < M; m++) ad[m] /= 10.0f;
 }
 
+// The materials' sums in LDS, one word per thread and material (m at
+// sums[LDS_LANES m] from the thread's first; consecutive lanes in consecutive
+// banks): an access by a label known only at run time is one LDS access, where
+// registers take a compare and a select per material and hold M registers and
+// their masks through the march.
+constexpr int LDS_LANES = 256;  // threads per block of the kernels that use them
+
+// Running sum of the current one-label material of such sums.
+struct LdsAccum {
+    float *sums;
+    float cur = 0.0f;
+    int cm = -1;
+    __device__ __forceinline__ void open(int m) {  // m < 0: none
+        if (m != cm) {
+            if (cm >= 0) sums[LDS_LANES * cm] = cur;
+            cm = m;
+            if (m >= 0) cur = sums[LDS_LANES * m];
+        }
+    }
+};
+
+// Adds x times each label's fraction of the weights w (summed in corner order)
+// to its material's sum, for a cell whose labels differ: label by label of
+// those the corners have (an absent one's fraction is 0 and leaves its sum alone).
+__device__ __forceinline__ void add_mixed(float *sums, uint32_t l0, const float (&w)[8], float x) {
+    uint32_t left = 0x11111111u;  // corners whose label is still to be added
+    do {
+        const uint32_t m = (l0 >> __builtin_ctz(left)) & 0xfu;
+        const uint32_t d0 = l0 ^ (m * 0x11111111u);  // nibble 0: the corner has label m
+        const uint32_t other = (((d0 & 0x77777777u) + 0x77777777u) | d0) >> 3;  // bit 4d set: another label
+        float sm = 0.0f;
+#pragma unroll
+        for (int d = 0; d < 8; d++) sm += ((other >> (4 * d)) & 1u) ? 0.0f : w[d];
+        sums[LDS_LANES * m] = __builtin_fmaf(x, sm, sums[LDS_LANES * m]);
+        left &= other;
+    } while (left != 0u);
+}
+
+// sample_v1 with the sums in LDS.
+__device__ __forceinline__ void sample_lds(const VolDev &vol, Cell &c, LdsAccum &a, float px, float py, float pz,
+                                           float wt) {
+    float fx = px - c.bx, fy = py - c.by, fz = pz - c.bz;
+    if (max(max(__float_as_uint(fx), __float_as_uint(fy)), __float_as_uint(fz)) >= 0x3f800000u) {
+        const float bx = floorf(px), by = floorf(py), bz = floorf(pz);
+        c.load(vol, bx, by, bz);
+        fx = px - bx;
+        fy = py - by;
+        fz = pz - bz;
+        a.open((int)c.l1);
+    }
+    float w[8];
+    weights8(fx, fy, fz, w);
+    const float x = wt * trilerp(c.d0, c.d1, w);
+    const float ssum = ((((((w[0] + w[1]) + w[2]) + w[3]) + w[4]) + w[5]) + w[6]) + w[7];
+    a.cur = c.uni ? __builtin_fmaf(x, ssum, a.cur) : a.cur;
+    if (!c.uni) add_mixed(a.sums, c.l0, w, x);
+}
+
 // Mesh terms of a ray for march_multi: `inside(alpha)` says whether a
 // subtractive mesh hides the sample at alpha (called with increasing alpha,
-// project_kernel.cu:498-521) and `add(ad)` adds the additive mesh area
-// densities after the step scaling (569-579).  NoMesh is the scene without
-// meshes.
+// project_kernel.cu:498-521), `until()` the largest alpha up to which that
+// answer holds, and `add(ad)` adds the additive mesh area densities after the
+// step scaling (569-579).  NoMesh is the scene without meshes.
 struct NoMesh {
     __device__ __forceinline__ bool inside(float) { return false; }
+    __device__ __forceinline__ float until() const { return INFINITY; }
     template <int M>
     __device__ __forceinline__ void add(float (&)[M]) {}
 };
 
+// Waves per SIMD of the kernels that run march_multi: 80 registers, a few
+// spilled outside the sample loops (4 waves without spills: 4.27 ms against
+// 3.98 on a 768^2 view of three volumes; 8: 3.73 there, 2.74 against 2.70 with
+// a mesh, and twice the spills).
+constexpr int MULTI_WAVES = 6;
+
+// Steps a lane takes in march_multi before it looks again at what the other
+// lanes of its wave wait for: lanes that leave a stretch early (an implant's
+// edge runs through the wave) idle until the others come to its end (128 steps:
+// +7 %, no limit: +75 %).
+constexpr int MULTI_STRETCH = 48;
+
+// The alphas at which the bases floor(p) of volumes i and j can agree, as
+// [lo, hi] (lo > hi: none): |p_i - p_j| is linear in alpha and must be below
+// one voxel on every axis, here below g, which leaves room for the rounding
+// of FP32 positions and for two steps between the compared samples.
+__device__ __forceinline__ void same_base(const float *si, const float *ri, const float *sj, const float *rj,
+                                          float step, float amax, float &lo, float &hi) {
+    lo = -INFINITY;
+    hi = INFINITY;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const float D = si[a] - sj[a], E = ri[a] - rj[a], r = fabsf(ri[a]) + fabsf(rj[a]);
+        const float g = 1.25f + 2.0f * step * r + 1e-6f * (fabsf(si[a]) + fabsf(sj[a]) + amax * r);
+        if (E == 0.0f) {
+            if (!(fabsf(D) < g)) hi = -INFINITY;
+        } else {
+            const float iE = 1.0f / E, a0 = (-g - D) * iE, a1 = (g - D) * iE;
+            lo = fmaxf(lo, fminf(a0, a1));
+            hi = fminf(hi, fmaxf(a0, a1));
+        }
+    }
+}
+
 // General march for 1..V volumes with priorities and the label cache shared
-// across volumes (project_kernel.cu:394-553), literal step by step.
+// across volumes (project_kernel.cu:394-553), bit for bit, in less work:
+//   * steps before the first volume and after the last only advance alpha (and
+//     the outside air), in jumps (steps.h);
+//   * where one volume has the sole say (the usual case: alone, or on top by
+//     its priority) its samples are taken by march_v1's loop up to the next
+//     event on the ray: a volume's entry or exit, a mesh's, the stretch below;
+//     a volume is looked at only where it counts;
+//   * the shared label cache hands a volume another volume's labels only where
+//     the two volumes' bases floor(p) agree.  The stretch of the ray where any
+//     two can (same_base) follows the cache volume by volume, as the reference
+//     does at every step; elsewhere each sample's labels are its own cell's.
+//     Outside that stretch consecutive bases differ, so every lookup replaces
+//     the cache and its state at the stretch's start does not matter.  A ray
+//     that starts inside it starts at least one voxel of the first volume
+//     early: hits and misses depend on the bases alone, and were there no
+//     miss in that window, all bases would stay that of its start, but the
+//     first volume's changes.
 template <int V, int M, typename Mesh = NoMesh>
 __device__ __forceinline__ void march_multi(const ViewDev &vd, int udx, int vdx, float step,
-                                            int atten, int air, float (&ad)[M], Mesh mesh = Mesh()) {
+                                            int atten, int air, float *sums, float (&ad)[M], Mesh mesh = Mesh()) {
     float rx, ry, rz, L;
     ray_dir(vd.W, udx, vdx, rx, ry, rz, L);
     float minA = L, maxA = 0.0f;
-#pragma unroll
-    for (int m = 0; m < M; m++) ad[m] = 0.0f;
+    for (int m = 0; m < M; m++) sums[LDS_LANES * m] = 0.0f;
     constexpr int VA = V > 0 ? V : 1;  // array extent (V = 0: meshes only)
     float ri[VA][3], mnv[VA], mxv[VA];
-    bool trace[VA];
+    float first = INFINITY, last = -INFINITY;  // the ray's part inside any volume
+    float rfirst = 0.0f;                       // largest speed (voxels per mm) in the first volume
+    bool have_first = false;
 #pragma unroll
     for (int i = 0; i < V; i++) {
         ri[i][0] = ri[i][1] = ri[i][2] = 0.0f;
-        mnv[i] = mxv[i] = 0.0f;
-        trace[i] = false;
+        mnv[i] = INFINITY;  // never inside
+        mxv[i] = -INFINITY;
         if (!vd.en[i]) continue;
-        trace[i] = slab(vd.A[i], vd.s[i], vd.lo[i], vd.hi[i], vd.max_ray_length, rx, ry, rz, ri[i],
-                        mnv[i], mxv[i]);
-        if (trace[i]) {
-            minA = fminf(minA, mnv[i]);
-            maxA = fmaxf(maxA, mxv[i]);
+        float mn, mx;
+        if (slab(vd.A[i], vd.s[i], vd.lo[i], vd.hi[i], vd.max_ray_length, rx, ry, rz, ri[i], mn, mx)) {
+            mnv[i] = mn;
+            mxv[i] = mx;
+            minA = fminf(minA, mn);
+            maxA = fmaxf(maxA, mx);
+            if (mn <= mx) {
+                first = fminf(first, mn);
+                last = fmaxf(last, mx);
+            }
         }
+        if (!have_first) rfirst = fmaxf(fabsf(ri[i][0]), fmaxf(fabsf(ri[i][1]), fabsf(ri[i][2])));
+        have_first = true;
     }
     const int N = (int)ceilf((maxA - minA) / step);
-    float acc_air = 0.0f;
-    if (atten) acc_air = (float)((double)acc_air + (double)(minA / step) * DRR_AIR_DENSITY);
-    if (atten) set_m<M>(ad, air, acc_air);
-
-    float pbx = 0.0f, pby = 0.0f, pbz = 0.0f;
-    bool have = false;
-    uint32_t l0 = 0, l1 = 0;
+    LdsAccum acc{sums};
+    acc.open(air);
+    if (atten) acc.cur = (float)(0.0 + (double)(minA / step) * DRR_AIR_DENSITY);
+    // steps outside every volume, up to lim: only the air
     float alpha = minA;
-    for (int t = 0; t < N; t++) {
-        float p[VA][3];
-        float seg[VA][M];
-#pragma unroll
-        for (int i = 0; i < V; i++) {
-#pragma unroll
-            for (int m = 0; m < M; m++) seg[i][m] = 0.0f;
-            p[i][0] = p[i][1] = p[i][2] = 0.0f;
-            if (!vd.en[i]) continue;
-            const VolDev &vol = vd.vol[i];
-            p[i][0] = sample_pos(vd.s[i][0], alpha, ri[i][0]);
-            p[i][1] = sample_pos(vd.s[i][1], alpha, ri[i][1]);
-            p[i][2] = sample_pos(vd.s[i][2], alpha, ri[i][2]);
-            const float bx = floorf(p[i][0]), by = floorf(p[i][1]), bz = floorf(p[i][2]);
-            if (!have || bx != pbx || by != pby || bz != pbz) {
-                const uint32_t cell = cell_index(vol, clamp_cell(bx, vol.nx), clamp_cell(by, vol.ny),
-                                                clamp_cell(bz, vol.nz));
-                fetch_labels(vol, cell, l0, l1);
-                pbx = bx;
-                pby = by;
-                pbz = bz;
-                have = true;
-            }
-            float w[8];
-            weights8(p[i][0] - bx, p[i][1] - by, p[i][2] - bz, w);
-            material_fractions<M>(l0, l1, w, seg[i]);
+    int t = 0;
+    auto advance = [&](float lim) __attribute__((always_inline)) {
+        if (!atten) {
+            skip_steps(N, lim, step, alpha, t);
+            return;
         }
-        int cp = V, n_at = 0;
-#pragma unroll
-        for (int i = 0; i < V; i++) {
-            if (!trace[i] || !vd.en[i]) continue;
-            if ((alpha < mnv[i]) || (alpha > mxv[i])) continue;
-            float any = 0.0f;
-#pragma unroll
-            for (int m = 0; m < M; m++) any += seg[i][m];
-            // any > 0 whenever a sum prefix is > 0 (all terms are >= 0)
-            if (0.0f == any) continue;
-            if (vd.prio[i] < cp) {
-                cp = vd.prio[i];
-                n_at = 1;
-            } else if (vd.prio[i] == cp) {
-                n_at += 1;
-            }
+        acc.open(air);
+        while (t < N && alpha < lim) {
+            const bool hidden = mesh.inside(alpha);
+            const float e = mesh.until();
+            const float up = e < INFINITY ? __uint_as_float(__float_as_uint(e) + 1u) : INFINITY;  // alpha < up: alpha <= e
+            const int t0 = t;
+            skip_steps(N, fminf(lim, up), step, alpha, t);
+            if (!hidden) air_steps(t - t0, acc.cur);
         }
-        if (mesh.inside(alpha)) {
-            // the volumes (and the outside air) are hidden inside a mesh
-        } else if (0 == n_at) {
-            if (atten) set_m<M>(ad, air, add_air(get_m<M>(ad, air)));
-        } else {
-            float weight = 1.0f / ((float)n_at);
-            weight *= (0 == t || N - 1 == t) ? 0.5f : 1.0f;
+    };
+
+    if (V > 0) {
+        float c0 = INFINITY, c1 = -INFINITY;  // where the label cache is followed
+#pragma unroll
+        for (int i = 0; i < V; i++)
+#pragma unroll
+            for (int j = i + 1; j < V; j++)
+                if (vd.en[i] && vd.en[j]) {
+                    float lo, hi;
+                    same_base(vd.s[i], ri[i], vd.s[j], ri[j], step, last, lo, hi);
+                    if (lo <= hi) {
+                        c0 = fminf(c0, lo - 4.0f * step);
+                        c1 = fmaxf(c1, hi + 4.0f * step);
+                    }
+                }
+        const float early = 1.0f / rfirst + 2.0f * step;
+        advance(c0 < first && c1 >= first - early ? first - early : first);
+
+        Cell c;       // the open cell of volume cv
+        int cv = -1;
+        float pbx = 0.0f, pby = 0.0f, pbz = 0.0f;  // the shared cache: base and labels
+        uint32_t s0 = 0, s1 = 0;
+        bool have = false;
+        while (t < N && alpha <= last) {
+            // what holds at alpha, and up to which alpha (e) it holds
+            const bool follow = (alpha >= c0) & (alpha <= c1);
+            const bool hidden = mesh.inside(alpha);
+            float e = mesh.until();
+            if (V > 1) e = fminf(e, alpha < c0 ? c0 : (follow ? c1 : INFINITY));
+            int cp = V, n_at = 0, users = 0;
+            bool use[VA];
 #pragma unroll
             for (int i = 0; i < V; i++) {
-                if (trace[i] && vd.prio[i] == cp && vd.en[i] == 1) {
-                    const VolDev &vol = vd.vol[i];
-                    const float bx = floorf(p[i][0]), by = floorf(p[i][1]), bz = floorf(p[i][2]);
-                    const uint32_t cell = cell_index(vol, clamp_cell(bx, vol.nx), clamp_cell(by, vol.ny),
-                                                    clamp_cell(bz, vol.nz));
-                    gfloat *rp = (gfloat *)cell_record(vol, cell);
-                    const float4 d0 = make_float4(rp[0], rp[1], rp[2], rp[3]);
-                    const float4 d1 = make_float4(rp[4], rp[5], rp[6], rp[7]);
-                    float w[8];
-                    weights8(p[i][0] - bx, p[i][1] - by, p[i][2] - bz, w);
-                    const float rho = trilerp(d0, d1, w);
+                const bool in = (alpha >= mnv[i]) & (alpha <= mxv[i]);
+                e = fminf(e, alpha < mnv[i] ? mnv[i] : (in ? mxv[i] : INFINITY));
+                const bool lower = in & (vd.prio[i] < cp), same = in & (vd.prio[i] == cp);
+                n_at = lower ? 1 : n_at + (same ? 1 : 0);
+                cp = lower ? vd.prio[i] : cp;
+            }
 #pragma unroll
-                    for (int m = 0; m < M; m++) ad[m] = __builtin_fmaf(weight * rho, seg[i][m], ad[m]);
+            for (int i = 0; i < V; i++) {
+                // the volumes of the chosen priority count where the ray meets
+                // them at all (mnv finite), inside or not
+                use[i] = vd.en[i] == 1 && (n_at > 0) & (vd.prio[i] == cp) & (mnv[i] < INFINITY);
+                users += use[i] ? 1 : 0;
+            }
+            // steps certainly before e (as march_v1 bounds its loop), short of
+            // the half-weight ends
+            const float inc = step + 1.1920929e-7f * (fminf(fabsf(e), 1.0e30f) + step);
+            const int k = (int)__builtin_amdgcn_fmed3f((e - alpha) / inc - 2.0f, 0.0f, 16777216.0f);
+            const int tl = t > 0 ? min(t + min(k, MULTI_STRETCH), N - 1) : 0;
+            if (!follow && t < tl) {
+                if (hidden | (n_at == 0)) {
+                    const int t0 = t;
+                    skip_steps(tl, INFINITY, step, alpha, t);
+                    if (!hidden && atten) {
+                        acc.open(air);
+                        air_steps(t - t0, acc.cur);
+                    }
+                    continue;
+                }
+                if (users == 1) {  // one volume, weight 1
+#pragma unroll
+                    for (int i = 0; i < V; i++) {
+                        if (!use[i]) continue;
+                        if (V > 1 && cv != i) c = Cell();
+                        cv = i;
+                        if (c.have) acc.open((int)c.l1);
+                        while (t < tl) {
+                            sample_lds(vd.vol[i], c, acc, sample_pos(vd.s[i][0], alpha, ri[i][0]),
+                                       sample_pos(vd.s[i][1], alpha, ri[i][1]),
+                                       sample_pos(vd.s[i][2], alpha, ri[i][2]), 1.0f);
+                            alpha += step;
+                            ++t;
+                        }
+                    }
+                    continue;
                 }
             }
+            // one step, whatever holds
+            float weight = n_at > 0 ? 1.0f / (float)n_at : 0.0f;
+            weight *= (0 == t || N - 1 == t) ? 0.5f : 1.0f;
+            cv = -1;
+#pragma unroll
+            for (int i = 0; i < V; i++) {
+                if (!vd.en[i] || !(use[i] | follow)) continue;
+                const float px = sample_pos(vd.s[i][0], alpha, ri[i][0]);
+                const float py = sample_pos(vd.s[i][1], alpha, ri[i][1]);
+                const float pz = sample_pos(vd.s[i][2], alpha, ri[i][2]);
+                c.load(vd.vol[i], floorf(px), floorf(py), floorf(pz));
+                uint32_t l0 = c.l0, l1 = c.l1;
+                if (V > 1 && follow) {
+                    if (!have || c.bx != pbx || c.by != pby || c.bz != pbz) {
+                        s0 = l0;
+                        s1 = l1;
+                        pbx = c.bx;
+                        pby = c.by;
+                        pbz = c.bz;
+                        have = true;
+                    }
+                    l0 = s0;
+                    l1 = s1;
+                }
+                if (hidden | !use[i]) continue;
+                float w[8];
+                weights8(px - c.bx, py - c.by, pz - c.bz, w);
+                const float x = weight * trilerp(c.d0, c.d1, w);
+                acc.open((int)l1);
+                if (l1 != 0xffffffffu) {  // one label: the other fractions are 0
+                    const float ssum = ((((((w[0] + w[1]) + w[2]) + w[3]) + w[4]) + w[5]) + w[6]) + w[7];
+                    acc.cur = __builtin_fmaf(x, ssum, acc.cur);
+                } else {
+                    add_mixed(sums, l0, w, x);
+                }
+            }
+            if (!hidden & (n_at == 0) & (atten != 0)) {
+                acc.open(air);
+                acc.cur = add_air(acc.cur);
+            }
+            alpha += step;
+            ++t;
         }
-        alpha += step;
     }
     if (atten) {
-        float a = get_m<M>(ad, air);
-        a = (float)((double)a + (double)((L - maxA) / step) * DRR_AIR_DENSITY);
-        set_m<M>(ad, air, a);
+        advance(INFINITY);
+        acc.open(air);
+        acc.cur = (float)((double)acc.cur + (double)((L - maxA) / step) * DRR_AIR_DENSITY);
     }
+    acc.open(-1);
 #pragma unroll
-    for (int m = 0; m < M; m++) ad[m] *= step;
+    for (int m = 0; m < M; m++) ad[m] = sums[LDS_LANES * m] * step;
     mesh.add(ad);
 #pragma unroll
     for (int m = 0; m < M; m++) ad[m] /= 10.0f;

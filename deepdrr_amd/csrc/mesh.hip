@@ -578,7 +578,9 @@ __global__ __launch_bounds__(256) void k_mesh_rays(MeshDev m, Geo1 g, float sx, 
     }
 }
 
-// The march's view of one ray's mesh terms (march.h, march_multi).
+// The march's view of one ray's mesh terms (march.h, march_multi): the range
+// (lo, hi] the ray is in or comes to next stays in registers, and the list is
+// read again only when alpha passes it.
 struct MeshRay {
     const float2 *iv;
     int n, k;
@@ -586,10 +588,22 @@ struct MeshRay {
     int64_t npix, idx;
     int n_layers, n_unique;
     const int *um;
-    __device__ __forceinline__ bool inside(float alpha) {
-        while (k < n && alpha > iv[k].y) ++k;
-        return k < n && alpha > iv[k].x;
+    float lo, hi;
+    bool hidden;
+    __device__ __forceinline__ void next() {
+        const float2 r = k < n ? iv[k] : make_float2(INFINITY, INFINITY);
+        lo = r.x;
+        hi = r.y;
     }
+    __device__ __forceinline__ bool inside(float alpha) {
+        while (alpha > hi) {
+            ++k;
+            next();
+        }
+        hidden = alpha > lo;
+        return hidden;
+    }
+    __device__ __forceinline__ float until() const { return hidden ? hi : lo; }
     template <int M>
     __device__ __forceinline__ void add(float (&ad)[M]) {
         for (int u = 0; u < n_unique; u++)
@@ -614,7 +628,7 @@ struct OutMesh {
 };
 
 template <int V, int M>
-__global__ __launch_bounds__(256) void k_project_mesh(ViewDev vd, SpectrumDev sp, float step, int atten, int air,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI_WAVES))) void k_project_mesh(ViewDev vd, SpectrumDev sp, float step, int atten, int air,
                                                       MeshTerms mt, OutMesh out, int tiles16_x) {
     const int lb = blockIdx.x;
     const int bx = lb % tiles16_x, by = lb / tiles16_x;
@@ -624,9 +638,12 @@ __global__ __launch_bounds__(256) void k_project_mesh(ViewDev vd, SpectrumDev sp
     if (udx >= vd.width || vdx >= vd.height) return;
     const int64_t npix = (int64_t)vd.width * vd.height;
     const int64_t idx = (int64_t)vdx * vd.width + udx;
-    MeshRay mr{mt.iv + idx * mt.K, mt.cnt[idx], 0, mt.add, npix, idx, mt.n_layers, mt.n_unique, mt.unique_material};
+    MeshRay mr{mt.iv + idx * mt.K, mt.cnt[idx], 0, mt.add, npix, idx, mt.n_layers, mt.n_unique, mt.unique_material,
+               0.0f,               0.0f,        false};
+    mr.next();
     float ad[M];
-    march_multi<V, M, MeshRay>(vd, udx, vdx, step, atten, air, ad, mr);
+    __shared__ float sums[M * LDS_LANES];  // each thread its own words
+    march_multi<V, M, MeshRay>(vd, udx, vdx, step, atten, air, sums + threadIdx.x, ad, mr);
     float I, P;
     spectral<M>(sp, ad, I, P);
     out.intensity[idx] = I;
