@@ -27,9 +27,19 @@
 // constant majorant, unbiased like the global one (Badal & Badano 2009 use a
 // global majorant; the local form is standard in Woodcock trackers).
 //
-// GPU mapping: every lane owns one history at a time and starts the next one
-// as soon as its photon is absorbed or scored (no waiting for the slowest
-// history of the wave); each loop iteration is one flight.
+// GPU mapping: every lane owns one history at a time and is in one of a few
+// states (a brick of its flight, a tentative collision, an interaction, ...);
+// each pass of the wave's loop runs the states' blocks one after the other for
+// the lanes that wait there.  What bounds it is VALU issue times the lanes that
+// are active in it: run flight by flight the blocks had 5.3 of 64 lanes active
+// on average.  So the short and frequent blocks (a brick step, the verdict on
+// a collision, the start of a flight) run on their own, the brick loop until a
+// share of its lanes has left it, and the long and rare ones (a trial of a
+// sampler, a turn, scoring, a new history) only once enough lanes wait for
+// any of them.  A lane's own sequence of operations and random numbers stays
+// what it is, so the flights, brick steps and scores do.  Measured on a 512^3
+// phantom with 1.6e7 histories: 7.55 ms flight by flight, 4.98 ms so (15 of 64
+// lanes active).
 #include <hip/hip_runtime.h>
 
 #include "drr_internal.h"
@@ -55,13 +65,15 @@ __device__ __forceinline__ Ranecu seed_history(uint64_t seed, uint64_t h) {
     return r;
 }
 
-// RANECU: two multiplicative congruential generators (Schrage's method), combined.
+// RANECU: two multiplicative congruential generators (Schrage's method),
+// combined.  Every product has factors below 2^24 (s / 53668 < 40014 and so
+// on), so the full-rate 24-bit multiplies give them.
 __device__ __forceinline__ float ranecu(Ranecu &r) {
-    int i1 = r.s1 / 53668;
-    r.s1 = 40014 * (r.s1 - i1 * 53668) - i1 * 12211;
+    const uint32_t i1 = (uint32_t)r.s1 / 53668u;
+    r.s1 = (int)(__umul24(40014u, (uint32_t)r.s1 - __umul24(i1, 53668u)) - __umul24(i1, 12211u));
     if (r.s1 < 0) r.s1 += 2147483563;
-    int i2 = r.s2 / 52774;
-    r.s2 = 40692 * (r.s2 - i2 * 52774) - i2 * 3791;
+    const uint32_t i2 = (uint32_t)r.s2 / 52774u;
+    r.s2 = (int)(__umul24(40692u, (uint32_t)r.s2 - __umul24(i2, 52774u)) - __umul24(i2, 3791u));
     if (r.s2 < 0) r.s2 += 2147483399;
     int z = r.s1 - r.s2;
     if (z < 1) z += 2147483562;
@@ -93,43 +105,33 @@ __device__ __forceinline__ void rotate(float &u, float &v, float &w, float ct, f
     w *= n;
 }
 
-// Klein-Nishina by Kahn's method; returns cos(theta), updates E.
-__device__ __forceinline__ float compton(Ranecu &rng, float &E) {
+// One trial of Klein-Nishina by Kahn's method: whether it is accepted; eta is
+// the ratio of the energies.
+__device__ __forceinline__ bool compton_trial(Ranecu &rng, float E, float &eta) {
     const float k = E * (1.0f / 510.99895f), ik = 1.0f / k;
     const float b1 = (1.0f + 2.0f * k) / (9.0f + 2.0f * k);
-    float eta, ct;
-    for (int it = 0; it < 1000; it++) {
-        const float r1 = ranecu(rng), r2 = ranecu(rng), r3 = ranecu(rng);
-        if (r1 <= b1) {
-            eta = 1.0f + 2.0f * k * r2;
-            if (r3 <= 4.0f * (1.0f / eta - 1.0f / (eta * eta))) break;
-        } else {
-            eta = (1.0f + 2.0f * k) / (1.0f + 2.0f * k * r2);
-            ct = 1.0f - (eta - 1.0f) * ik;
-            if (r3 <= 0.5f * (ct * ct + 1.0f / eta)) break;
-        }
-    }
-    ct = 1.0f - (eta - 1.0f) * ik;
+    const float r1 = ranecu(rng), r2 = ranecu(rng), r3 = ranecu(rng);
+    const bool low = r1 <= b1;
+    const float q = 1.0f + 2.0f * k * r2;
+    eta = low ? q : (1.0f + 2.0f * k) / q;
+    const float ie = 1.0f / eta, ct = 1.0f - (eta - 1.0f) * ik;
+    return r3 <= (low ? 4.0f * (ie - 1.0f / (eta * eta)) : 0.5f * (ct * ct + ie));
+}
+
+// cos(theta) of an accepted trial, and the scattered energy.
+__device__ __forceinline__ float compton_angle(float eta, float &E) {
+    const float k = E * (1.0f / 510.99895f), ik = 1.0f / k;
+    const float ct = 1.0f - (eta - 1.0f) * ik;
     E = E / eta;
     return fminf(1.0f, fmaxf(-1.0f, ct));
 }
 
-// Thomson angular distribution (1 + cos^2) / 2 by rejection.
-__device__ __forceinline__ float rayleigh(Ranecu &rng) {
-    float c = 0.0f;
-    for (int it = 0; it < 1000; it++) {
-        c = 2.0f * ranecu(rng) - 1.0f;
-        if (ranecu(rng) <= 0.5f * (1.0f + c * c)) break;
-    }
-    return c;
-}
+constexpr int MAX_TRIALS = 1000;  // of a rejection sampler, then the last is taken
 
 struct Photon {
     float x[3], d[3];
     float E;
     int nc, nr;
-    bool alive;
-    bool inside;
 };
 
 constexpr float TWO_PI = 6.283185307179586f;
@@ -179,9 +181,29 @@ __global__ __launch_bounds__(256) void k_mc_bricks(const uint2 *__restrict__ vox
     if (lane == 0) const_cast<float4 *>(b.maj)[bi] = make_float4(mpe, mc, mr, 0.0f);
 }
 
-// 7 waves per SIMD (72 VGPRs, one spilled): 3 % more histories/s than the
-// compiler's own 74 VGPRs at 6 waves; 8 waves spill 11 and lose 3 %
-__global__ __launch_bounds__(256, 7) void k_mc(const uint2 *__restrict__ vox, int nx, int ny, int nz, drr_mc_params_t p,
+// The schedule; us of a scatter call on the 512^3 phantom with 1.6e7 histories.
+// Waves per SIMD: 6 5550, 7 4980, 8 5150 (spills)
+constexpr int MC_WAVES = 7;
+// lanes waiting for the long blocks before they run: 24 5210, 32 4980, 40 5060
+constexpr int MC_WAIT = 32;
+// sixteenths of the brick loop's lanes still in it when it ends: 3 5070, 4 4980;
+// at an earlier stage 2 and 6 were 1 % and 2 % slower than 4, 8 7 %
+constexpr int MC_STOP = 4;
+
+// What a lane's photon waits for (from REAL on: the long blocks).
+enum : int {
+    WALK,  // the next brick of its flight
+    HIT,   // the verdict on a tentative collision
+    FLY,   // a new flight
+    REAL,  // an interaction
+    COMP,  // a trial of the Compton sampler
+    RAYL,  // a trial of the Rayleigh sampler
+    OUT,   // the detector: it has left the box (or was never in it)
+    DEAD,  // a new history
+    DONE,  // nothing: the lane's histories are spent
+};
+
+__global__ __launch_bounds__(256, MC_WAVES) void k_mc(const uint2 *__restrict__ vox, int nx, int ny, int nz, drr_mc_params_t p,
                                             Bricks bk, int64_t first, int64_t count, uint64_t seed, float *img,
                                             float *img2, unsigned long long *nsteps, unsigned long long *nbsteps) {
     __shared__ float s_e[DRR_MAX_BINS], s_cdf[DRR_MAX_BINS];
@@ -204,192 +226,217 @@ __global__ __launch_bounds__(256, 7) void k_mc(const uint2 *__restrict__ vox, in
     const float iuu = 1.0f / (p.detector_u[0] * p.detector_u[0] + p.detector_u[1] * p.detector_u[1] + p.detector_u[2] * p.detector_u[2]);
     const float ivv = 1.0f / (p.detector_v[0] * p.detector_v[0] + p.detector_v[1] * p.detector_v[1] + p.detector_v[2] * p.detector_v[2]);
     const float *A = p.ijk_from_world;
+    const int n3[3] = {nx, ny, nz};
     unsigned long long steps = 0, bsteps = 0;
-    Photon ph;
-    ph.alive = false;
+    uint32_t steps_h = 0, bsteps_h = 0;  // of the current history
+    Photon ph{};
     Ranecu rng{1, 1};
     float fpe = 0.f, fc = 0.f, fr = 0.f;
     float t_exit = 0.f;
+    // the direction: bricks per step along each axis (signed, in the brick
+    // table) and the distance between brick faces (inf across the direction)
+    int sl[3] = {0, 0, 0};
+    float td[3] = {0.f, 0.f, 0.f};
+    // the flight: brick, bricks left before the box's side and distance to the
+    // next face along each axis, the distance flown, the optical depth left,
+    // the brick's majorant
+    int lin = 0, left_b[3] = {0, 0, 0};
+    float tn[3] = {0.f, 0.f, 0.f};
+    float t = 0.f, tau = 0.f, mub = 0.f;
+    float mt = 0.f, mpe = 0.f, mc = 0.f;  // of an interaction's voxel
+    int tries = 0;
+    int state = h < count ? DEAD : DONE;
     for (;;) {
-        if (!ph.alive && h >= count) break;
-        {
-            // a dead lane waits for a new history until 4 lanes of the wave are
-            // dead or none is alive, so the long start of a history runs for
-            // several lanes at once (each lane keeps its own sequence of
-            // histories, so results do not change; measured against starting
-            // at once: 4 lanes +3 %, 8 +1-2 %, 12 and 16 no change, 32 slower)
-            const unsigned long long alive = __ballot(ph.alive);
-            const int ndead = __popcll(__ballot(!ph.alive));
-            if (!ph.alive && alive != 0ull && ndead < 4) continue;
-        }
-        if (!ph.alive) {
-            rng = seed_history(seed, (uint64_t)(first + h));
-            h += stride;
-            // energy from the spectrum
-            const float u = ranecu(rng);
-            int lo = 0, hi = p.n_bins - 1;
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                if (s_cdf[mid] >= u) hi = mid; else lo = mid + 1;
+        const int n_wait = __popcll(__ballot(state >= REAL)), n_done = __popcll(__ballot(state == DONE));
+        if (n_done == 64) break;
+        // The long blocks run once MC_WAIT lanes wait for them, or no photon flies.
+        if (n_wait - n_done >= MC_WAIT || n_wait == 64) {
+            bool turn = false;  // the photon has a new direction
+            float ct = 1.0f;
+            if (state == REAL) {
+                const float u = ranecu(rng) * mt;
+                // below mpe: photoelectric absorption
+                state = u < mpe ? DEAD : (u < mpe + mc ? COMP : RAYL);
+                tries = 0;
             }
-            ph.E = s_e[lo];
-            // direction uniform in the cone about the axis
-            ph.d[0] = p.cone_axis[0];
-            ph.d[1] = p.cone_axis[1];
-            ph.d[2] = p.cone_axis[2];
-            const float ct = 1.0f - ranecu(rng) * (1.0f - p.cone_cos);
-            rotate(ph.d[0], ph.d[1], ph.d[2], ct, TWO_PI * ranecu(rng));
-            ph.x[0] = p.source_world[0];
-            ph.x[1] = p.source_world[1];
-            ph.x[2] = p.source_world[2];
-            ph.nc = ph.nr = 0;
-            ph.alive = true;
-            // entry into the volume box [-0.5, n-0.5] in IJK
-            float tmin = 0.0f, tmax = INFINITY;
-            const float nn[3] = {(float)nx, (float)ny, (float)nz};
-            bool hit = true;
-            for (int a = 0; a < 3; a++) {
-                const float q0 = A[4 * a] * ph.x[0] + A[4 * a + 1] * ph.x[1] + A[4 * a + 2] * ph.x[2] + A[4 * a + 3];
-                const float dq = A[4 * a] * ph.d[0] + A[4 * a + 1] * ph.d[1] + A[4 * a + 2] * ph.d[2];
-                if (dq != 0.0f) {
-                    const float idq = 1.0f / dq;
-                    const float t0 = (-0.5f - q0) * idq, t1 = (nn[a] - 0.5f - q0) * idq;
-                    tmin = fmaxf(tmin, fminf(t0, t1));
-                    tmax = fminf(tmax, fmaxf(t0, t1));
-                } else if (q0 < -0.5f || q0 > nn[a] - 0.5f) {
-                    hit = false;
+            // one trial of each sampler: a lane whose trial fails waits for the
+            // next round, where others join it
+            if (state == COMP) {
+                float eta;
+                if (compton_trial(rng, ph.E, eta) || ++tries == MAX_TRIALS) {
+                    ct = compton_angle(eta, ph.E);
+                    ph.nc++;
+                    turn = true;
                 }
             }
-            ph.inside = hit && tmin < tmax;
-            if (ph.inside) {
-                for (int a = 0; a < 3; a++) ph.x[a] += tmin * ph.d[a];
-                t_exit = tmax - tmin;
+            if (state == RAYL) {  // Thomson's (1 + cos^2) / 2 by rejection
+                ct = 2.0f * ranecu(rng) - 1.0f;
+                if (ranecu(rng) <= 0.5f * (1.0f + ct * ct) || ++tries == MAX_TRIALS) {
+                    ph.nr++;
+                    turn = true;
+                }
+            }
+            if (turn && (ph.E < E_MIN || ph.nc + ph.nr > p.max_interactions)) {
+                turn = false;
+                state = DEAD;
+            }
+            if (state == OUT) {
+                // out of the box (t_exit 0: never in it), straight to the detector plane
+                state = DEAD;
+                for (int a = 0; a < 3; a++) ph.x[a] += t_exit * ph.d[a];
+                const float dn = ph.d[0] * p.detector_normal[0] + ph.d[1] * p.detector_normal[1] + ph.d[2] * p.detector_normal[2];
+                const float tp = ((p.detector_origin[0] - ph.x[0]) * p.detector_normal[0] +
+                                  (p.detector_origin[1] - ph.x[1]) * p.detector_normal[1] +
+                                  (p.detector_origin[2] - ph.x[2]) * p.detector_normal[2]) / dn;
+                if (!(dn <= 0.0f) && !(tp < 0.0f)) {
+                    float r[3];
+                    for (int a = 0; a < 3; a++) r[a] = ph.x[a] + tp * ph.d[a] - p.detector_origin[a];
+                    const float fu = (r[0] * p.detector_u[0] + r[1] * p.detector_u[1] + r[2] * p.detector_u[2]) * iuu;
+                    const float fv = (r[0] * p.detector_v[0] + r[1] * p.detector_v[1] + r[2] * p.detector_v[2]) * ivv;
+                    if (fu >= 0.0f && fv >= 0.0f && fu < (float)W && fv < (float)H) {
+                        const int iu = min((int)fu, W - 1), iv = min((int)fv, H - 1);
+                        const int cls = (ph.nc + ph.nr == 0) ? 0 : (ph.nc == 1 && ph.nr == 0) ? 1 : (ph.nr == 1 && ph.nc == 0) ? 2 : 3;
+                        const int64_t o = cls * npix + (int64_t)iv * W + iu;
+                        unsafeAtomicAdd(img + o, ph.E);
+                        if (img2) unsafeAtomicAdd(img2 + o, ph.E * ph.E);
+                    }
+                }
+            }
+            bool born = false;
+            if (state == DEAD) {
+                steps += steps_h;
+                bsteps += bsteps_h;
+                steps_h = bsteps_h = 0;
+                state = DONE;
+                if (h < count) {
+                    born = true;
+                    turn = true;
+                    rng = seed_history(seed, (uint64_t)(first + h));
+                    h += stride;
+                    // energy from the spectrum
+                    const float u = ranecu(rng);
+                    int lo = 0, hi = p.n_bins - 1;
+                    while (lo < hi) {
+                        const int mid = (lo + hi) >> 1;
+                        if (s_cdf[mid] >= u) hi = mid; else lo = mid + 1;
+                    }
+                    ph.E = s_e[lo];
+                    // direction uniform in the cone about the axis
+                    ph.d[0] = p.cone_axis[0];
+                    ph.d[1] = p.cone_axis[1];
+                    ph.d[2] = p.cone_axis[2];
+                    ct = 1.0f - ranecu(rng) * (1.0f - p.cone_cos);
+                    ph.x[0] = p.source_world[0];
+                    ph.x[1] = p.source_world[1];
+                    ph.x[2] = p.source_world[2];
+                    ph.nc = ph.nr = 0;
+                }
+            }
+            if (turn) {
+                rotate(ph.d[0], ph.d[1], ph.d[2], ct, TWO_PI * ranecu(rng));
+                // the volume box [-0.5, n-0.5] in IJK: entry (of a new photon) and exit
+                float tmin = 0.0f, tmax = INFINITY;
+                bool hit = true;
+                int row = 1;
+#pragma unroll
+                for (int a = 0; a < 3; a++) {
+                    const float q0 = A[4 * a] * ph.x[0] + A[4 * a + 1] * ph.x[1] + A[4 * a + 2] * ph.x[2] + A[4 * a + 3];
+                    const float dq = A[4 * a] * ph.d[0] + A[4 * a + 1] * ph.d[1] + A[4 * a + 2] * ph.d[2];
+                    const float idq = 1.0f / dq;  // one division per axis
+                    const float hi = (float)n3[a] - 0.5f;
+                    if (dq != 0.0f) {
+                        const float t0 = (-0.5f - q0) * idq, t1 = (hi - q0) * idq;
+                        tmin = fmaxf(tmin, fminf(t0, t1));
+                        tmax = fminf(tmax, fmaxf(t0, t1));
+                    } else if (q0 < -0.5f || q0 > hi) {
+                        hit = false;
+                    }
+                    td[a] = dq != 0.0f ? (float)BRICK * fabsf(idq) : INFINITY;
+                    sl[a] = dq > 0.0f ? row : -row;
+                    row *= bk.nb[a];
+                }
+                state = FLY;
+                t_exit = fmaxf(tmax, 0.0f);
+                if (born) {
+                    const bool in = hit && tmin < tmax;
+                    state = in ? FLY : OUT;
+                    t_exit = in ? tmax - tmin : 0.0f;
+                    if (in)
+                        for (int a = 0; a < 3; a++) ph.x[a] += tmin * ph.d[a];
+                }
                 cross_sections(p, ph.E, fpe, fc, fr);
             }
         }
-        if (ph.inside) {
-            // one flight: optical depth tau spent brick by brick at each
-            // brick's majorant, up to a tentative collision or the box exit
-            ++steps;
-            float tau = -__logf(ranecu(rng));
-            int bi[3], sg[3];
-            float tn[3], td[3];
-            for (int a = 0; a < 3; a++) {
-                const float qp = A[4 * a] * ph.x[0] + A[4 * a + 1] * ph.x[1] + A[4 * a + 2] * ph.x[2] + A[4 * a + 3] + 0.5f;
-                const float dq = A[4 * a] * ph.d[0] + A[4 * a + 1] * ph.d[1] + A[4 * a + 2] * ph.d[2];
-                bi[a] = min(max((int)floorf(qp * (1.0f / BRICK)), 0), bk.nb[a] - 1);
-                const float idq = 1.0f / dq;  // one division per axis, not two
-                if (dq > 0.0f) {
-                    tn[a] = ((float)(BRICK * (bi[a] + 1)) - qp) * idq;
-                    td[a] = (float)BRICK * idq;
-                    sg[a] = 1;
-                } else if (dq < 0.0f) {
-                    tn[a] = ((float)(BRICK * bi[a]) - qp) * idq;
-                    td[a] = -(float)BRICK * idq;
-                    sg[a] = -1;
-                } else {
-                    tn[a] = INFINITY;
-                    td[a] = INFINITY;
-                    sg[a] = 0;
-                }
-                tn[a] = fmaxf(tn[a], 0.0f);
+        if ((state == HIT) | (state == FLY)) {
+            if (state == HIT) {
+                t += tau / mub;
+                for (int a = 0; a < 3; a++) ph.x[a] += t * ph.d[a];
+                t_exit -= t;
             }
-            float t = 0.0f, mub = 0.0f, s = 0.0f;
-            bool coll = false;
-            for (;;) {
-                ++bsteps;
-                const float4 mj = bk.maj[((int64_t)bi[2] * bk.nb[1] + bi[1]) * bk.nb[0] + bi[0]];
-                mub = (mj.x * fpe + mj.y * fc) + mj.z * fr;
-                const int a = (tn[0] <= tn[1] && tn[0] <= tn[2]) ? 0 : (tn[1] <= tn[2] ? 1 : 2);
-                const float tnext = fminf(tn[a], t_exit);
-                const float seg = tnext - t;
-                if (mub > 0.0f) {
-                    if (tau < mub * seg) {
-                        s = t + tau / mub;
-                        coll = true;
-                        break;
-                    }
-                    tau -= mub * seg;
-                }
-                t = tnext;
-                if (tnext >= t_exit) break;
-                bi[a] += sg[a];
-                if (bi[a] < 0 || bi[a] >= bk.nb[a]) break;
-                tn[a] += td[a];
-            }
-            if (!coll) {
-                for (int a = 0; a < 3; a++) ph.x[a] += t_exit * ph.d[a];
-                ph.inside = false;  // left the box: fly to the detector below
-            } else {
-                for (int a = 0; a < 3; a++) ph.x[a] += s * ph.d[a];
-                t_exit -= s;
+            float qp[3];
+            for (int a = 0; a < 3; a++)
+                qp[a] = A[4 * a] * ph.x[0] + A[4 * a + 1] * ph.x[1] + A[4 * a + 2] * ph.x[2] + A[4 * a + 3] + 0.5f;
+            if (state == HIT) {
                 int ix[3];
-                const int nn[3] = {nx, ny, nz};
-                for (int a = 0; a < 3; a++) {
-                    const float q = A[4 * a] * ph.x[0] + A[4 * a + 1] * ph.x[1] + A[4 * a + 2] * ph.x[2] + A[4 * a + 3];
-                    ix[a] = min(max((int)floorf(q + 0.5f), 0), nn[a] - 1);
-                }
+                for (int a = 0; a < 3; a++) ix[a] = min(max((int)floorf(qp[a]), 0), n3[a] - 1);
                 const int64_t vi = ((int64_t)ix[2] * ny + ix[1]) * nx + ix[0];
                 const uint2 rv = vox[vi];  // (density bits, label)
                 const float rho = __uint_as_float(rv.x);
                 const int m = (int)rv.y;
-                const float mpe = rho * s_a[0][m] * fpe;
-                const float mc = rho * s_a[1][m] * fc;
+                mpe = rho * s_a[0][m] * fpe;
+                mc = rho * s_a[1][m] * fc;
                 const float mr = rho * s_a[2][m] * fr;
-                const float mt = mpe + mc + mr;
-                if (ranecu(rng) * mub < mt) {
-                    const float u = ranecu(rng) * mt;
-                    float ct;
-                    if (u < mpe) {
-                        ph.alive = false;  // photoelectric absorption
-                        continue;
-                    } else if (u < mpe + mc) {
-                        ct = compton(rng, ph.E);
-                        ph.nc++;
-                    } else {
-                        ct = rayleigh(rng);
-                        ph.nr++;
-                    }
-                    rotate(ph.d[0], ph.d[1], ph.d[2], ct, TWO_PI * ranecu(rng));
-                    if (ph.E < E_MIN || ph.nc + ph.nr > p.max_interactions) {
-                        ph.alive = false;
-                        continue;
-                    }
-                    // new direction / energy: distance to the box exit and majorant
-                    float tmax = INFINITY;
-                    const float nnf[3] = {(float)nx, (float)ny, (float)nz};
-                    for (int a = 0; a < 3; a++) {
-                        const float q0 = A[4 * a] * ph.x[0] + A[4 * a + 1] * ph.x[1] + A[4 * a + 2] * ph.x[2] + A[4 * a + 3];
-                        const float dq = A[4 * a] * ph.d[0] + A[4 * a + 1] * ph.d[1] + A[4 * a + 2] * ph.d[2];
-                        if (dq != 0.0f) {
-                            const float idq = 1.0f / dq;
-                            tmax = fminf(tmax, fmaxf((-0.5f - q0) * idq, (nnf[a] - 0.5f - q0) * idq));
-                        }
-                    }
-                    t_exit = fmaxf(tmax, 0.0f);
-                    cross_sections(p, ph.E, fpe, fc, fr);
+                mt = mpe + mc + mr;
+                state = ranecu(rng) * mub < mt ? REAL : FLY;
+            }
+            if (state == FLY) {
+                // one flight: optical depth tau spent brick by brick at each
+                // brick's majorant, up to a tentative collision or the box exit
+                ++steps_h;
+                tau = -__logf(ranecu(rng));
+                lin = 0;
+#pragma unroll
+                for (int a = 0; a < 3; a++) {
+                    const int bi = min(max((int)floorf(qp[a] * (1.0f / BRICK)), 0), bk.nb[a] - 1);
+                    const bool up = sl[a] > 0, across = td[a] == INFINITY;
+                    const float idq = copysignf(td[a] * (1.0f / BRICK), up ? 1.0f : -1.0f);  // 1 / dq: BRICK is a power of 2
+                    tn[a] = across ? INFINITY : fmaxf(((float)(BRICK * (up ? bi + 1 : bi)) - qp[a]) * idq, 0.0f);
+                    left_b[a] = up ? bk.nb[a] - 1 - bi : bi;
+                    lin += abs(sl[a]) * bi;
+                }
+                t = 0.0f;
+                state = WALK;
+            }
+        }
+        // brick by brick, until more lanes wait for what comes after
+        const int stop = (__popcll(__ballot(state == WALK)) * MC_STOP) >> 4;
+        int left;
+        do {
+            if (state == WALK) {
+                ++bsteps_h;
+                const float4 mj = bk.maj[(uint32_t)lin];
+                mub = (mj.x * fpe + mj.y * fc) + mj.z * fr;
+                // the axis whose face comes first
+                const bool a0 = (tn[0] <= tn[1]) & (tn[0] <= tn[2]), a1 = !a0 & (tn[1] <= tn[2]), a2 = !(a0 | a1);
+                const float tnext = fminf(a0 ? tn[0] : (a1 ? tn[1] : tn[2]), t_exit);
+                const float depth = mub * (tnext - t);
+                if ((mub > 0.0f) & (tau < depth)) {
+                    state = HIT;
+                } else {
+                    tau -= mub > 0.0f ? depth : 0.0f;
+                    t = tnext;
+                    tn[0] += a0 ? td[0] : 0.0f;
+                    tn[1] += a1 ? td[1] : 0.0f;
+                    tn[2] += a2 ? td[2] : 0.0f;
+                    lin += a0 ? sl[0] : (a1 ? sl[1] : sl[2]);
+                    left_b[0] -= a0 ? 1 : 0;
+                    left_b[1] -= a1 ? 1 : 0;
+                    left_b[2] -= a2 ? 1 : 0;
+                    if ((tnext >= t_exit) | ((left_b[0] | left_b[1] | left_b[2]) < 0)) state = OUT;
                 }
             }
-            continue;
-        }
-        // outside the box, straight to the detector plane
-        ph.alive = false;
-        const float dn = ph.d[0] * p.detector_normal[0] + ph.d[1] * p.detector_normal[1] + ph.d[2] * p.detector_normal[2];
-        if (dn <= 0.0f) continue;
-        const float t = ((p.detector_origin[0] - ph.x[0]) * p.detector_normal[0] +
-                         (p.detector_origin[1] - ph.x[1]) * p.detector_normal[1] +
-                         (p.detector_origin[2] - ph.x[2]) * p.detector_normal[2]) / dn;
-        if (t < 0.0f) continue;
-        float r[3];
-        for (int a = 0; a < 3; a++) r[a] = ph.x[a] + t * ph.d[a] - p.detector_origin[a];
-        const float fu = (r[0] * p.detector_u[0] + r[1] * p.detector_u[1] + r[2] * p.detector_u[2]) * iuu;
-        const float fv = (r[0] * p.detector_v[0] + r[1] * p.detector_v[1] + r[2] * p.detector_v[2]) * ivv;
-        if (!(fu >= 0.0f && fv >= 0.0f && fu < (float)W && fv < (float)H)) continue;
-        const int iu = min((int)fu, W - 1), iv = min((int)fv, H - 1);
-        const int cls = (ph.nc + ph.nr == 0) ? 0 : (ph.nc == 1 && ph.nr == 0) ? 1 : (ph.nr == 1 && ph.nc == 0) ? 2 : 3;
-        const int64_t o = cls * npix + (int64_t)iv * W + iu;
-        unsafeAtomicAdd(img + o, ph.E);
-        if (img2) unsafeAtomicAdd(img2 + o, ph.E * ph.E);
+            left = __popcll(__ballot(state == WALK));
+        } while (left > stop);
     }
     if (nsteps) {
         for (int o = 32; o > 0; o >>= 1) steps += __shfl_xor(steps, o);
