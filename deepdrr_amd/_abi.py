@@ -25,6 +25,7 @@ SIGNATURES = {
     "drr_ctx_create": (C.c_int, [C.c_int, C.POINTER(_P)]),
     "drr_ctx_destroy": (C.c_int, [_P]),
     "drr_ctx_set_scene": (C.c_int, [_P, C.POINTER(Scene)]),
+    "drr_ctx_set_single_sums": (C.c_int, [_P, C.c_int]),
     "drr_ctx_set_spectrum": (C.c_int, [_P, C.c_int, _P, _P, _P]),
     "drr_ctx_last_kernel_ms": (C.c_int, [_P, C.POINTER(C.c_float)]),
     "drr_volume_create": (C.c_int, [_P, _P, _P, C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(_P)]),

@@ -15,7 +15,7 @@
 
 #include "drr_internal.h"
 #include "epilogue.h"
-#include "fast_march.h"
+#include "fast_single.h"
 #include "jobs.h"
 #include "march.h"
 
@@ -208,7 +208,7 @@ struct drr_batch_s {
     drr_ctx *ctx = nullptr;
     int M = 0;
     bool atten = false;
-    bool fast = false;  // DRR_MARCH_FAST at creation
+    int march = MARCH_V1_EXACT;  // the context's at creation
     drr_batch_tuning_t tune{};
     JobTable t;
     ImgSeg *d_imgs = nullptr;
@@ -220,8 +220,8 @@ struct drr_batch_s {
     bool launched = false;
 };
 
-template <int M, bool ATTEN, int TW, bool FAST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FAST ? FAST_WAVES : MarchOcc<M + (ATTEN ? 1 : 0)>::waves)))
+template <int M, bool ATTEN, int TW, int MARCH>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MARCH == MARCH_V1_FAST ? FAST_WAVES : MarchOcc<M + (ATTEN ? 1 : 0)>::waves)))
 void k_batch_march(const JobDev *__restrict__ jobs, const VolDev *__restrict__ vols,
                    const int2 *__restrict__ items, const int *__restrict__ seg, int *counters,
                    SpectrumDev sp, float step, int air, float *__restrict__ I, float *__restrict__ P,
@@ -229,12 +229,7 @@ void k_batch_march(const JobDev *__restrict__ jobs, const VolDev *__restrict__ v
     for_each_tile<TW>(jobs, items, seg, counters, [&](int, const JobDev &J, int udx, int vdx, bool valid) {
         if (!valid) return;
         float ad[M];
-        if constexpr (FAST) {
-            __shared__ float sums[M * LDS_LANES];  // each thread its own words
-            march_fast<M, ATTEN>(J.g, vols[J.vol], udx, vdx, step, air, sums + threadIdx.x, ad);
-        } else {
-            march_v1<M, ATTEN>(J.g, vols[J.vol], udx, vdx, step, air, ad);
-        }
+        march_single_volume<M, ATTEN, MARCH>(J.g, vols[J.vol], udx, vdx, step, air, ad);
         float inten, pp;
         spectral<M>(sp, ad, inten, pp);
         const int64_t pix = (int64_t)vdx * J.g.width + udx;
@@ -250,40 +245,40 @@ void k_batch_march(const JobDev *__restrict__ jobs, const VolDev *__restrict__ v
     });
 }
 
-template <int M, bool ATTEN, bool FAST>
+template <int M, bool ATTEN, int MARCH>
 static void launch_march_tw(int tw, const JobTable &t, hipStream_t st, SpectrumDev sp, float step, int air,
                             float *I, float *P, float *AD) {
     dim3 g(t.grid), b(t.block);
     if (tw == 16)
-        k_batch_march<M, ATTEN, 16, FAST><<<g, b, 0, st>>>(t.d_jobs, t.d_vols, t.d_items, t.d_seg, t.d_counters,
-                                                            sp, step, air, I, P, AD);
+        k_batch_march<M, ATTEN, 16, MARCH><<<g, b, 0, st>>>(t.d_jobs, t.d_vols, t.d_items, t.d_seg, t.d_counters,
+                                                             sp, step, air, I, P, AD);
     else
-        k_batch_march<M, ATTEN, 8, FAST><<<g, b, 0, st>>>(t.d_jobs, t.d_vols, t.d_items, t.d_seg, t.d_counters,
-                                                           sp, step, air, I, P, AD);
+        k_batch_march<M, ATTEN, 8, MARCH><<<g, b, 0, st>>>(t.d_jobs, t.d_vols, t.d_items, t.d_seg, t.d_counters,
+                                                            sp, step, air, I, P, AD);
 }
 
 template <int M>
-static void launch_march_m(bool atten, bool fast, int tw, const JobTable &t, hipStream_t st, SpectrumDev sp,
+static void launch_march_m(bool atten, int march, int tw, const JobTable &t, hipStream_t st, SpectrumDev sp,
                            float step, int air, float *I, float *P, float *AD) {
-    if (fast) {
-        if (atten)
-            launch_march_tw<M, true, true>(tw, t, st, sp, step, air, I, P, AD);
-        else
-            launch_march_tw<M, false, true>(tw, t, st, sp, step, air, I, P, AD);
-    } else {
-        if (atten)
-            launch_march_tw<M, true, false>(tw, t, st, sp, step, air, I, P, AD);
-        else
-            launch_march_tw<M, false, false>(tw, t, st, sp, step, air, I, P, AD);
+#define DRR_MARCH_CASE(MARCH)                                                      \
+    case MARCH:                                                                    \
+        if (atten)                                                                 \
+            launch_march_tw<M, true, MARCH>(tw, t, st, sp, step, air, I, P, AD);   \
+        else                                                                       \
+            launch_march_tw<M, false, MARCH>(tw, t, st, sp, step, air, I, P, AD);  \
+        break;
+    switch (march) {
+        DRR_MARCH_CASE(MARCH_V1_EXACT) DRR_MARCH_CASE(MARCH_V1_FAST) DRR_MARCH_CASE(MARCH_V1_SINGLE)
     }
+#undef DRR_MARCH_CASE
 }
 
-static void launch_march(const JobTable &t, int M, bool atten, bool fast, int tw, hipStream_t st,
+static void launch_march(const JobTable &t, int M, bool atten, int march, int tw, hipStream_t st,
                          SpectrumDev sp, float step, int air, float *I, float *P, float *AD) {
     switch (M) {
 #define DRR_CASE(MM)                                                             \
     case MM:                                                                     \
-        launch_march_m<MM>(atten, fast, tw, t, st, sp, step, air, I, P, AD);     \
+        launch_march_m<MM>(atten, march, tw, t, st, sp, step, air, I, P, AD);     \
         break;
         DRR_CASE(1) DRR_CASE(2) DRR_CASE(3) DRR_CASE(4) DRR_CASE(5) DRR_CASE(6) DRR_CASE(7) DRR_CASE(8) \
         DRR_CASE(9) DRR_CASE(10) DRR_CASE(11) DRR_CASE(12) DRR_CASE(13) DRR_CASE(14) DRR_CASE(15) DRR_CASE(16)
@@ -341,9 +336,9 @@ static void launch_multi_v(const JobTable &t, int M, hipStream_t st, SpectrumDev
 
 // Every job of a table: the persistent single-volume march, then the
 // multi-volume groups.
-static void launch_all(const JobTable &t, int M, bool atten, bool fast, int tw, hipStream_t st, SpectrumDev sp,
+static void launch_all(const JobTable &t, int M, bool atten, int march, int tw, hipStream_t st, SpectrumDev sp,
                        float step, int air, float *I, float *P, float *AD) {
-    if (t.n_items > 0) launch_march(t, M, atten, fast, tw, st, sp, step, air, I, P, AD);
+    if (t.n_items > 0) launch_march(t, M, atten, march, tw, st, sp, step, air, I, P, AD);
     launch_multi_v<2>(t, M, st, sp, step, atten ? 1 : 0, air, I, P, AD);
     launch_multi_v<3>(t, M, st, sp, step, atten ? 1 : 0, air, I, P, AD);
     launch_multi_v<4>(t, M, st, sp, step, atten ? 1 : 0, air, I, P, AD);
@@ -372,7 +367,7 @@ static hipError_t capture(drr_batch *B, SpectrumDev sp, float step, int air, flo
     hipError_t e = hipStreamBeginCapture(B->cap, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return e;
     k_jobs_reset<<<1, 64, 0, B->cap>>>(B->t.d_counters);
-    launch_all(B->t, B->M, B->atten, B->fast, B->tune.tile_w, B->cap, sp, step, air, I, P, nullptr);
+    launch_all(B->t, B->M, B->atten, B->march, B->tune.tile_w, B->cap, sp, step, air, I, P, nullptr);
     e = hipStreamEndCapture(B->cap, &B->graph_march);
     if (e != hipSuccess) return e;
     e = hipGraphInstantiate(&B->exec_march, B->graph_march, nullptr, nullptr, 0);
@@ -414,7 +409,7 @@ extern "C" int drr_batch_create(drr_ctx *ctx, const drr_volume *const *vols, int
     B->ctx = ctx;
     B->M = ctx->scene.n_materials;
     B->atten = ctx->scene.attenuate_outside != 0;
-    B->fast = ctx->scene.march == DRR_MARCH_FAST;
+    B->march = march_v1_mode(ctx);
     B->tune = tuning ? *tuning : drr_batch_tuning_t{8, 8, 4, 8};
     int rc = drr_jobs_build(ctx, vols, n_vols, jobs, n_jobs, B->tune, B->t);
     if (rc != DRR_OK) {
@@ -489,7 +484,7 @@ extern "C" int drr_project_jobs(drr_ctx *ctx, const drr_volume *const *vols, int
     SpectrumDev sp{ctx->d_energies, ctx->d_pdf, ctx->d_mu, ctx->n_bins};
     (void)hipEventRecord(ctx->ev0, st);
     k_jobs_reset<<<1, 64, 0, st>>>(t.d_counters);
-    launch_all(t, ctx->scene.n_materials, ctx->scene.attenuate_outside != 0, ctx->scene.march == DRR_MARCH_FAST,
+    launch_all(t, ctx->scene.n_materials, ctx->scene.attenuate_outside != 0, march_v1_mode(ctx),
                tune.tile_w, st, sp, ctx->scene.step, ctx->scene.air_index, intensity, photon_prob, area_density);
     hipError_t e = hipGetLastError();
     (void)hipEventRecord(ctx->ev1, st);
@@ -600,7 +595,7 @@ extern "C" int drr_project_jobs_noalloc(drr_ctx *ctx, const drr_volume *const *v
     SpectrumDev sp{ctx->d_energies, ctx->d_pdf, ctx->d_mu, ctx->n_bins};
     (void)hipEventRecord(ctx->ev0, st);
     k_jobs_reset<<<1, 64, 0, st>>>(t.d_counters);  // the previous call's counters are left in scratch
-    launch_all(t, ctx->scene.n_materials, ctx->scene.attenuate_outside != 0, ctx->scene.march == DRR_MARCH_FAST,
+    launch_all(t, ctx->scene.n_materials, ctx->scene.attenuate_outside != 0, march_v1_mode(ctx),
                tune.tile_w, st, sp, ctx->scene.step, ctx->scene.air_index, intensity, photon_prob, area_density);
     e = hipGetLastError();
     (void)hipEventRecord(ctx->ev1, st);

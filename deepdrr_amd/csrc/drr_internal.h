@@ -38,6 +38,7 @@ struct drr_ctx_s {
     int device = 0;
     drr_scene_t scene{0.1f, 0, 0, 0, DRR_MARCH_EXACT};
     bool have_scene = false;
+    bool single_sums = false;  // the fast march adds every sample singly (drr_ctx_set_single_sums)
     int n_bins = 0;
     float *d_energies = nullptr;  // [B]
     float *d_pdf = nullptr;       // [B]

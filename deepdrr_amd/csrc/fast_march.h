@@ -16,9 +16,11 @@
 //   roundings are as large as the 1e-5 the fast march promises to stay within
 //   of them (4e-5 on the clinical view where every cell is summed at once).
 //   So a material whose running sum has passed FAST_CLOSED_SUM is added sample
-//   by sample again.  A cell of constant density is the exception: its samples
-//   all round the same way when they are added, so n times what one adds is
-//   what the reference adds, at any size of the sum.
+//   by sample again.  Below that a cell's mean takes what the roundings add to
+//   it where they do not cancel, in a density that hardly changes from sample to
+//   sample (mean_rounding; without it a smooth body's image came to 2.6e-5 of
+//   the exact march's, with it to 7.4e-6).  A cell of constant density is summed
+//   at once at any size of the sum: its samples all round the same way.
 // * A cell with two labels (nearly every cell on a material boundary) splits
 //   the density by the second label's fraction f, also a cubic: the sum of
 //   density x f has the even moments up to u^6, about the mean of the samples'
@@ -44,8 +46,8 @@ namespace drr {
 
 // Running sum (density x step, mm g/cm^3) up to which cells are summed at once:
 // images of clinical views are then within 7.8e-6 of the exact march's (6.4e-6
-// with every sample added singly, 1.2e-5 at 128), at 17.5 ms for 48 mixed views
-// against 24.2 singly.
+// with every sample added singly, 1.2e-5 at 128, 1.6e-5 at 204.8), at 17.5 ms
+// for 48 mixed views against 24.2 singly.
 constexpr float FAST_CLOSED_SUM = 102.4f;
 // Waves per SIMD of the kernels that march fast: 80 registers hold the entry
 // block (at 8 waves' 64 it spills: 6.1 ms against 5.6 on the clinical view; 7
@@ -86,6 +88,17 @@ __device__ __forceinline__ Cubic cell_cubic(float v00, float x00, float v10, flo
 // the low three bits plus 7 carry into bit 3 and never into the next nibble).
 __device__ __forceinline__ uint32_t nz_nibbles(uint32_t x) {
     return (((x & 0x77777777u) + 0x77777777u) | x) & 0x88888888u;
+}
+
+// What rounding to cur's precision adds to the mean of samples that are added to
+// cur one by one, where the samples run from lo to hi.  The rounding error of a
+// term x is a sawtooth in x, whose integral is its square, so over a ramp the
+// mean of the errors is (el^2 - eh^2) / (2 (hi - lo)) with those at the ends.
+__device__ __forceinline__ float mean_rounding(float cur, float lo, float hi) {
+    const float el = ((cur + lo) - cur) - lo, eh = ((cur + hi) - cur) - hi, d = hi - lo;
+    const float s = 0.5f * (el + eh);
+    // (el - eh is d where the ends round to the same value)
+    return fabsf(d) > 9.5367432e-7f * fabsf(hi) ? s * ((el - eh) * __builtin_amdgcn_rcpf(d)) : s;
 }
 
 // Two-label cells: the corners' indicators of the second label as lerps along x
@@ -158,14 +171,15 @@ __device__ __forceinline__ void fast_run(const VolDev &vol, float *acc, float sx
         float cur = *pa, sq = 0.0f;
         Cubic fc = cell_cubic(c.d0.x, c.d0.y - c.d0.x, c.d0.z, c.d0.w - c.d0.z, c.d1.x, c.d1.y - c.d1.x, c.d1.z,
                               c.d1.w - c.d1.z, mx, my, mz, rix, riy, riz);
+        const float h = 0.5f * inc * nf, h2 = h * h;  // the samples' extent is [-h, h]
         bool one = true;  // the samples are to be added one by one
         bool tw = false, ex = false;  // two labels; three or more
         Second e;
         if (c.uni) {
+            const float ev = __builtin_fmaf(fc.c2, h2, fc.c0), od = h * __builtin_fmaf(fc.c3, h2, fc.c1);
             const bool flat = (fc.c1 == 0.0f) & (fc.c2 == 0.0f);
-            const float mean = flat ? (cur + fc.c0) - cur : fc.c0;
             one = !(flat | (cur < acut));
-            if (!one) *pa = cur + __builtin_fmaf(fc.c2, S2, nf * mean);
+            if (!one) *pa = cur + __builtin_fmaf(fc.c2, S2, nf * (fc.c0 + mean_rounding(cur, ev - od, ev + od)));
         } else {
             const uint32_t xa = l0 ^ (la * 0x11111111u);  // nonzero nibbles: corners not la
             const uint32_t lb = (l0 >> (__builtin_ctz(xa) & ~3u)) & 0xfu;

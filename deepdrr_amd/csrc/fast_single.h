@@ -1,0 +1,418 @@
+// fast_single.h -- the fast march with every sample added singly (single_sums of
+// the context), for images whose photons are then counted with noise.
+//
+// A Poisson count drawn for a given seed is a step function of its mean: where
+// the photon probability moves by a rounding, one count in some thousand comes
+// out one photon off, and the image with noise moves by a hundred times what
+// the image without it does.  So views that feed the noise are marched with
+// the sums in the order in which they were always added, sample by sample,
+// and a seed's noise stays what it was; with fast_march.h's sums eight views
+// of 500 x 400 take 5.3 ms in place of 5.9, noise and all, but their noise
+// differs by 1.4e-4 of the image.
+//
+// The samples t in [t, tlim), all of weight 1, have the same FP32 alpha sequence
+// as sample_v1 and, in cells whose labels agree, the same sequential FP32
+// additions into the area densities, but each sample's density is formed far
+// more cheaply than by the exact filter.  Along the ray the trilinear density
+// of a cell is a cubic in the distance u = alpha - a0 from the sample where the
+// ray entered the cell; on entering a cell its four coefficients are formed
+// from the 8 corner densities, the entry fractions and the ray direction, with
+// the distance to the exit face, and each sample then costs three multiply-adds
+// and the loop's bookkeeping.  The entry sample uses the exact march's position
+// and floor; the samples after it are placed by the exact alpha sequence (u is
+// exact) on the exact line instead of at their rounded FP32 positions, and a
+// sample within rounding of a face may take either cell (the density is
+// continuous there).  A cell with two labels splits the density by the second
+// label's fraction, also a cubic (single_run); a cell with more takes the exact
+// filter's formulas.  The sums stay within about 1e-7 relative of the exact
+// march's; nothing depends on the launch or on other lanes.
+#pragma once
+
+#include "fast_march.h"
+
+namespace drr {
+
+// How a kernel marches a single-volume view.
+enum : int { MARCH_V1_EXACT, MARCH_V1_FAST, MARCH_V1_SINGLE };
+inline int march_v1_mode(const drr_ctx *ctx) {
+    if (ctx->scene.march != DRR_MARCH_FAST) return MARCH_V1_EXACT;
+    return ctx->single_sums ? MARCH_V1_SINGLE : MARCH_V1_FAST;
+}
+// Coefficients of the trilinear interpolant of corner values (v0 = corners
+// 0..3, v1 = 4..7, corner d = dx + 2 dy + 4 dz) along the ray p(u) = p0 + u r
+// from fractions f = p0 - b: value(u) = ((k3 u + k2) u + k1) u + k0.
+__device__ __forceinline__ void cell_cubic(const float4 &v0, const float4 &v1, float fx, float fy, float fz,
+                                           float rx, float ry, float rz, float &k0, float &k1, float &k2,
+                                           float &k3) {
+    // x: e_yz(u) = A_yz + B_yz u, the lerp of corners (0yz, 1yz)
+    const float X00 = v0.y - v0.x, X10 = v0.w - v0.z, X01 = v1.y - v1.x, X11 = v1.w - v1.z;
+    const float A00 = __builtin_fmaf(fx, X00, v0.x), A10 = __builtin_fmaf(fx, X10, v0.z);
+    const float A01 = __builtin_fmaf(fx, X01, v1.x), A11 = __builtin_fmaf(fx, X11, v1.z);
+    const float B00 = rx * X00, B10 = rx * X10, B01 = rx * X01, B11 = rx * X11;
+    // y: g_z(u) = G_z0 + G_z1 u + G_z2 u^2
+    const float P0 = A10 - A00, Q0 = B10 - B00, P1 = A11 - A01, Q1 = B11 - B01;
+    const float G00 = __builtin_fmaf(fy, P0, A00), G01 = __builtin_fmaf(fy, Q0, __builtin_fmaf(ry, P0, B00));
+    const float G02 = ry * Q0;
+    const float G10 = __builtin_fmaf(fy, P1, A01), G11 = __builtin_fmaf(fy, Q1, __builtin_fmaf(ry, P1, B01));
+    const float G12 = ry * Q1;
+    // z: the cubic
+    const float D0 = G10 - G00, D1 = G11 - G01, D2 = G12 - G02;
+    k0 = __builtin_fmaf(fz, D0, G00);
+    k1 = __builtin_fmaf(fz, D1, __builtin_fmaf(rz, D0, G01));
+    k2 = __builtin_fmaf(fz, D2, __builtin_fmaf(rz, D1, G02));
+    k3 = rz * D2;
+}
+
+struct SingleCell {
+    // density = ((c3 u + c2) u + c1) u + c0 (single_run keeps the second label's
+    // corner indicators here instead in a two-label cell, zeros in a cell with more)
+    float c0 = 0.f, c1 = 0.f, c2 = 0.f, c3 = 0.f;
+    float a0 = 0.f;    // alpha of the entry sample (u = alpha - a0)
+    float nex = 0.f;   // distance to the exit face, in steps
+
+    // Enter cell c at alpha with fractions (fx, fy, fz) (those of the exact
+    // march) and the ray direction r in voxels per mm.  Per axis, the exit
+    // face is reached after fma(-f, j, h) steps with j = 1 / (r step) and
+    // h = j going up, 0 going down (j = 0, h = +inf where r = 0).
+    __device__ __forceinline__ void enter(const Cell &c, float alpha, float fx, float fy, float fz, float rx,
+                                          float ry, float rz, float jx, float jy, float jz, float hx, float hy,
+                                          float hz) {
+        a0 = alpha;
+        cell_cubic(c.d0, c.d1, fx, fy, fz, rx, ry, rz, c0, c1, c2, c3);
+        nex = fminf(__builtin_fmaf(-fx, jx, hx), fminf(__builtin_fmaf(-fy, jy, hy), __builtin_fmaf(-fz, jz, hz)));
+    }
+};
+
+// The samples of the entered cells (single_run): n for this lane, the density
+// cubic in fc (tw: a two-label cell, whose corner data fc and e hold instead)
+// and the two-label formulas where tw (TWO: some lane of the wave has a
+// two-label cell; the two forms are separate loops).
+template <bool TWO>
+__device__ __forceinline__ void single_cell(const Cell &c, const SingleCell &fc, Accum &a, float &sq, float e0,
+                                          float e1, float e2, float e3, bool tw, int n, float sx, float sy,
+                                          float sz, float rix, float riy, float riz, float step, float &alpha) {
+    float u = 0.0f;
+    for (int k = 0;; ++k) {
+        const bool in = k < n;
+        if (__ballot(in) == 0) break;
+        float rho = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(fc.c3, u, fc.c2), u, fc.c1), u, fc.c0);
+        const float g = in ? 1.0f : 0.0f;
+        if (TWO) {
+            // two labels: density and q-fraction at the sample's FP32 position
+            // (that of the exact filter), each by nested lerps
+            const float fx = __builtin_fmaf(alpha, rix, sx) - (c.bx + 1.0f);
+            const float fy = __builtin_fmaf(alpha, riy, sy) - (c.by + 1.0f);
+            const float fz = __builtin_fmaf(alpha, riz, sz) - (c.bz + 1.0f);
+            const float a00 = __builtin_fmaf(fx, c.d0.y - c.d0.x, c.d0.x);
+            const float a10 = __builtin_fmaf(fx, c.d0.w - c.d0.z, c.d0.z);
+            const float a01 = __builtin_fmaf(fx, c.d1.y - c.d1.x, c.d1.x);
+            const float a11 = __builtin_fmaf(fx, c.d1.w - c.d1.z, c.d1.z);
+            const float b0 = __builtin_fmaf(fy, a10 - a00, a00), b1 = __builtin_fmaf(fy, a11 - a01, a01);
+            const float x = __builtin_fmaf(fz, b1 - b0, b0);
+            const float i00 = __builtin_fmaf(fx, e0, fc.c0), i10 = __builtin_fmaf(fx, e1, fc.c1);
+            const float i01 = __builtin_fmaf(fx, e2, fc.c2), i11 = __builtin_fmaf(fx, e3, fc.c3);
+            const float j0 = __builtin_fmaf(fy, i10 - i00, i00), j1 = __builtin_fmaf(fy, i11 - i01, i01);
+            const float fq = __builtin_fmaf(fz, j1 - j0, j0);
+            const float xq = x * fq;
+            sq = __builtin_fmaf(g, tw ? xq : 0.0f, sq);
+            rho = tw ? x - xq : rho;
+        }
+        a.cur = __builtin_fmaf(g, rho, a.cur);
+        alpha = __builtin_fmaf(g, step, alpha);
+        u = alpha - fc.a0;
+    }
+}
+
+// The samples of a cell with three or more labels (ex), after single_cell has
+// taken the cell's samples for the other lanes: the exact filter's formulas at
+// the same FP32 alpha sequence, re-walked from the entry sample a0, added into
+// ad[] sample by sample (the lane has no running sum in such a cell).
+template <int M>
+__device__ __forceinline__ void single_exact(const Cell &c, float (&ad)[M], bool ex, int n, float a0, float sx,
+                                           float sy, float sz, float rix, float riy, float riz, float step) {
+    float al = a0;
+    for (int k = 0;; ++k) {
+        const bool in = (k < n) & ex;
+        if (__ballot(in) == 0) break;
+        if (in) {
+            const float fx = __builtin_fmaf(al, rix, sx) - (c.bx + 1.0f);
+            const float fy = __builtin_fmaf(al, riy, sy) - (c.by + 1.0f);
+            const float fz = __builtin_fmaf(al, riz, sz) - (c.bz + 1.0f);
+            float w[8];
+            weights8(fx, fy, fz, w);
+            const float x = trilerp(c.d0, c.d1, w);
+#pragma unroll
+            for (int m = 0; m < M; m++) {
+                const uint32_t xm = c.l0 ^ (0x11111111u * (uint32_t)m);
+                if (((xm - 0x11111111u) & ~xm & 0x88888888u) != 0u) {
+                    float sm = 0.0f;
+#pragma unroll
+                    for (int d = 0; d < 8; d++) sm += (corner_label(c.l0, c.l1, d) == (uint32_t)m) ? w[d] : 0.0f;
+                    ad[m] = __builtin_fmaf(x, sm, ad[m]);
+                }
+            }
+        }
+        al += step;
+    }
+}
+
+template <int M>
+__device__ __forceinline__ void single_run(const VolDev &vol, Cell &c, SingleCell &fc, float (&ad)[M], Accum &a,
+                                         float sx, float sy, float sz, float rix, float riy, float riz,
+                                         float step, float &alpha, int &t, int tlim, float amax) {
+    // Cell by cell: every lane still marching enters the cell of its current
+    // sample together (one execution of the long cell-entry block for the whole
+    // wave), then the wave runs the samples of those cells until every lane has
+    // taken its own.  Lanes whose cells end early idle for the rest of that inner
+    // loop, which costs less than running the entry block once for each group
+    // of lanes that leave together.  A cell's sample count n is fixed on entry:
+    // the samples at u = 0, step, 2 step, ... (for a far source, at the FP32
+    // increment) before the exit distance (at least the entry sample, at
+    // most the samples left before tlim); a sample within the FP32 alpha
+    // sequence's drift of the face may so fall to either cell, where the
+    // density is continuous.  The inner loop's test is a wave vote and
+    // its per-lane choices are 0/1 factors: per-lane branches and loop exits cost
+    // scalar instructions (exec-mask bookkeeping), enough to become the limit in
+    // a loop this short.  With g = 1, fma(g, rho, cur) = cur + rho and
+    // fma(g, step, alpha) = alpha + step exactly; with g = 0 both leave the
+    // value unchanged.
+    //
+    // Materials: a cell whose labels agree adds each sample's density to the
+    // running sum of its material (Accum).  A cell with exactly two labels
+    // (nearly every cell on a material boundary) forms each sample's density
+    // and the fraction f_q of its second label q at the sample's FP32 position,
+    // as the exact filter does (across a boundary the density changes by up to
+    // several g/cm^3 per voxel, so that position's rounding shows at 1e-5 in
+    // the sums, unlike in a cell of one material), each by nested lerps:
+    // rho (1 - f_q) goes to the running sum of the first material and rho f_q
+    // to a second running sum sq of ad[q], written back when q or the first
+    // material changes and when the run ends; so every term is still added into
+    // its material's area density one sample at a time, as the exact filter
+    // adds it.  A cell with three or more labels takes the exact filter's
+    // formulas, its density cubic set to zero.  In a wave with no two-label
+    // cell the two-label formulas are skipped; a lane in a one-label cell
+    // selects its cubic's value and adds zero to sq, so its results do not
+    // depend on the other lanes.
+    if (__ballot(t < tlim) == 0) return;
+    // exit distances in steps (reciprocals to 1 ulp are plenty there), kept in
+    // registers (an empty asm stops the compiler from forming them again on
+    // every cell entry)
+    const float istep = 1.0f / step;
+    float jx = rix == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(rix) * istep;
+    float jy = riy == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(riy) * istep;
+    float jz = riz == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(riz) * istep;
+    float hx = rix == 0.0f ? INFINITY : (rix < 0.0f ? 0.0f : jx);
+    float hy = riy == 0.0f ? INFINITY : (riy < 0.0f ? 0.0f : jy);
+    float hz = riz == 0.0f ? INFINITY : (riz < 0.0f ? 0.0f : jz);
+    // Each FP32 `alpha += step` moves alpha by step rounded to alpha's ulp, off
+    // step by up to half an ulp.  Below 2^14 steps (about 1.6 m at 0.1 mm) that
+    // is under 2^-11 of a step and the samples a cell's count assumes stay
+    // within rounding of its face.  Beyond (a far source: at 4 km alpha moves a
+    // quarter step more, or not at all) the exit distances are scaled by step
+    // over the larger of the increments at the ray's current alpha and at its
+    // largest, those of the two binades a far ray spans, so a cell's count ends
+    // at its exit face (a ray that also crosses lower binades, starting near its
+    // source, has their increments within 3/4 of an ulp of amax of these); where
+    // alpha stops moving, every entry takes one sample.
+    if (amax > 16384.0f * step) {
+        const float s_lo = (alpha + step) - alpha, s_hi = (amax + step) - amax;
+        const float fac = (s_lo > 0.0f && s_hi > 0.0f) ? step / fmaxf(s_lo, s_hi) : 0.0f;
+        jx *= fac;
+        jy *= fac;
+        jz *= fac;
+        hx = fac > 0.0f ? hx * fac : 0.0f;
+        hy = fac > 0.0f ? hy * fac : 0.0f;
+        hz = fac > 0.0f ? hz * fac : 0.0f;
+    }
+    asm volatile("" : "+v"(jx), "+v"(jy), "+v"(jz), "+v"(hx), "+v"(hy), "+v"(hz));
+    float sq = 0.0f;  // ad[q] while q (the second material of two-label cells) is >= 0
+    int q = -1;
+    // two labels: the q-indicators' x-differences (read only where tw, so not
+    // cleared for other cells)
+    float e0 = 0.f, e1 = 0.f, e2 = 0.f, e3 = 0.f;
+    do {
+        int n = 0;        // samples of the entered cell
+        bool ex = false;  // three or more labels: the exact filter
+        bool tw = false;  // two labels
+        if (t < tlim) {
+            const float px = sample_pos(sx, alpha, rix), py = sample_pos(sy, alpha, riy),
+                        pz = sample_pos(sz, alpha, riz);
+            const float bx = floorf(px), by = floorf(py), bz = floorf(pz);
+            c.load(vol, bx, by, bz);
+            const float fx = px - bx, fy = py - by, fz = pz - bz;
+            fc.enter(c, alpha, fx, fy, fz, rix, riy, riz, jx, jy, jz, hx, hy, hz);
+            int ncm = (int)c.l1;  // the first material (the common one in a one-label cell)
+            int qn = -1;          // the second material of a two-label cell
+            if (!c.uni) {
+                const uint32_t l0 = c.l0;
+                const uint32_t la = l0 & 0xfu;
+                const uint32_t xa = l0 ^ (la * 0x11111111u);  // nonzero nibbles: corners not la
+                const uint32_t lb = (l0 >> (__builtin_ctz(xa) & ~3u)) & 0xfu;
+                const uint32_t xb = l0 ^ (lb * 0x11111111u);
+                const uint32_t na = nz_nibbles(xa), nb = nz_nibbles(xb);
+                if ((na & nb) == 0u) {
+                    // the first material keeps the running sum when it already has it
+                    const bool sw = (int)lb == a.cm;
+                    ncm = (int)(sw ? lb : la);
+                    qn = (int)(sw ? la : lb);
+                    const uint32_t iq = sw ? na : nb;  // bit set: corner not q
+                    // q-indicators of the corners: bases of the x-lerps in fc.c0..c3,
+                    // their differences in e0..e3
+                    fc.c0 = (iq & 0x8u) ? 0.f : 1.f;
+                    fc.c1 = (iq & 0x800u) ? 0.f : 1.f;
+                    fc.c2 = (iq & 0x80000u) ? 0.f : 1.f;
+                    fc.c3 = (iq & 0x8000000u) ? 0.f : 1.f;
+                    e0 = ((iq & 0x80u) ? 0.f : 1.f) - fc.c0;
+                    e1 = ((iq & 0x8000u) ? 0.f : 1.f) - fc.c1;
+                    e2 = ((iq & 0x800000u) ? 0.f : 1.f) - fc.c2;
+                    e3 = ((iq & 0x80000000u) ? 0.f : 1.f) - fc.c3;
+                    tw = true;
+                } else {
+                    ex = true;
+                    fc.c0 = fc.c1 = fc.c2 = fc.c3 = 0.0f;
+                }
+            }
+            if (q >= 0 && (ncm != a.cm || (qn >= 0 && qn != q))) {
+                set_m<M>(ad, q, sq);
+                q = -1;
+            }
+            if (ncm != a.cm) {
+                if (a.cm >= 0) set_m<M>(ad, a.cm, a.cur);
+                a.cm = ncm;
+                a.cur = get_m<M>(ad, ncm);
+            }
+            if (qn >= 0 && q < 0) {
+                q = qn;
+                sq = get_m<M>(ad, qn);
+            }
+            // the samples before the exit face, clamped to [1, tlim - t] after
+            // the conversion (which saturates infinities and takes NaN to 0), so
+            // every entry takes at least one sample
+            n = min(max((int)ceilf(fc.nex), 1), tlim - t);
+        }
+        if (__ballot(tw) != 0)
+            single_cell<true>(c, fc, a, sq, e0, e1, e2, e3, tw, n, sx, sy, sz, rix, riy, riz, step, alpha);
+        else
+            single_cell<false>(c, fc, a, sq, e0, e1, e2, e3, tw, n, sx, sy, sz, rix, riy, riz, step, alpha);
+        if (__ballot(ex) != 0) single_exact<M>(c, ad, ex, n, fc.a0, sx, sy, sz, rix, riy, riz, step);
+        t += n;
+    } while (__ballot(t < tlim) != 0);
+    if (q >= 0) set_m<M>(ad, q, sq);
+    // sample_v1 adds a mixed cell's terms into ad[] directly and expects no
+    // running sum there: write a two-label cell's first material back
+    if (!c.uni && a.cm >= 0) {
+        set_m<M>(ad, a.cm, a.cur);
+        a.cm = -1;
+        a.cur = 0.0f;
+    }
+}
+
+// Single-volume march (project_kernel.cu:334-584 with NUM_VOLUMES == 1).
+// On return ad[] holds the final area densities in g/cm^2.
+template <int M, bool ATTEN>
+__device__ __forceinline__ void march_fast_single(const Geo1 &g, const VolDev &vol, int udx, int vdx,
+                                                  float step, int air, float (&ad)[M]) {
+    RayV1 r;
+    march_setup_v1(g, udx, vdx, step, r);
+#pragma unroll
+    for (int m = 0; m < M; m++) ad[m] = 0.0f;
+    float acc = 0.0f;  // air accumulator while no volume is sampled
+    if (ATTEN) acc = (float)((double)acc + (double)(r.minA / step) * DRR_AIR_DENSITY);
+
+    const int N = r.N;
+    float alpha = r.minA;
+    int t = 0;
+    if (r.trace) {
+        const float sx = g.s[0], sy = g.s[1], sz = g.s[2];
+        const float rix = r.ri[0], riy = r.ri[1], riz = r.ri[2];
+        // Phase 1: steps well before the volume: only the alpha sequence.
+        const float rdom = fmaxf(fabsf(rix), fmaxf(fabsf(riy), fabsf(riz)));
+        const float lim = r.mnv - (1.0f / rdom + 2.0f * step);
+        skip_steps(N, lim, step, alpha, t);
+        if (ATTEN) air_steps(t, acc);
+        // Phase 2: approach window, label cache tracked as the reference does.
+        Cell c;
+        while (t < N && alpha < r.mnv) {
+            const float px = sample_pos(sx, alpha, rix);
+            const float py = sample_pos(sy, alpha, riy);
+            const float pz = sample_pos(sz, alpha, riz);
+            const float bx = floorf(px), by = floorf(py), bz = floorf(pz);
+            if (!c.have || bx != c.bx || by != c.by || bz != c.bz) c.load(vol, bx, by, bz);
+            if (ATTEN) acc = add_air(acc);
+            alpha += step;
+            ++t;
+        }
+        if (ATTEN) set_m<M>(ad, air, acc);
+        // Phase 3: inside [minAlpha_vol, maxAlpha_vol]: sample and accumulate.
+        // While the ray is in a cell whose 8 labels agree (material m0), only
+        // ad[m0] changes; it is kept in `cur` and written back on leaving, so
+        // every FP32 addition is the one the reference performs.  The end
+        // samples t == 0 and t == N-1 carry weight 0.5 (project_kernel.cu:
+        // 541), the others 1.
+        Accum acc3;
+        if (c.have && c.uni) {
+            acc3.cm = (int)c.l1;
+            acc3.cur = get_m<M>(ad, acc3.cm);
+        }
+        // The loop runs while t < tlim with no test on alpha: tlim is at most
+        // the last weight-1 sample (N - 2) and at most the samples whose alpha
+        // is certainly <= maxAlpha_vol.  Each FP32 `alpha += step` adds at
+        // most step + 2^-24 (|mxv| + step) while alpha <= mxv, so with
+        // inc = step + 2^-23 (|mxv| + step) the next K = floor((mxv - alpha)
+        // / inc) - 2 samples stay inside (the -2 covers the FP32 quotient and
+        // difference).  Past tlim the loop re-enters one sample at a time with
+        // the full test; the last sample (t == N-1) re-enters with weight 0.5.
+        float wt = (0 == t) ? 0.5f : 1.0f;
+        const float inc = step + 1.1920929e-7f * (fabsf(r.mxv) + step);
+        const float kf = (r.mxv - alpha) / inc - 2.0f;
+        // (clamped in float to a range the conversion holds, then to N - 1 in
+        // integers, where (float)(N - 1 - t) could round up)
+        int tlim = min(t + (int)__builtin_amdgcn_fmed3f(kf, 0.0f, 16777216.0f), N - 1);
+        for (;;) {
+            // a sample of weight 0.5 (the first) takes the exact filter
+            if (wt != 1.0f && t < tlim) {
+                sample_v1<M>(vol, c, ad, acc3, sample_pos(sx, alpha, rix), sample_pos(sy, alpha, riy),
+                             sample_pos(sz, alpha, riz), wt);
+                wt = 1.0f;
+                alpha += step;
+                ++t;
+            }
+            SingleCell fc;  // no cell entered: the first sample enters one
+            single_run<M>(vol, c, fc, ad, acc3, sx, sy, sz, rix, riy, riz, step, alpha, t, tlim, r.mxv);
+            // a fresh comparison after the loop (an empty asm hides alpha's
+            // in-loop history), so the loop does not carry one
+            asm volatile("" : "+v"(alpha));
+            if (!(alpha <= r.mxv) || t >= N) break;
+            if (t == N - 1) wt = 0.5f;
+            tlim = t + 1;
+        }
+        if (acc3.cm >= 0) set_m<M>(ad, acc3.cm, acc3.cur);
+        if (ATTEN) acc = get_m<M>(ad, air);
+    }
+    // Phase 4: the rest of the steps sample nothing.
+    if (ATTEN) {
+        air_steps(N - t, acc);
+        acc = (float)((double)acc + (double)((r.L - r.maxA) / step) * DRR_AIR_DENSITY);
+        set_m<M>(ad, air, acc);
+    }
+#pragma unroll
+    for (int m = 0; m < M; m++) ad[m] *= step;
+#pragma unroll
+    for (int m = 0; m < M; m++) ad[m] /= 10.0f;
+}
+
+// The single-volume march of a thread of a block of at most LDS_LANES.
+template <int M, bool ATTEN, int MARCH>
+__device__ __forceinline__ void march_single_volume(const Geo1 &g, const VolDev &vol, int udx, int vdx, float step,
+                                                    int air, float (&ad)[M]) {
+    if constexpr (MARCH == MARCH_V1_FAST) {
+        __shared__ float sums[M * LDS_LANES];  // each thread its own words
+        march_fast<M, ATTEN>(g, vol, udx, vdx, step, air, sums + threadIdx.x, ad);
+    } else if constexpr (MARCH == MARCH_V1_SINGLE) {
+        march_fast_single<M, ATTEN>(g, vol, udx, vdx, step, air, ad);
+    } else {
+        march_v1<M, ATTEN>(g, vol, udx, vdx, step, air, ad);
+    }
+}
+
+}  // namespace drr

@@ -5,7 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include "drr_internal.h"
-#include "fast_march.h"
+#include "fast_single.h"
 #include "march.h"
 
 using namespace drr;
@@ -78,8 +78,8 @@ struct OutDev {
     float *solid_angle;   // [H][W] or NULL
 };
 
-template <int M, bool ATTEN, bool FAST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FAST ? FAST_WAVES : MarchOcc<M>::waves))) void k_project_v1(Geo1 g, VolDev vol, SpectrumDev sp, float step,
+template <int M, bool ATTEN, int MARCH>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MARCH == MARCH_V1_FAST ? FAST_WAVES : MarchOcc<M>::waves))) void k_project_v1(Geo1 g, VolDev vol, SpectrumDev sp, float step,
                                                     int air, OutDev out, int tiles16_x) {
     const int lb = blockIdx.x;
     const int bx = lb % tiles16_x, by = lb / tiles16_x;
@@ -88,12 +88,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FAST ? FAST
     lane_pixel(bx * 2 + (wave & 1), by * 2 + (wave >> 1), lane, udx, vdx);
     if (udx >= g.width || vdx >= g.height) return;
     float ad[M];
-    if constexpr (FAST) {
-        __shared__ float sums[M * LDS_LANES];  // each thread its own words
-        march_fast<M, ATTEN>(g, vol, udx, vdx, step, air, sums + threadIdx.x, ad);
-    } else {
-        march_v1<M, ATTEN>(g, vol, udx, vdx, step, air, ad);
-    }
+    march_single_volume<M, ATTEN, MARCH>(g, vol, udx, vdx, step, air, ad);
     float I, P;
     spectral<M>(sp, ad, I, P);
     const int64_t npix = (int64_t)g.width * g.height;
@@ -134,19 +129,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI_WAVES
 }
 
 template <int M>
-static void launch_v1(bool atten, bool fast, dim3 g, dim3 b, hipStream_t st, const Geo1 &geo, const VolDev &vol,
+static void launch_v1(bool atten, int march, dim3 g, dim3 b, hipStream_t st, const Geo1 &geo, const VolDev &vol,
                       const SpectrumDev &sp, float step, int air, const OutDev &o, int tx) {
-    if (fast) {
-        if (atten)
-            k_project_v1<M, true, true><<<g, b, 0, st>>>(geo, vol, sp, step, air, o, tx);
-        else
-            k_project_v1<M, false, true><<<g, b, 0, st>>>(geo, vol, sp, step, air, o, tx);
-    } else {
-        if (atten)
-            k_project_v1<M, true, false><<<g, b, 0, st>>>(geo, vol, sp, step, air, o, tx);
-        else
-            k_project_v1<M, false, false><<<g, b, 0, st>>>(geo, vol, sp, step, air, o, tx);
+#define DRR_MARCH_CASE(MARCH)                                                                    \
+    case MARCH:                                                                                  \
+        if (atten)                                                                               \
+            k_project_v1<M, true, MARCH><<<g, b, 0, st>>>(geo, vol, sp, step, air, o, tx);       \
+        else                                                                                     \
+            k_project_v1<M, false, MARCH><<<g, b, 0, st>>>(geo, vol, sp, step, air, o, tx);      \
+        break;
+    switch (march) {
+        DRR_MARCH_CASE(MARCH_V1_EXACT) DRR_MARCH_CASE(MARCH_V1_FAST) DRR_MARCH_CASE(MARCH_V1_SINGLE)
     }
+#undef DRR_MARCH_CASE
 }
 
 template <int V>
@@ -187,7 +182,7 @@ extern "C" int drr_project(drr_ctx *ctx, const drr_volume *const *vols, const dr
         switch (sc.n_materials) {
 #define DRR_CASE(MM) \
     case MM:                                                                                           \
-        launch_v1<MM>(sc.attenuate_outside != 0, sc.march == DRR_MARCH_FAST, grid, block, st, geo, vol0, sp, \
+        launch_v1<MM>(sc.attenuate_outside != 0, march_v1_mode(ctx), grid, block, st, geo, vol0, sp, \
                       sc.step, sc.air_index, o, tx);                                                     \
         break;
             DRR_CASE(1) DRR_CASE(2) DRR_CASE(3) DRR_CASE(4) DRR_CASE(5) DRR_CASE(6) DRR_CASE(7) DRR_CASE(8) \

@@ -123,6 +123,12 @@ int drr_ctx_set_scene(drr_ctx *ctx, const drr_scene_t *scene) {
     return DRR_OK;
 }
 
+int drr_ctx_set_single_sums(drr_ctx *ctx, int single) {
+    if (!ctx) return drr_set_error(DRR_ERR_INVALID, "drr_ctx_set_single_sums: NULL argument");
+    ctx->single_sums = single != 0;
+    return DRR_OK;
+}
+
 int drr_ctx_set_spectrum(drr_ctx *ctx, int n_bins, const float *energies_keV, const float *pdf,
                          const float *mu_over_rho) {
     if (!ctx || !energies_keV || !pdf || !mu_over_rho)

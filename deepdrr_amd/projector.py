@@ -403,8 +403,13 @@ class Projector:
             self._mesh_key = key
         return self._mesh
 
+    def _set_sums(self):
+        # noise drawn for a seed follows the photon probabilities' roundings
+        _abi.call("drr_ctx_set_single_sums", self._ctx, 1 if self.add_noise else 0)
+
     def _launch_view(self, proj: geo.CameraProjection, intensity, photon_prob, area_density, solid_angle, stream):
         view = self.view_for(proj)
+        self._set_sums()
         if self.meshes:
             src = np.ascontiguousarray(np.asarray(proj.center_in_world), np.float32)
             sdd = self.source_to_detector_distance
@@ -485,6 +490,7 @@ class Projector:
                         and self.intensity_upper_bound is None)
         host_epilogue = (self.add_noise and not device_noise) or self.intensity_upper_bound is not None \
             or self.mc_scatter_histories > 0
+        self._set_sums()
         plan = plan_for_projector(self, camera_projections, volume_indices,
                                   neglog=self.neglog and not host_epilogue and not device_noise, tuning=tuning)
         try:

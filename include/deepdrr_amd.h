@@ -64,10 +64,10 @@ typedef struct {
 /* How a single-volume view is marched (drr_scene_t.march).  EXACT: the
  * reference's per-sample trilinear filter with its FP32 operation order
  * (area densities bit-identical to the oracle's transcription).  FAST: the same
- * samples, each term still added into its material's area density one sample
- * at a time, with each sample's density formed from a per-cell cubic along the
- * ray (a cell with two labels: nested lerps at the sample's position; with
- * more: the exact filter), so values are within rounding of EXACT and images
+ * samples, with the densities formed from a per-cell cubic along the ray (a
+ * cell with three or more labels: the exact filter) and a cell's samples added
+ * together while its material's sum is short enough for the additions'
+ * roundings not to show, so values are within rounding of EXACT and images
  * within 1e-5 relative.  Views over several volumes or with meshes are marched
  * exactly in both modes.  No counterpart in the reference. */
 #define DRR_MARCH_EXACT 0
@@ -97,6 +97,13 @@ int drr_ctx_destroy(drr_ctx *ctx);
 
 /* Scene settings: step, material count, air handling (projector.py:365-386). */
 int drr_ctx_set_scene(drr_ctx *ctx, const drr_scene_t *scene);
+
+/* Whether FAST marches of this context (drr_project, drr_project_jobs and
+ * batches created from now on) add every sample into its sum singly: 0 (the
+ * default) no, otherwise yes.  A Poisson count drawn for a seed is a step
+ * function of its mean, so images with noise keep their counts only if the
+ * photon probabilities keep their roundings. */
+int drr_ctx_set_single_sums(drr_ctx *ctx, int single);
 
 /* Spectrum and mu/rho table, host pointers: energies_keV[B], pdf[B],
  * mu_over_rho[B * n_materials] indexed [bin * M + m] (projector.py:1660-1689). */
