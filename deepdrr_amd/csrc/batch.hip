@@ -468,13 +468,15 @@ extern "C" int drr_batch_destroy(drr_batch *B) {
     return DRR_OK;
 }
 
-extern "C" int drr_project_jobs(drr_ctx *ctx, const drr_volume *const *vols, int n_vols, const drr_job_t *jobs,
-                                int n_jobs, float *intensity, float *photon_prob, float *area_density,
-                                void *stream) {
+extern "C" int drr_project_jobs_march(drr_ctx *ctx, const drr_volume *const *vols, int n_vols, const drr_job_t *jobs,
+                                      int n_jobs, int march, float *intensity, float *photon_prob,
+                                      float *area_density, void *stream) {
     if (!ctx || !vols || !jobs || !intensity)
         return drr_set_error(DRR_ERR_INVALID, "drr_project_jobs: NULL argument");
     if (!ctx->have_scene || ctx->n_bins < 1)
         return drr_set_error(DRR_ERR_STATE, "drr_project_jobs: scene/spectrum not set");
+    if (march != DRR_MARCH_EXACT && march != DRR_MARCH_FAST)
+        return drr_set_error(DRR_ERR_INVALID, "drr_project_jobs: march must be DRR_MARCH_EXACT or DRR_MARCH_FAST");
     DevSwitch ds(ctx->device);
     JobTable t;
     const drr_batch_tuning_t tune{8, 8, 4, 8};
@@ -484,7 +486,7 @@ extern "C" int drr_project_jobs(drr_ctx *ctx, const drr_volume *const *vols, int
     SpectrumDev sp{ctx->d_energies, ctx->d_pdf, ctx->d_mu, ctx->n_bins};
     (void)hipEventRecord(ctx->ev0, st);
     k_jobs_reset<<<1, 64, 0, st>>>(t.d_counters);
-    launch_all(t, ctx->scene.n_materials, ctx->scene.attenuate_outside != 0, march_v1_mode(ctx),
+    launch_all(t, ctx->scene.n_materials, ctx->scene.attenuate_outside != 0, march_v1_mode(ctx, march),
                tune.tile_w, st, sp, ctx->scene.step, ctx->scene.air_index, intensity, photon_prob, area_density);
     hipError_t e = hipGetLastError();
     (void)hipEventRecord(ctx->ev1, st);
@@ -494,6 +496,13 @@ extern "C" int drr_project_jobs(drr_ctx *ctx, const drr_volume *const *vols, int
     if (e != hipSuccess) return drr_hip_error(e, "drr_project_jobs launch");
     if (e2 != hipSuccess) return drr_hip_error(e2, "drr_project_jobs");
     return DRR_OK;
+}
+
+extern "C" int drr_project_jobs(drr_ctx *ctx, const drr_volume *const *vols, int n_vols, const drr_job_t *jobs,
+                                int n_jobs, float *intensity, float *photon_prob, float *area_density,
+                                void *stream) {
+    return drr_project_jobs_march(ctx, vols, n_vols, jobs, n_jobs, ctx ? ctx->scene.march : DRR_MARCH_EXACT, intensity,
+                                  photon_prob, area_density, stream);
 }
 
 // ---- drr_project_jobs without device allocation ------------------------------

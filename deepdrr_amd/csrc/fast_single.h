@@ -34,10 +34,11 @@ namespace drr {
 
 // How a kernel marches a single-volume view.
 enum : int { MARCH_V1_EXACT, MARCH_V1_FAST, MARCH_V1_SINGLE };
-inline int march_v1_mode(const drr_ctx *ctx) {
-    if (ctx->scene.march != DRR_MARCH_FAST) return MARCH_V1_EXACT;
+inline int march_v1_mode(const drr_ctx *ctx, int march) {
+    if (march != DRR_MARCH_FAST) return MARCH_V1_EXACT;
     return ctx->single_sums ? MARCH_V1_SINGLE : MARCH_V1_FAST;
 }
+inline int march_v1_mode(const drr_ctx *ctx) { return march_v1_mode(ctx, ctx->scene.march); }
 // Coefficients of the trilinear interpolant of corner values (v0 = corners
 // 0..3, v1 = 4..7, corner d = dx + 2 dy + 4 dz) along the ray p(u) = p0 + u r
 // from fractions f = p0 - b: value(u) = ((k3 u + k2) u + k1) u + k0.

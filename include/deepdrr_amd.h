@@ -253,6 +253,11 @@ int drr_batch_destroy(drr_batch *batch);
  * starting at n_materials * out_offset -- what drr_adjoint_jobs can reuse. */
 int drr_project_jobs(drr_ctx *ctx, const drr_volume *const *vols, int n_vols, const drr_job_t *jobs,
                      int n_jobs, float *intensity, float *photon_prob, float *area_density, void *stream);
+/* drr_project_jobs with the march (DRR_MARCH_EXACT or DRR_MARCH_FAST) named by
+ * the call in place of the scene's. */
+int drr_project_jobs_march(drr_ctx *ctx, const drr_volume *const *vols, int n_vols, const drr_job_t *jobs,
+                           int n_jobs, int march, float *intensity, float *photon_prob, float *area_density,
+                           void *stream);
 
 /* drr_project_jobs for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid
