@@ -35,7 +35,12 @@
 // their own afterwards.  The materials' sums live in LDS, one word per lane and
 // material: an entry reads and writes the words its labels name, which in
 // registers takes a compare and a select per material and holds the
-// materials' registers and lane masks through the loop.  Nothing depends on
+// materials' registers and lane masks through the loop.  The record of the
+// cell after is loaded before the present one is summed: the wait for it was
+// most of a small launch, where no other wave fills it (one view of 256^2
+// through 128^3: 323 us without, 274 with; 16 views of 1536^2 through the
+// clinical CT: 97.2 ms, 86.4), and does nothing where VALU issue is the bound
+// (48 views of 765 x 768: 17.9 ms either way).  Nothing depends on
 // the launch or on other lanes, so results are the same from run to run and
 // from kernel to kernel.
 #pragma once
@@ -49,10 +54,10 @@ namespace drr {
 // with every sample added singly, 1.2e-5 at 128, 1.6e-5 at 204.8), at 17.5 ms
 // for 48 mixed views against 24.2 singly.
 constexpr float FAST_CLOSED_SUM = 102.4f;
-// Waves per SIMD of the kernels that march fast: 80 registers hold the entry
-// block (at 8 waves' 64 it spills: 6.1 ms against 5.6 on the clinical view; 7
-// waves: 5.8).
-constexpr int FAST_WAVES = 6;
+// Waves per SIMD of the kernels that march fast: 96 registers hold the entry
+// block and the record on its way (6 waves spill 16: 7.4 ms against 5.7 on the
+// clinical view; 4 waves: 5.7).
+constexpr int FAST_WAVES = 5;
 
 // A trilinear interpolant along the ray p(u) = p_m + u r as a cubic in u:
 // value(u) = ((c3 u + c2) u + c1) u + c0, from the lerps along x of the corner
@@ -145,12 +150,14 @@ __device__ __forceinline__ void fast_run(const VolDev &vol, float *acc, float sx
     float hz = riz == 0.0f ? hno : (riz < 0.0f ? 0.0f : jz);
     asm volatile("" : "+v"(jx), "+v"(jy), "+v"(jz), "+v"(hx), "+v"(hy), "+v"(hz));
     const float inc2_12 = inc * inc * (1.0f / 12.0f);
+    if (t >= tlim) return;
+    float px = sample_pos(sx, alpha, rix), py = sample_pos(sy, alpha, riy), pz = sample_pos(sz, alpha, riz);
+    Cell next;
+    next.load(vol, floorf(px), floorf(py), floorf(pz));
     while (t < tlim) {
         const float alpha0 = alpha;
-        const float px = sample_pos(sx, alpha, rix), py = sample_pos(sy, alpha, riy), pz = sample_pos(sz, alpha, riz);
-        const float bx = floorf(px), by = floorf(py), bz = floorf(pz);
-        Cell c;
-        c.load(vol, bx, by, bz);
+        const Cell c = next;
+        const float bx = c.bx, by = c.by, bz = c.bz;
         const float fx = px - bx, fy = py - by, fz = pz - bz;
         const float nex =
             fminf(__builtin_fmaf(-fx, jx, hx), fminf(__builtin_fmaf(-fy, jy, hy), __builtin_fmaf(-fz, jz, hz)));
@@ -163,6 +170,8 @@ __device__ __forceinline__ void fast_run(const VolDev &vol, float *acc, float sx
         const float nf = (float)n;
         const float um = inc * __builtin_fmaf(0.5f, nf, -0.5f);  // from the entry sample to the middle
         alpha = __builtin_fmaf(nf, inc, alpha);
+        px = sample_pos(sx, alpha, rix), py = sample_pos(sy, alpha, riy), pz = sample_pos(sz, alpha, riz);
+        next.load(vol, floorf(px), floorf(py), floorf(pz));
         const float mx = __builtin_fmaf(rix, um, fx), my = __builtin_fmaf(riy, um, fy), mz = __builtin_fmaf(riz, um, fz);
         // sum of u^2 over the samples
         const float S2 = inc2_12 * (nf * __builtin_fmaf(nf, nf, -1.0f));
