@@ -221,7 +221,7 @@ struct drr_batch_s {
 };
 
 template <int M, bool ATTEN, int TW, int MARCH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MARCH == MARCH_V1_FAST ? FAST_WAVES : MarchOcc<M + (ATTEN ? 1 : 0)>::waves)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MARCH == MARCH_V1_FAST ? FAST_WAVES : MARCH == MARCH_V1_SINGLE ? SINGLE_WAVES : MarchOcc<M + (ATTEN ? 1 : 0)>::waves)))
 void k_batch_march(const JobDev *__restrict__ jobs, const VolDev *__restrict__ vols,
                    const int2 *__restrict__ items, const int *__restrict__ seg, int *counters,
                    SpectrumDev sp, float step, int air, float *__restrict__ I, float *__restrict__ P,

@@ -6,9 +6,8 @@
 // out one photon off, and the image with noise moves by a hundred times what
 // the image without it does.  So views that feed the noise are marched with
 // the sums in the order in which they were always added, sample by sample,
-// and a seed's noise stays what it was; with fast_march.h's sums eight views
-// of 500 x 400 take 5.3 ms in place of 5.9, noise and all, but their noise
-// differs by 1.4e-4 of the image.
+// and a seed's noise stays what it was: with fast_march.h's sums that of eight
+// views of 500 x 400 differs by 1.4e-4 of the image.
 //
 // The samples t in [t, tlim), all of weight 1, have the same FP32 alpha sequence
 // as sample_v1 and, in cells whose labels agree, the same sequential FP32
@@ -26,11 +25,25 @@
 // label's fraction, also a cubic (single_run); a cell with more takes the exact
 // filter's formulas.  The sums stay within about 1e-7 relative of the exact
 // march's; nothing depends on the launch or on other lanes.
+//
+// VALU issue bounds it.  The sums live in LDS, one word per lane and material
+// (in registers the entry block took a compare and a select per material, and
+// their lane masks spilled 95 scalar registers through the loop), and a
+// sample's distance from the cell's first is k inc, with no alpha to follow:
+// 8 views of 500 x 400 through 256 x 256 x 300 march in 4.06 ms, 4.60 before.  The
+// next cell's record is loaded before this one's samples, for the small
+// launches, which wait for it (fast_march.h): 4 views of 356 x 225 through
+// 150 x 172 x 79 take 0.85 ms, 0.95 without.
 #pragma once
 
 #include "fast_march.h"
 
 namespace drr {
+
+// Waves per SIMD of the kernels that march so: 8 views of 500 x 400 take 4.06 ms at
+// 5 and 4.09 at 6 (with spills), 2 views of 299 x 102 0.87 and 0.91, 4 views of
+// 356 x 225 0.85 and 0.94.
+constexpr int SINGLE_WAVES = 5;
 
 // How a kernel marches a single-volume view.
 enum : int { MARCH_V1_EXACT, MARCH_V1_FAST, MARCH_V1_SINGLE };
@@ -64,103 +77,37 @@ __device__ __forceinline__ void cell_cubic(const float4 &v0, const float4 &v1, f
     k3 = rz * D2;
 }
 
-struct SingleCell {
-    // density = ((c3 u + c2) u + c1) u + c0 (single_run keeps the second label's
-    // corner indicators here instead in a two-label cell, zeros in a cell with more)
-    float c0 = 0.f, c1 = 0.f, c2 = 0.f, c3 = 0.f;
-    float a0 = 0.f;    // alpha of the entry sample (u = alpha - a0)
-    float nex = 0.f;   // distance to the exit face, in steps
-
-    // Enter cell c at alpha with fractions (fx, fy, fz) (those of the exact
-    // march) and the ray direction r in voxels per mm.  Per axis, the exit
-    // face is reached after fma(-f, j, h) steps with j = 1 / (r step) and
-    // h = j going up, 0 going down (j = 0, h = +inf where r = 0).
-    __device__ __forceinline__ void enter(const Cell &c, float alpha, float fx, float fy, float fz, float rx,
-                                          float ry, float rz, float jx, float jy, float jz, float hx, float hy,
-                                          float hz) {
-        a0 = alpha;
-        cell_cubic(c.d0, c.d1, fx, fy, fz, rx, ry, rz, c0, c1, c2, c3);
-        nex = fminf(__builtin_fmaf(-fx, jx, hx), fminf(__builtin_fmaf(-fy, jy, hy), __builtin_fmaf(-fz, jz, hz)));
-    }
-};
-
-// The samples of the entered cells (single_run): n for this lane, the density
-// cubic in fc (tw: a two-label cell, whose corner data fc and e hold instead)
-// and the two-label formulas where tw (TWO: some lane of the wave has a
-// two-label cell; the two forms are separate loops).
-template <bool TWO>
-__device__ __forceinline__ void single_cell(const Cell &c, const SingleCell &fc, Accum &a, float &sq, float e0,
-                                          float e1, float e2, float e3, bool tw, int n, float sx, float sy,
-                                          float sz, float rix, float riy, float riz, float step, float &alpha) {
-    float u = 0.0f;
-    for (int k = 0;; ++k) {
-        const bool in = k < n;
-        if (__ballot(in) == 0) break;
-        float rho = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(fc.c3, u, fc.c2), u, fc.c1), u, fc.c0);
-        const float g = in ? 1.0f : 0.0f;
-        if (TWO) {
-            // two labels: density and q-fraction at the sample's FP32 position
-            // (that of the exact filter), each by nested lerps
-            const float fx = __builtin_fmaf(alpha, rix, sx) - (c.bx + 1.0f);
-            const float fy = __builtin_fmaf(alpha, riy, sy) - (c.by + 1.0f);
-            const float fz = __builtin_fmaf(alpha, riz, sz) - (c.bz + 1.0f);
-            const float a00 = __builtin_fmaf(fx, c.d0.y - c.d0.x, c.d0.x);
-            const float a10 = __builtin_fmaf(fx, c.d0.w - c.d0.z, c.d0.z);
-            const float a01 = __builtin_fmaf(fx, c.d1.y - c.d1.x, c.d1.x);
-            const float a11 = __builtin_fmaf(fx, c.d1.w - c.d1.z, c.d1.z);
-            const float b0 = __builtin_fmaf(fy, a10 - a00, a00), b1 = __builtin_fmaf(fy, a11 - a01, a01);
-            const float x = __builtin_fmaf(fz, b1 - b0, b0);
-            const float i00 = __builtin_fmaf(fx, e0, fc.c0), i10 = __builtin_fmaf(fx, e1, fc.c1);
-            const float i01 = __builtin_fmaf(fx, e2, fc.c2), i11 = __builtin_fmaf(fx, e3, fc.c3);
-            const float j0 = __builtin_fmaf(fy, i10 - i00, i00), j1 = __builtin_fmaf(fy, i11 - i01, i01);
-            const float fq = __builtin_fmaf(fz, j1 - j0, j0);
-            const float xq = x * fq;
-            sq = __builtin_fmaf(g, tw ? xq : 0.0f, sq);
-            rho = tw ? x - xq : rho;
-        }
-        a.cur = __builtin_fmaf(g, rho, a.cur);
-        alpha = __builtin_fmaf(g, step, alpha);
-        u = alpha - fc.a0;
-    }
+// Of a two-label cell (tw): the second label's share of the density at the sample
+// at al, at its FP32 position (that of the exact filter), by nested lerps of the
+// densities and of the label's indicators (first corners v, differences e along
+// x); rho becomes the first label's.  Otherwise 0, and rho stays.
+__device__ __forceinline__ float second_share(const Cell &c, float al, float sx, float sy, float sz, float rix,
+                                              float riy, float riz, float v00, float v10, float v01, float v11,
+                                              float e00, float e10, float e01, float e11, float &rho, bool tw) {
+    const float fx = __builtin_fmaf(al, rix, sx) - (c.bx + 1.0f);
+    const float fy = __builtin_fmaf(al, riy, sy) - (c.by + 1.0f);
+    const float fz = __builtin_fmaf(al, riz, sz) - (c.bz + 1.0f);
+    const float a00 = __builtin_fmaf(fx, c.d0.y - c.d0.x, c.d0.x);
+    const float a10 = __builtin_fmaf(fx, c.d0.w - c.d0.z, c.d0.z);
+    const float a01 = __builtin_fmaf(fx, c.d1.y - c.d1.x, c.d1.x);
+    const float a11 = __builtin_fmaf(fx, c.d1.w - c.d1.z, c.d1.z);
+    const float b0 = __builtin_fmaf(fy, a10 - a00, a00), b1 = __builtin_fmaf(fy, a11 - a01, a01);
+    const float x = __builtin_fmaf(fz, b1 - b0, b0);
+    const float i00 = __builtin_fmaf(fx, e00, v00), i10 = __builtin_fmaf(fx, e10, v10);
+    const float i01 = __builtin_fmaf(fx, e01, v01), i11 = __builtin_fmaf(fx, e11, v11);
+    const float j0 = __builtin_fmaf(fy, i10 - i00, i00), j1 = __builtin_fmaf(fy, i11 - i01, i01);
+    const float xq = x * __builtin_fmaf(fz, j1 - j0, j0);
+    rho = tw ? x - xq : rho;
+    return tw ? xq : 0.0f;
 }
 
-// The samples of a cell with three or more labels (ex), after single_cell has
-// taken the cell's samples for the other lanes: the exact filter's formulas at
-// the same FP32 alpha sequence, re-walked from the entry sample a0, added into
-// ad[] sample by sample (the lane has no running sum in such a cell).
+// The samples t in [t, tlim), all of weight 1; on return alpha and t are those
+// after them.  a: the sums, every one of them in LDS (a.cur is not used), and in
+// a.cm the material whose sum the last cell's samples went to first.
 template <int M>
-__device__ __forceinline__ void single_exact(const Cell &c, float (&ad)[M], bool ex, int n, float a0, float sx,
-                                           float sy, float sz, float rix, float riy, float riz, float step) {
-    float al = a0;
-    for (int k = 0;; ++k) {
-        const bool in = (k < n) & ex;
-        if (__ballot(in) == 0) break;
-        if (in) {
-            const float fx = __builtin_fmaf(al, rix, sx) - (c.bx + 1.0f);
-            const float fy = __builtin_fmaf(al, riy, sy) - (c.by + 1.0f);
-            const float fz = __builtin_fmaf(al, riz, sz) - (c.bz + 1.0f);
-            float w[8];
-            weights8(fx, fy, fz, w);
-            const float x = trilerp(c.d0, c.d1, w);
-#pragma unroll
-            for (int m = 0; m < M; m++) {
-                const uint32_t xm = c.l0 ^ (0x11111111u * (uint32_t)m);
-                if (((xm - 0x11111111u) & ~xm & 0x88888888u) != 0u) {
-                    float sm = 0.0f;
-#pragma unroll
-                    for (int d = 0; d < 8; d++) sm += (corner_label(c.l0, c.l1, d) == (uint32_t)m) ? w[d] : 0.0f;
-                    ad[m] = __builtin_fmaf(x, sm, ad[m]);
-                }
-            }
-        }
-        al += step;
-    }
-}
-
-template <int M>
-__device__ __forceinline__ void single_run(const VolDev &vol, Cell &c, SingleCell &fc, float (&ad)[M], Accum &a,
-                                         float sx, float sy, float sz, float rix, float riy, float riz,
-                                         float step, float &alpha, int &t, int tlim, float amax) {
+__device__ __forceinline__ void single_run(const VolDev &vol, LdsAccum &a, bool &uni, float sx, float sy, float sz,
+                                           float rix, float riy, float riz, float step, float &alpha, int &t,
+                                           int tlim, float amax) {
     // Cell by cell: every lane still marching enters the cell of its current
     // sample together (one execution of the long cell-entry block for the whole
     // wave), then the wave runs the samples of those cells until every lane has
@@ -174,27 +121,23 @@ __device__ __forceinline__ void single_run(const VolDev &vol, Cell &c, SingleCel
     // density is continuous.  The inner loop's test is a wave vote and
     // its per-lane choices are 0/1 factors: per-lane branches and loop exits cost
     // scalar instructions (exec-mask bookkeeping), enough to become the limit in
-    // a loop this short.  With g = 1, fma(g, rho, cur) = cur + rho and
-    // fma(g, step, alpha) = alpha + step exactly; with g = 0 both leave the
-    // value unchanged.
+    // a loop this short.
     //
-    // Materials: a cell whose labels agree adds each sample's density to the
-    // running sum of its material (Accum).  A cell with exactly two labels
+    // Materials: a cell whose labels agree adds each sample's density to the sum
+    // of its material.  A cell with exactly two labels
     // (nearly every cell on a material boundary) forms each sample's density
     // and the fraction f_q of its second label q at the sample's FP32 position,
     // as the exact filter does (across a boundary the density changes by up to
     // several g/cm^3 per voxel, so that position's rounding shows at 1e-5 in
     // the sums, unlike in a cell of one material), each by nested lerps:
-    // rho (1 - f_q) goes to the running sum of the first material and rho f_q
-    // to a second running sum sq of ad[q], written back when q or the first
-    // material changes and when the run ends; so every term is still added into
-    // its material's area density one sample at a time, as the exact filter
-    // adds it.  A cell with three or more labels takes the exact filter's
-    // formulas, its density cubic set to zero.  In a wave with no two-label
+    // rho (1 - f_q) goes to the sum of the first material and rho f_q to that of
+    // q; the first is the one that the ray's last samples went to, if the cell
+    // has it.  A cell with three or more labels takes the exact filter's
+    // formulas.  In a wave with no two-label
     // cell the two-label formulas are skipped; a lane in a one-label cell
     // selects its cubic's value and adds zero to sq, so its results do not
     // depend on the other lanes.
-    if (__ballot(t < tlim) == 0) return;
+    if (t >= tlim) return;
     // exit distances in steps (reciprocals to 1 ulp are plenty there), kept in
     // registers (an empty asm stops the compiler from forming them again on
     // every cell entry)
@@ -226,85 +169,121 @@ __device__ __forceinline__ void single_run(const VolDev &vol, Cell &c, SingleCel
         hz = fac > 0.0f ? hz * fac : 0.0f;
     }
     asm volatile("" : "+v"(jx), "+v"(jy), "+v"(jz), "+v"(hx), "+v"(hy), "+v"(hz));
-    float sq = 0.0f;  // ad[q] while q (the second material of two-label cells) is >= 0
-    int q = -1;
-    // two labels: the q-indicators' x-differences (read only where tw, so not
-    // cleared for other cells)
-    float e0 = 0.f, e1 = 0.f, e2 = 0.f, e3 = 0.f;
-    do {
-        int n = 0;        // samples of the entered cell
-        bool ex = false;  // three or more labels: the exact filter
-        bool tw = false;  // two labels
-        if (t < tlim) {
-            const float px = sample_pos(sx, alpha, rix), py = sample_pos(sy, alpha, riy),
-                        pz = sample_pos(sz, alpha, riz);
-            const float bx = floorf(px), by = floorf(py), bz = floorf(pz);
-            c.load(vol, bx, by, bz);
-            const float fx = px - bx, fy = py - by, fz = pz - bz;
-            fc.enter(c, alpha, fx, fy, fz, rix, riy, riz, jx, jy, jz, hx, hy, hz);
-            int ncm = (int)c.l1;  // the first material (the common one in a one-label cell)
-            int qn = -1;          // the second material of a two-label cell
-            if (!c.uni) {
-                const uint32_t l0 = c.l0;
-                const uint32_t la = l0 & 0xfu;
-                const uint32_t xa = l0 ^ (la * 0x11111111u);  // nonzero nibbles: corners not la
-                const uint32_t lb = (l0 >> (__builtin_ctz(xa) & ~3u)) & 0xfu;
-                const uint32_t xb = l0 ^ (lb * 0x11111111u);
-                const uint32_t na = nz_nibbles(xa), nb = nz_nibbles(xb);
-                if ((na & nb) == 0u) {
-                    // the first material keeps the running sum when it already has it
-                    const bool sw = (int)lb == a.cm;
-                    ncm = (int)(sw ? lb : la);
-                    qn = (int)(sw ? la : lb);
-                    const uint32_t iq = sw ? na : nb;  // bit set: corner not q
-                    // q-indicators of the corners: bases of the x-lerps in fc.c0..c3,
-                    // their differences in e0..e3
-                    fc.c0 = (iq & 0x8u) ? 0.f : 1.f;
-                    fc.c1 = (iq & 0x800u) ? 0.f : 1.f;
-                    fc.c2 = (iq & 0x80000u) ? 0.f : 1.f;
-                    fc.c3 = (iq & 0x8000000u) ? 0.f : 1.f;
-                    e0 = ((iq & 0x80u) ? 0.f : 1.f) - fc.c0;
-                    e1 = ((iq & 0x8000u) ? 0.f : 1.f) - fc.c1;
-                    e2 = ((iq & 0x800000u) ? 0.f : 1.f) - fc.c2;
-                    e3 = ((iq & 0x80000000u) ? 0.f : 1.f) - fc.c3;
-                    tw = true;
-                } else {
-                    ex = true;
-                    fc.c0 = fc.c1 = fc.c2 = fc.c3 = 0.0f;
-                }
-            }
-            if (q >= 0 && (ncm != a.cm || (qn >= 0 && qn != q))) {
-                set_m<M>(ad, q, sq);
-                q = -1;
-            }
-            if (ncm != a.cm) {
-                if (a.cm >= 0) set_m<M>(ad, a.cm, a.cur);
-                a.cm = ncm;
-                a.cur = get_m<M>(ad, ncm);
-            }
-            if (qn >= 0 && q < 0) {
-                q = qn;
-                sq = get_m<M>(ad, qn);
-            }
-            // the samples before the exit face, clamped to [1, tlim - t] after
-            // the conversion (which saturates infinities and takes NaN to 0), so
-            // every entry takes at least one sample
-            n = min(max((int)ceilf(fc.nex), 1), tlim - t);
+    // alpha moves by inc from sample to sample while it stays below top (steps.h)
+    float inc = 0.0f, top = -INFINITY;
+    float px = sample_pos(sx, alpha, rix), py = sample_pos(sy, alpha, riy), pz = sample_pos(sz, alpha, riz);
+    Cell next;
+    next.load(vol, floorf(px), floorf(py), floorf(pz));
+    while (t < tlim) {
+        const float a0 = alpha;  // u = alpha - a0
+        if (!(a0 < top)) {
+            const float a1 = a0 + step, a2 = a1 + step;
+            inc = a1 - a0;
+            top = a2 - a1 == inc ? binade_top(a0) : a0;
         }
-        if (__ballot(tw) != 0)
-            single_cell<true>(c, fc, a, sq, e0, e1, e2, e3, tw, n, sx, sy, sz, rix, riy, riz, step, alpha);
-        else
-            single_cell<false>(c, fc, a, sq, e0, e1, e2, e3, tw, n, sx, sy, sz, rix, riy, riz, step, alpha);
-        if (__ballot(ex) != 0) single_exact<M>(c, ad, ex, n, fc.a0, sx, sy, sz, rix, riy, riz, step);
+        const Cell c = next;
+        const float bx = c.bx, by = c.by, bz = c.bz;
+        uni = c.uni;
+        const float fx = px - bx, fy = py - by, fz = pz - bz;
+        // density = ((c3 u + c2) u + c1) u + c0
+        float c0, c1, c2, c3;
+        cell_cubic(c.d0, c.d1, fx, fy, fz, rix, riy, riz, c0, c1, c2, c3);
+        // per axis, the exit face is reached after fma(-f, j, h) steps with
+        // j = 1 / (r step) and h = j going up, 0 going down (j = 0, h = +inf
+        // where r = 0)
+        const float nex =
+            fminf(__builtin_fmaf(-fx, jx, hx), fminf(__builtin_fmaf(-fy, jy, hy), __builtin_fmaf(-fz, jz, hz)));
+        // the samples before the exit face, clamped to [1, tlim - t] after
+        // the conversion (which saturates infinities and takes NaN to 0), so
+        // every entry takes at least one sample
+        int n = min(max((int)ceilf(nex), 1), tlim - t);
         t += n;
-    } while (__ballot(t < tlim) != 0);
-    if (q >= 0) set_m<M>(ad, q, sq);
-    // sample_v1 adds a mixed cell's terms into ad[] directly and expects no
-    // running sum there: write a two-label cell's first material back
-    if (!c.uni && a.cm >= 0) {
-        set_m<M>(ad, a.cm, a.cur);
-        a.cm = -1;
-        a.cur = 0.0f;
+        bool tw = false, ex = false;  // two labels; three or more
+        int m1 = (int)c.l1, m2 = 0;   // the first and second material
+        // two labels: the indicators of the second as lerps along x
+        float v00, v10, v01, v11, e00, e10, e01, e11;
+        if (!c.uni) {
+            const uint32_t l0 = c.l0;
+            const uint32_t la = l0 & 0xfu;
+            const uint32_t xa = l0 ^ (la * 0x11111111u);  // nonzero nibbles: corners not la
+            const uint32_t lb = (l0 >> (__builtin_ctz(xa) & ~3u)) & 0xfu;
+            const uint32_t xb = l0 ^ (lb * 0x11111111u);
+            const uint32_t na = nz_nibbles(xa), nb = nz_nibbles(xb);
+            tw = (na & nb) == 0u;
+            ex = !tw;
+            const bool sw = (int)lb == a.cm;
+            m1 = (int)(sw ? lb : la);
+            m2 = (int)(sw ? la : lb);
+            const uint32_t iq = sw ? na : nb;  // bit set: corner not the second
+            v00 = (iq & 0x8u) ? 0.f : 1.f;
+            v10 = (iq & 0x800u) ? 0.f : 1.f;
+            v01 = (iq & 0x80000u) ? 0.f : 1.f;
+            v11 = (iq & 0x8000000u) ? 0.f : 1.f;
+            e00 = ((iq & 0x80u) ? 0.f : 1.f) - v00;
+            e10 = ((iq & 0x8000u) ? 0.f : 1.f) - v10;
+            e01 = ((iq & 0x800000u) ? 0.f : 1.f) - v01;
+            e11 = ((iq & 0x80000000u) ? 0.f : 1.f) - v11;
+            a.cm = ex ? -1 : m1;
+        } else {
+            a.cm = m1;
+        }
+        float *pa = a.sums + LDS_LANES * m1, *pb = a.sums + LDS_LANES * m2;
+        float cur = *pa, sq = *pb;
+        alpha = __builtin_fmaf((float)n, inc, a0);
+        px = sample_pos(sx, alpha, rix), py = sample_pos(sy, alpha, riy), pz = sample_pos(sz, alpha, riz);
+        next.load(vol, floorf(px), floorf(py), floorf(pz));
+        const bool even = alpha <= top;  // alpha - a0 is k inc at the cell's k-th sample, exactly
+        const int ne = even & !ex ? n : 0;
+        // (with g = 1, fma(g, rho, cur) = cur + rho exactly; with 0 it stays)
+        if (__ballot(tw) != 0) {
+            float u = 0.0f, al = a0;
+            for (int k = 0;; ++k) {
+                const bool in = k < ne;
+                if (__ballot(in) == 0) break;
+                const float g = in ? 1.0f : 0.0f;
+                float rho = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(c3, u, c2), u, c1), u, c0);
+                const float xq = second_share(c, al, sx, sy, sz, rix, riy, riz, v00, v10, v01, v11, e00, e10, e01, e11, rho, tw);
+                sq = __builtin_fmaf(g, xq, sq);
+                cur = __builtin_fmaf(g, rho, cur);
+                u += inc;
+                al += inc;
+            }
+        } else {
+            float u = 0.0f;
+            for (int k = 0;; ++k) {
+                const bool in = k < ne;
+                if (__ballot(in) == 0) break;
+                const float rho = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(c3, u, c2), u, c1), u, c0);
+                cur = __builtin_fmaf(in ? 1.0f : 0.0f, rho, cur);
+                u += inc;
+            }
+        }
+        if (!even) {  // across a binade's top, step by step
+            alpha = a0;
+            for (int k = 0; k < n; ++k) {
+                const float u = alpha - a0;
+                float rho = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(c3, u, c2), u, c1), u, c0);
+                const float xq = second_share(c, alpha, sx, sy, sz, rix, riy, riz, v00, v10, v01, v11, e00, e10, e01, e11, rho, tw);
+                sq += xq;
+                cur += rho;
+                alpha += step;
+            }
+            px = sample_pos(sx, alpha, rix), py = sample_pos(sy, alpha, riy), pz = sample_pos(sz, alpha, riz);
+            next.load(vol, floorf(px), floorf(py), floorf(pz));
+        }
+        if (tw) *pb = sq;
+        if (ex) {
+            float al = a0;
+            for (int k = 0; k < n; ++k) {
+                float w[8];
+                weights8(__builtin_fmaf(al, rix, sx) - (bx + 1.0f), __builtin_fmaf(al, riy, sy) - (by + 1.0f),
+                         __builtin_fmaf(al, riz, sz) - (bz + 1.0f), w);
+                add_mixed(a.sums, c.l0, w, trilerp(c.d0, c.d1, w));
+                al += step;
+            }
+        } else {
+            *pa = cur;
+        }
     }
 }
 
@@ -312,11 +291,10 @@ __device__ __forceinline__ void single_run(const VolDev &vol, Cell &c, SingleCel
 // On return ad[] holds the final area densities in g/cm^2.
 template <int M, bool ATTEN>
 __device__ __forceinline__ void march_fast_single(const Geo1 &g, const VolDev &vol, int udx, int vdx,
-                                                  float step, int air, float (&ad)[M]) {
+                                                  float step, int air, float *sums, float (&ad)[M]) {
     RayV1 r;
     march_setup_v1(g, udx, vdx, step, r);
-#pragma unroll
-    for (int m = 0; m < M; m++) ad[m] = 0.0f;
+    for (int m = 0; m < M; m++) sums[LDS_LANES * m] = 0.0f;
     float acc = 0.0f;  // air accumulator while no volume is sampled
     if (ATTEN) acc = (float)((double)acc + (double)(r.minA / step) * DRR_AIR_DENSITY);
 
@@ -343,18 +321,15 @@ __device__ __forceinline__ void march_fast_single(const Geo1 &g, const VolDev &v
             alpha += step;
             ++t;
         }
-        if (ATTEN) set_m<M>(ad, air, acc);
+        if (ATTEN) sums[LDS_LANES * air] = acc;
         // Phase 3: inside [minAlpha_vol, maxAlpha_vol]: sample and accumulate.
         // While the ray is in a cell whose 8 labels agree (material m0), only
         // ad[m0] changes; it is kept in `cur` and written back on leaving, so
         // every FP32 addition is the one the reference performs.  The end
         // samples t == 0 and t == N-1 carry weight 0.5 (project_kernel.cu:
         // 541), the others 1.
-        Accum acc3;
-        if (c.have && c.uni) {
-            acc3.cm = (int)c.l1;
-            acc3.cur = get_m<M>(ad, acc3.cm);
-        }
+        LdsAccum acc3{sums};
+        if (c.have && c.uni) acc3.open((int)c.l1);
         // The loop runs while t < tlim with no test on alpha: tlim is at most
         // the last weight-1 sample (N - 2) and at most the samples whose alpha
         // is certainly <= maxAlpha_vol.  Each FP32 `alpha += step` adds at
@@ -370,16 +345,27 @@ __device__ __forceinline__ void march_fast_single(const Geo1 &g, const VolDev &v
         // integers, where (float)(N - 1 - t) could round up)
         int tlim = min(t + (int)__builtin_amdgcn_fmed3f(kf, 0.0f, 16777216.0f), N - 1);
         for (;;) {
-            // a sample of weight 0.5 (the first) takes the exact filter
+            // a sample of weight 0.5 (the first, the last) takes the exact filter
             if (wt != 1.0f && t < tlim) {
-                sample_v1<M>(vol, c, ad, acc3, sample_pos(sx, alpha, rix), sample_pos(sy, alpha, riy),
-                             sample_pos(sz, alpha, riz), wt);
+                sample_lds(vol, c, acc3, sample_pos(sx, alpha, rix), sample_pos(sy, alpha, riy),
+                           sample_pos(sz, alpha, riz), wt);
                 wt = 1.0f;
                 alpha += step;
                 ++t;
             }
-            SingleCell fc;  // no cell entered: the first sample enters one
-            single_run<M>(vol, c, fc, ad, acc3, sx, sy, sz, rix, riy, riz, step, alpha, t, tlim, r.mxv);
+            if (t < tlim) {
+                const int m = acc3.cm;
+                acc3.open(-1);  // every sum to LDS
+                acc3.cm = m;
+                bool uni = true;
+                single_run<M>(vol, acc3, uni, sx, sy, sz, rix, riy, riz, step, alpha, t, tlim, r.mxv);
+                // the next sample enters its cell anew; a running sum goes on only in
+                // a material whose samples were one label's
+                const int cm = uni ? acc3.cm : -1;
+                acc3.cm = -1;
+                acc3.open(cm);
+                c = Cell{};
+            }
             // a fresh comparison after the loop (an empty asm hides alpha's
             // in-loop history), so the loop does not carry one
             asm volatile("" : "+v"(alpha));
@@ -387,17 +373,17 @@ __device__ __forceinline__ void march_fast_single(const Geo1 &g, const VolDev &v
             if (t == N - 1) wt = 0.5f;
             tlim = t + 1;
         }
-        if (acc3.cm >= 0) set_m<M>(ad, acc3.cm, acc3.cur);
-        if (ATTEN) acc = get_m<M>(ad, air);
+        acc3.open(-1);
+        if (ATTEN) acc = sums[LDS_LANES * air];
     }
     // Phase 4: the rest of the steps sample nothing.
     if (ATTEN) {
         air_steps(N - t, acc);
         acc = (float)((double)acc + (double)((r.L - r.maxA) / step) * DRR_AIR_DENSITY);
-        set_m<M>(ad, air, acc);
+        sums[LDS_LANES * air] = acc;
     }
 #pragma unroll
-    for (int m = 0; m < M; m++) ad[m] *= step;
+    for (int m = 0; m < M; m++) ad[m] = sums[LDS_LANES * m] * step;
 #pragma unroll
     for (int m = 0; m < M; m++) ad[m] /= 10.0f;
 }
@@ -406,11 +392,12 @@ __device__ __forceinline__ void march_fast_single(const Geo1 &g, const VolDev &v
 template <int M, bool ATTEN, int MARCH>
 __device__ __forceinline__ void march_single_volume(const Geo1 &g, const VolDev &vol, int udx, int vdx, float step,
                                                     int air, float (&ad)[M]) {
-    if constexpr (MARCH == MARCH_V1_FAST) {
+    if constexpr (MARCH != MARCH_V1_EXACT) {
         __shared__ float sums[M * LDS_LANES];  // each thread its own words
-        march_fast<M, ATTEN>(g, vol, udx, vdx, step, air, sums + threadIdx.x, ad);
-    } else if constexpr (MARCH == MARCH_V1_SINGLE) {
-        march_fast_single<M, ATTEN>(g, vol, udx, vdx, step, air, ad);
+        if constexpr (MARCH == MARCH_V1_FAST)
+            march_fast<M, ATTEN>(g, vol, udx, vdx, step, air, sums + threadIdx.x, ad);
+        else
+            march_fast_single<M, ATTEN>(g, vol, udx, vdx, step, air, sums + threadIdx.x, ad);
     } else {
         march_v1<M, ATTEN>(g, vol, udx, vdx, step, air, ad);
     }

@@ -79,7 +79,7 @@ struct OutDev {
 };
 
 template <int M, bool ATTEN, int MARCH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MARCH == MARCH_V1_FAST ? FAST_WAVES : MarchOcc<M>::waves))) void k_project_v1(Geo1 g, VolDev vol, SpectrumDev sp, float step,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MARCH == MARCH_V1_FAST ? FAST_WAVES : MARCH == MARCH_V1_SINGLE ? SINGLE_WAVES : MarchOcc<M>::waves))) void k_project_v1(Geo1 g, VolDev vol, SpectrumDev sp, float step,
                                                     int air, OutDev out, int tiles16_x) {
     const int lb = blockIdx.x;
     const int bx = lb % tiles16_x, by = lb / tiles16_x;
