@@ -36,6 +36,7 @@ struct drr_volume_s {
 
 struct drr_ctx_s {
     int device = 0;
+    int n_cus = 0;  // compute units
     drr_scene_t scene{0.1f, 0, 0, 0, DRR_MARCH_EXACT};
     bool have_scene = false;
     bool single_sums = false;  // the fast march adds every sample singly (drr_ctx_set_single_sums)

@@ -71,6 +71,18 @@ int drr_launch_expand(const float *density, const uint8_t *labels, int nx, int n
 // each XCD a contiguous band of its own (for L2 locality) made the XCDs with
 // the central bands finish last -- 4-8% slower at 1536^2, measured.
 
+// Rows of a wave's 8-pixel-wide tile: 8, or 4 where an exactly marched view has
+// at most ten waves of 8 rows per CU.  Such a launch takes as long as its
+// slowest wave, which waits for a cell record at every step where one of its
+// rays changes cells; half a wave's rays do so at fewer steps.  Through 128^3,
+// 256^2 (4 waves per CU): 779 us, 692 with 4 rows (690 with 2); 384^2: 748, 715;
+// 512^2 (16): 771, 846.  389 x 323 through 201 x 180 x 151 (8): 1216, 1118 (1291
+// with 2).  The fast march enters its cells together anyhow: 256^2 265, 259;
+// 384^2 262, 275.
+static int wave_rows(int march, int64_t waves, int cus) {
+    return march == MARCH_V1_EXACT && waves <= (int64_t)10 * cus ? 4 : 8;
+}
+
 struct OutDev {
     float *intensity;
     float *photon_prob;
@@ -80,13 +92,12 @@ struct OutDev {
 
 template <int M, bool ATTEN, int MARCH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MARCH == MARCH_V1_FAST ? FAST_WAVES : MARCH == MARCH_V1_SINGLE ? SINGLE_WAVES : MarchOcc<M>::waves))) void k_project_v1(Geo1 g, VolDev vol, SpectrumDev sp, float step,
-                                                    int air, OutDev out, int tiles16_x) {
+                                                    int air, OutDev out, int tiles16_x, int rows) {
     const int lb = blockIdx.x;
     const int bx = lb % tiles16_x, by = lb / tiles16_x;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    int udx, vdx;
-    lane_pixel(bx * 2 + (wave & 1), by * 2 + (wave >> 1), lane, udx, vdx);
-    if (udx >= g.width || vdx >= g.height) return;
+    const int udx = bx * 16 + (wave & 1) * 8 + (lane & 7), vdx = (by * 2 + (wave >> 1)) * rows + (lane >> 3);
+    if (lane >= 8 * rows || udx >= g.width || vdx >= g.height) return;
     float ad[M];
     march_single_volume<M, ATTEN, MARCH>(g, vol, udx, vdx, step, air, ad);
     float I, P;
@@ -130,13 +141,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI_WAVES
 
 template <int M>
 static void launch_v1(bool atten, int march, dim3 g, dim3 b, hipStream_t st, const Geo1 &geo, const VolDev &vol,
-                      const SpectrumDev &sp, float step, int air, const OutDev &o, int tx) {
+                      const SpectrumDev &sp, float step, int air, const OutDev &o, int tx, int rows) {
 #define DRR_MARCH_CASE(MARCH)                                                                    \
     case MARCH:                                                                                  \
         if (atten)                                                                               \
-            k_project_v1<M, true, MARCH><<<g, b, 0, st>>>(geo, vol, sp, step, air, o, tx);       \
+            k_project_v1<M, true, MARCH><<<g, b, 0, st>>>(geo, vol, sp, step, air, o, tx, rows);  \
         else                                                                                     \
-            k_project_v1<M, false, MARCH><<<g, b, 0, st>>>(geo, vol, sp, step, air, o, tx);      \
+            k_project_v1<M, false, MARCH><<<g, b, 0, st>>>(geo, vol, sp, step, air, o, tx, rows); \
         break;
     switch (march) {
         DRR_MARCH_CASE(MARCH_V1_EXACT) DRR_MARCH_CASE(MARCH_V1_FAST) DRR_MARCH_CASE(MARCH_V1_SINGLE)
@@ -177,13 +188,15 @@ extern "C" int drr_project(drr_ctx *ctx, const drr_volume *const *vols, const dr
     const drr_scene_t &sc = ctx->scene;
     const int tx = (view->width + 15) / 16, ty = (view->height + 15) / 16;
     dim3 grid((unsigned)(tx * ty)), block(256);
+    const int rows = wave_rows(march_v1_mode(ctx), (int64_t)tx * ty * 4, ctx->n_cus);
+    const dim3 grid1((unsigned)(tx * ((view->height + 2 * rows - 1) / (2 * rows))));
     (void)hipEventRecord(ctx->ev0, st);
     if (view->n_volumes == 1) {
         switch (sc.n_materials) {
 #define DRR_CASE(MM) \
     case MM:                                                                                           \
-        launch_v1<MM>(sc.attenuate_outside != 0, march_v1_mode(ctx), grid, block, st, geo, vol0, sp, \
-                      sc.step, sc.air_index, o, tx);                                                     \
+        launch_v1<MM>(sc.attenuate_outside != 0, march_v1_mode(ctx), grid1, block, st, geo, vol0, sp, \
+                      sc.step, sc.air_index, o, tx, rows);                                               \
         break;
             DRR_CASE(1) DRR_CASE(2) DRR_CASE(3) DRR_CASE(4) DRR_CASE(5) DRR_CASE(6) DRR_CASE(7) DRR_CASE(8) \
         DRR_CASE(9) DRR_CASE(10) DRR_CASE(11) DRR_CASE(12) DRR_CASE(13) DRR_CASE(14) DRR_CASE(15) DRR_CASE(16)

@@ -85,7 +85,8 @@ int drr_ctx_create(int device_id, drr_ctx **out) {
     if (!g.ok) return drr_set_error(DRR_ERR_HIP, "drr_ctx_create: hipSetDevice failed");
     drr_ctx *c = new drr_ctx();
     c->device = device_id;
-    if (hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
+    if (hipDeviceGetAttribute(&c->n_cus, hipDeviceAttributeMultiprocessorCount, device_id) != hipSuccess ||
+        hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
         delete c;
         return drr_set_error(DRR_ERR_HIP, "drr_ctx_create: hipEventCreate failed");
     }
