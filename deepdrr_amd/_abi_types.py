@@ -110,7 +110,7 @@ def make_view(world_from_index, width, height, max_ray_length, vols, allow_empty
     bounds_hi(3), priority, enabled (none only with ``allow_empty``, a scene of
     meshes alone)."""
     v = View()
-    v.world_from_index[:] = [float(x) for x in np.asarray(world_from_index, np.float32).reshape(9)]
+    v.world_from_index[:] = np.asarray(world_from_index, np.float32).reshape(9).tolist()
     v.max_ray_length = float(np.float32(max_ray_length))
     v.width = int(width)
     v.height = int(height)
@@ -119,10 +119,10 @@ def make_view(world_from_index, width, height, max_ray_length, vols, allow_empty
     v.n_volumes = len(vols)
     for i, d in enumerate(vols):
         vv = v.vol[i]
-        vv.ijk_from_world[:] = [float(x) for x in np.asarray(d["ijk_from_world"], np.float32).reshape(12)]
-        vv.source_ijk[:] = [float(x) for x in np.asarray(d["source_ijk"], np.float32).reshape(3)]
-        vv.bounds_lo[:] = [float(x) for x in np.asarray(d["bounds_lo"], np.float32).reshape(3)]
-        vv.bounds_hi[:] = [float(x) for x in np.asarray(d["bounds_hi"], np.float32).reshape(3)]
+        vv.ijk_from_world[:] = np.asarray(d["ijk_from_world"], np.float32).reshape(12).tolist()
+        vv.source_ijk[:] = np.asarray(d["source_ijk"], np.float32).reshape(3).tolist()
+        vv.bounds_lo[:] = np.asarray(d["bounds_lo"], np.float32).reshape(3).tolist()
+        vv.bounds_hi[:] = np.asarray(d["bounds_hi"], np.float32).reshape(3).tolist()
         vv.priority = int(d["priority"])
         vv.enabled = int(d["enabled"])
     return v

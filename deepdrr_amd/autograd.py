@@ -25,7 +25,7 @@ import numpy as np
 from . import _abi, geo
 from ._abi_types import MARCH_FAST, Job, Scene, make_view
 from .material import attenuation_table
-from .projector import world_from_index_rows
+from .projector import cameras
 from .spectral_data import get_spectrum, spectrum_tables
 
 
@@ -65,8 +65,9 @@ class PoseGeometry:
         w_from_ijk = T @ self.world_from_ijk
         ijk_from_w = np.linalg.inv(w_from_ijk)
         out = []
-        for proj in projections:
-            src = np.array(proj.center_in_world)
+        if not projections:
+            return out
+        for proj, rows, src in zip(projections, *cameras(projections, 1.0)):
             s_ijk = (ijk_from_w @ np.append(src, 1.0))[:3]
             w, h = proj.intrinsic.sensor_size
             vol = dict(ijk_from_world=ijk_from_w[:3].astype(np.float32).reshape(12),
@@ -74,7 +75,7 @@ class PoseGeometry:
                        bounds_lo=np.full(3, -0.5, np.float32),
                        bounds_hi=np.array([s - 0.5 for s in self.shape], np.float32),
                        priority=0, enabled=1)
-            out.append((make_view(world_from_index_rows(proj, 1.0), w, h, self.max_ray_length, [vol]),
+            out.append((make_view(rows, w, h, self.max_ray_length, [vol]),
                         src.astype(np.float32)))
         return out
 

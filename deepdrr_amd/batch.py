@@ -175,24 +175,18 @@ def plan_for_projector(projector, projections: Sequence[geo.CameraProjection],
                        volume_indices: Optional[Sequence[int]] = None, neglog: Optional[bool] = None,
                        tuning=None) -> BatchPlan:
     """Batch plan over an initialised ``Projector``'s volumes."""
-    from .projector import build_view
+    from .projector import build_views
 
     if not projector.initialized:
         raise RuntimeError("Projector has not been initialized.")
     if not hasattr(projector, "max_ray_length"):
         projector.max_ray_length = projector.source_to_detector_distance * 4
-    views = []
     sdd = projector.source_to_detector_distance
+    views = build_views(projector.volumes, projector.priorities, projections, projector.max_ray_length,
+                        sdd if sdd > 0 else 1.0, which=volume_indices)
     if volume_indices is None:
         # every view over all the projector's volumes, as project() renders it
         volume_indices = [0] * len(projections)
-        for proj in projections:
-            views.append(build_view(projector.volumes, projector.priorities, proj, projector.max_ray_length,
-                                    sdd if sdd > 0 else 1.0))
-    else:
-        for proj, vi in zip(projections, volume_indices):
-            views.append(build_view([projector.volumes[vi]], [projector.priorities[vi]], proj,
-                                    projector.max_ray_length, sdd if sdd > 0 else 1.0))
     key = None
     if tuning == "auto":
         from . import autotune

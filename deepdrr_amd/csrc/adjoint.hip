@@ -23,6 +23,9 @@
 // touched voxel.
 #include <hip/hip_runtime.h>
 
+#include <cstring>
+#include <vector>
+
 #include "drr_internal.h"
 #include "jobs.h"
 #include "march.h"
@@ -624,10 +627,6 @@ __global__ __launch_bounds__(256) void k_adjoint_v1(Geo1 g, VolDev vol, Spectrum
     if (POSE) flush_pose_wave(gpose, a.gPose);
 }
 
-__global__ void k_pose_zero(double *acc) {
-    if (threadIdx.x < 6) acc[threadIdx.x] = 0.0;
-}
-
 __global__ void k_pose_finish(const double *acc, float *gPose) {
     if (threadIdx.x < 6) gPose[threadIdx.x] += (float)acc[threadIdx.x];
 }
@@ -957,21 +956,13 @@ extern "C" int drr_adjoint_jobs(drr_ctx *ctx, const drr_volume *vol, const drr_j
     const bool pose = grad_pose != nullptr;
     const int blocks_per_cu = pose ? AdjOcc<1>::waves : AdjOcc<0>::waves;  // pose only: 4, as with density
     const drr_batch_tuning_t tune{ADJ_TILE, ADJ_TILE, 4, blocks_per_cu};
-    rc = drr_jobs_build_tiles(ctx, vols, 1, jobs, n_jobs, tune, t);
+    // beside the tables: FP64 pose accumulator [6], then the job sources [3 * n_jobs]
+    std::vector<char> extra(sizeof(double) * 6 + sizeof(float) * 3 * n_jobs, 0);
+    if (source_world) std::memcpy(extra.data() + sizeof(double) * 6, source_world, sizeof(float) * 3 * n_jobs);
+    rc = drr_jobs_build_tiles(ctx, vols, 1, jobs, n_jobs, tune, t, extra.data(), extra.size());
     if (rc != DRR_OK) return rc;
-    // scratch: FP64 pose accumulator [6], then the job sources [3 * n_jobs]
-    double *d_pose64 = nullptr;
-    hipError_t e = hipMalloc(&d_pose64, sizeof(double) * 6 + sizeof(float) * 3 * n_jobs);
-    float *d_sw = e == hipSuccess ? reinterpret_cast<float *>(d_pose64 + 6) : nullptr;
-    if (e == hipSuccess && source_world)
-        e = hipMemcpy(d_sw, source_world, sizeof(float) * 3 * n_jobs, hipMemcpyHostToDevice);
-    else if (e == hipSuccess)
-        e = hipMemset(d_sw, 0, sizeof(float) * 3 * n_jobs);
-    if (e != hipSuccess) {
-        drr_jobs_free(t);
-        (void)hipFree(d_pose64);
-        return drr_hip_error(e, "drr_adjoint_jobs: scratch");
-    }
+    double *d_pose64 = static_cast<double *>(t.d_extra);
+    float *d_sw = reinterpret_cast<float *>(d_pose64 + 6);
     const VolDev v = vol_to_dev(vol);
     SpectrumDev sp{ctx->d_energies, ctx->d_pdf, ctx->d_mu, ctx->n_bins};
     AdjArgs a{};
@@ -985,7 +976,6 @@ extern "C" int drr_adjoint_jobs(drr_ctx *ctx, const drr_volume *vol, const drr_j
     hipStream_t st = (hipStream_t)stream;
     (void)hipEventRecord(ctx->ev0, st);
     k_jobs_reset<<<1, 64, 0, st>>>(t.d_counters);
-    if (pose) k_pose_zero<<<1, 64, 0, st>>>(d_pose64);
     switch (sc.n_materials) {
 #define DRR_CASE(MM)                                                                                  \
     case MM:                                                                                          \
@@ -999,12 +989,11 @@ extern "C" int drr_adjoint_jobs(drr_ctx *ctx, const drr_volume *vol, const drr_j
 #undef DRR_CASE
     }
     if (pose) k_pose_finish<<<1, 64, 0, st>>>(d_pose64, grad_pose);
-    e = hipGetLastError();
+    hipError_t e = hipGetLastError();
     (void)hipEventRecord(ctx->ev1, st);
     ctx->timed = true;
     hipError_t e2 = hipStreamSynchronize(st);
     drr_jobs_free(t);
-    (void)hipFree(d_pose64);
     if (prev >= 0 && prev != ctx->device) (void)hipSetDevice(prev);
     if (e != hipSuccess) return drr_hip_error(e, "drr_adjoint_jobs launch");
     if (e2 != hipSuccess) return drr_hip_error(e2, "drr_adjoint_jobs");

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstring>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -25,25 +26,11 @@ __global__ void k_jobs_reset(int *counters) {
     if (threadIdx.x < 8) counters[threadIdx.x] = 0;
 }
 
-void drr_jobs_free(JobTable &t) {
-    (void)hipFree(t.d_jobs);
-    (void)hipFree(t.d_vols);
-    (void)hipFree(t.d_items);
-    (void)hipFree(t.d_seg);
-    (void)hipFree(t.d_counters);
-    (void)hipFree(t.d_mjobs);
-    (void)hipFree(t.d_mitems);
-    t.d_jobs = nullptr;
-    t.d_vols = nullptr;
-    t.d_items = nullptr;
-    t.d_seg = nullptr;
-    t.d_counters = nullptr;
-    t.d_mjobs = nullptr;
-    t.d_mitems = nullptr;
-}
+void drr_jobs_free(JobTable &t) { t.buf.reset(); }
 
 static int jobs_build_impl(drr_ctx *ctx, const drr_volume *const *vols, int n_vols, const drr_job_t *jobs,
-                           int n_jobs, const drr_batch_tuning_t &tune, bool allow_multi, JobTable &t);
+                           int n_jobs, const drr_batch_tuning_t &tune, bool allow_multi, JobTable &t,
+                           const void *extra, size_t extra_bytes);
 
 int drr_jobs_build(drr_ctx *ctx, const drr_volume *const *vols, int n_vols, const drr_job_t *jobs,
                    int n_jobs, const drr_batch_tuning_t &tune, JobTable &t) {
@@ -51,7 +38,7 @@ int drr_jobs_build(drr_ctx *ctx, const drr_volume *const *vols, int n_vols, cons
         return drr_set_error(DRR_ERR_INVALID, "jobs: tile must be 8x8 or 16x4");
     if (tune.waves_per_block < 1 || tune.waves_per_block > 4 || tune.blocks_per_cu < 1 || tune.blocks_per_cu > 32)
         return drr_set_error(DRR_ERR_INVALID, "jobs: waves_per_block in [1,4], blocks_per_cu in [1,32]");
-    return jobs_build_impl(ctx, vols, n_vols, jobs, n_jobs, tune, true, t);
+    return jobs_build_impl(ctx, vols, n_vols, jobs, n_jobs, tune, true, t, nullptr, 0);
 }
 
 namespace {
@@ -156,51 +143,63 @@ int jobs_prepare(drr_ctx *ctx, const drr_volume *const *vols, int n_vols, const 
     for (int q = 0; q <= 8; q++) h.seg[q] = (int)(t.n_items * q / 8);
     h.vols.resize(n_vols);
     for (int v = 0; v < n_vols; v++) h.vols[v] = vol_to_dev(vols[v]);
-    int cus = 0;
-    hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device);
-    if (e != hipSuccess) return drr_hip_error(e, "hipDeviceGetAttribute(multiprocessor count)");
     t.block = 64 * tune.waves_per_block;
-    t.grid = cus * tune.blocks_per_cu;
+    t.grid = ctx->n_cus * tune.blocks_per_cu;
     return DRR_OK;
 }
 }  // namespace
 
 int drr_jobs_build_tiles(drr_ctx *ctx, const drr_volume *const *vols, int n_vols, const drr_job_t *jobs,
-                         int n_jobs, const drr_batch_tuning_t &tune, JobTable &t) {
-    return jobs_build_impl(ctx, vols, n_vols, jobs, n_jobs, tune, false, t);
+                         int n_jobs, const drr_batch_tuning_t &tune, JobTable &t, const void *extra,
+                         size_t extra_bytes) {
+    return jobs_build_impl(ctx, vols, n_vols, jobs, n_jobs, tune, false, t, extra, extra_bytes);
 }
 
+namespace {
+constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
+}  // namespace
+
+// The tables of one call lie in one buffer and go there in one copy, 256-B
+// aligned: counters | segments | volumes | jobs | multi-volume jobs | extra |
+// tiles (single-volume, then multi-volume).
 static int jobs_build_impl(drr_ctx *ctx, const drr_volume *const *vols, int n_vols, const drr_job_t *jobs,
-                           int n_jobs, const drr_batch_tuning_t &tune, bool allow_multi, JobTable &t) {
+                           int n_jobs, const drr_batch_tuning_t &tune, bool allow_multi, JobTable &t,
+                           const void *extra, size_t extra_bytes) {
     JobHost h;
     int rc = jobs_prepare(ctx, vols, n_vols, jobs, n_jobs, tune, -1, "jobs", allow_multi, t, h);
     if (rc != DRR_OK) return rc;
-    hipError_t e;
-#define JCHK(x)                                             \
-    do {                                                    \
-        e = (x);                                            \
-        if (e != hipSuccess) {                              \
-            drr_jobs_free(t);                               \
-            return drr_hip_error(e, #x);                    \
-        }                                                   \
-    } while (0)
-    JCHK(hipMalloc(&t.d_jobs, sizeof(JobDev) * n_jobs));
-    JCHK(hipMalloc(&t.d_vols, sizeof(VolDev) * n_vols));
-    JCHK(hipMalloc(&t.d_items, sizeof(int2) * std::max<size_t>(1, h.items.size())));
-    JCHK(hipMalloc(&t.d_seg, sizeof(int) * 9));
-    JCHK(hipMalloc(&t.d_counters, sizeof(int) * 8));
-    JCHK(hipMemcpy(t.d_jobs, h.jobs.data(), sizeof(JobDev) * n_jobs, hipMemcpyHostToDevice));
-    JCHK(hipMemcpy(t.d_vols, h.vols.data(), sizeof(VolDev) * n_vols, hipMemcpyHostToDevice));
-    if (!h.items.empty())
-        JCHK(hipMemcpy(t.d_items, h.items.data(), sizeof(int2) * h.items.size(), hipMemcpyHostToDevice));
-    JCHK(hipMemcpy(t.d_seg, h.seg, sizeof(int) * 9, hipMemcpyHostToDevice));
-    if (!h.mjobs.empty()) {
-        JCHK(hipMalloc(&t.d_mjobs, sizeof(JobMultiDev) * h.mjobs.size()));
-        JCHK(hipMalloc(&t.d_mitems, sizeof(int2) * h.mitems.size()));
-        JCHK(hipMemcpy(t.d_mjobs, h.mjobs.data(), sizeof(JobMultiDev) * h.mjobs.size(), hipMemcpyHostToDevice));
-        JCHK(hipMemcpy(t.d_mitems, h.mitems.data(), sizeof(int2) * h.mitems.size(), hipMemcpyHostToDevice));
+    const size_t off_seg = 256, off_vols = 512;
+    const size_t off_jobs = align256(off_vols + sizeof(VolDev) * h.vols.size());
+    const size_t off_mjobs = align256(off_jobs + sizeof(JobDev) * h.jobs.size());
+    const size_t off_extra = align256(off_mjobs + sizeof(JobMultiDev) * h.mjobs.size());
+    const size_t off_items = align256(off_extra + extra_bytes);
+    const size_t n_items = h.items.size() + h.mitems.size(), bytes = off_items + sizeof(int2) * n_items;
+    hipError_t e = t.buf.take(ctx->pool, bytes);
+    if (e != hipSuccess) return drr_hip_error(e, "jobs: device tables");
+    std::vector<char> host(bytes);
+    auto put = [&](size_t off, const void *p, size_t n) {
+        if (n) std::memcpy(host.data() + off, p, n);
+    };
+    put(off_seg, h.seg, sizeof(int) * 9);
+    put(off_vols, h.vols.data(), sizeof(VolDev) * h.vols.size());
+    put(off_jobs, h.jobs.data(), sizeof(JobDev) * h.jobs.size());
+    put(off_mjobs, h.mjobs.data(), sizeof(JobMultiDev) * h.mjobs.size());
+    if (extra) put(off_extra, extra, extra_bytes);
+    put(off_items, h.items.data(), sizeof(int2) * h.items.size());
+    put(off_items + sizeof(int2) * h.items.size(), h.mitems.data(), sizeof(int2) * h.mitems.size());
+    e = hipMemcpy(t.buf.as<char>(), host.data(), bytes, hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        drr_jobs_free(t);
+        return drr_hip_error(e, "jobs: device tables");
     }
-#undef JCHK
+    t.d_counters = t.buf.as<int>();
+    t.d_seg = t.buf.as<int>(off_seg);
+    t.d_vols = t.buf.as<VolDev>(off_vols);
+    t.d_jobs = t.buf.as<JobDev>(off_jobs);
+    t.d_mjobs = t.buf.as<JobMultiDev>(off_mjobs);
+    t.d_extra = t.buf.as<void>(off_extra);
+    t.d_items = t.buf.as<int2>(off_items);
+    t.d_mitems = t.d_items + h.items.size();
     return DRR_OK;
 }
 
@@ -211,9 +210,7 @@ struct drr_batch_s {
     int march = MARCH_V1_EXACT;  // the context's at creation
     drr_batch_tuning_t tune{};
     JobTable t;
-    ImgSeg *d_imgs = nullptr;
-    unsigned int *d_keys = nullptr;
-    hipStream_t cap = nullptr;
+    PoolBuf imgs_keys;  // the images, then their neglog keys
     hipGraph_t graph_march = nullptr, graph_epi = nullptr;
     hipGraphExec_t exec_march = nullptr, exec_epi = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr;  // before march, after march, after epilogue
@@ -350,12 +347,10 @@ static void batch_free(drr_batch *B) {
     if (B->exec_epi) (void)hipGraphExecDestroy(B->exec_epi);
     if (B->graph_march) (void)hipGraphDestroy(B->graph_march);
     if (B->graph_epi) (void)hipGraphDestroy(B->graph_epi);
-    if (B->cap) (void)hipStreamDestroy(B->cap);
     for (hipEvent_t e : {B->ev0, B->ev1, B->ev2})
         if (e) (void)hipEventDestroy(e);
     drr_jobs_free(B->t);
-    (void)hipFree(B->d_imgs);
-    (void)hipFree(B->d_keys);
+    B->imgs_keys.reset();
     delete B;
 }
 
@@ -364,18 +359,23 @@ static void batch_free(drr_batch *B) {
 // march.  Captured work allocates nothing and records no memset nodes.
 static hipError_t capture(drr_batch *B, SpectrumDev sp, float step, int air, float *I, float *P,
                           float *images, int neglog) {
-    hipError_t e = hipStreamBeginCapture(B->cap, hipStreamCaptureModeThreadLocal);
+    std::lock_guard<std::mutex> lk(B->ctx->cap_mu);
+    hipError_t e = hipSuccess;
+    if (!B->ctx->cap) e = hipStreamCreateWithFlags(&B->ctx->cap, hipStreamNonBlocking);
     if (e != hipSuccess) return e;
-    k_jobs_reset<<<1, 64, 0, B->cap>>>(B->t.d_counters);
-    launch_all(B->t, B->M, B->atten, B->march, B->tune.tile_w, B->cap, sp, step, air, I, P, nullptr);
-    e = hipStreamEndCapture(B->cap, &B->graph_march);
+    e = hipStreamBeginCapture(B->ctx->cap, hipStreamCaptureModeThreadLocal);
+    if (e != hipSuccess) return e;
+    k_jobs_reset<<<1, 64, 0, B->ctx->cap>>>(B->t.d_counters);
+    launch_all(B->t, B->M, B->atten, B->march, B->tune.tile_w, B->ctx->cap, sp, step, air, I, P, nullptr);
+    e = hipStreamEndCapture(B->ctx->cap, &B->graph_march);
     if (e != hipSuccess) return e;
     e = hipGraphInstantiate(&B->exec_march, B->graph_march, nullptr, nullptr, 0);
     if (e != hipSuccess || !neglog) return e;
-    e = hipStreamBeginCapture(B->cap, hipStreamCaptureModeThreadLocal);
+    e = hipStreamBeginCapture(B->ctx->cap, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return e;
-    int rc = drr_enqueue_neglog(I, images, B->d_imgs, B->t.n_jobs, B->t.max_npix, B->d_keys, 0.01f, B->cap);
-    hipError_t e2 = hipStreamEndCapture(B->cap, &B->graph_epi);
+    int rc = drr_enqueue_neglog(I, images, B->imgs_keys.as<ImgSeg>(), B->t.n_jobs,
+                                B->t.max_npix, B->imgs_keys.as<unsigned int>(sizeof(ImgSeg) * B->t.n_jobs), 0.01f, B->ctx->cap);
+    hipError_t e2 = hipStreamEndCapture(B->ctx->cap, &B->graph_epi);
     if (rc != DRR_OK) return hipErrorLaunchFailure;
     if (e2 != hipSuccess) return e2;
     return hipGraphInstantiate(&B->exec_epi, B->graph_epi, nullptr, nullptr, 0);
@@ -425,10 +425,10 @@ extern "C" int drr_batch_create(drr_ctx *ctx, const drr_volume *const *vols, int
             return drr_hip_error(e, #x);                               \
         }                                                              \
     } while (0)
-    BCHK(hipMalloc(&B->d_imgs, sizeof(ImgSeg) * n_jobs));
-    BCHK(hipMalloc(&B->d_keys, sizeof(unsigned int) * 4 * n_jobs));
-    BCHK(hipMemcpy(B->d_imgs, B->t.imgs.data(), sizeof(ImgSeg) * n_jobs, hipMemcpyHostToDevice));
-    BCHK(hipStreamCreateWithFlags(&B->cap, hipStreamNonBlocking));
+    if (neglog) {
+        BCHK(B->imgs_keys.take(ctx->pool, (sizeof(ImgSeg) + 4 * sizeof(unsigned int)) * n_jobs));
+        BCHK(hipMemcpy(B->imgs_keys.as<ImgSeg>(), B->t.imgs.data(), sizeof(ImgSeg) * n_jobs, hipMemcpyHostToDevice));
+    }
     BCHK(hipEventCreate(&B->ev0));
     BCHK(hipEventCreate(&B->ev1));
     BCHK(hipEventCreate(&B->ev2));
@@ -463,7 +463,8 @@ extern "C" int drr_batch_last_march_ms(drr_batch *B, float *ms) {
 extern "C" int drr_batch_destroy(drr_batch *B) {
     if (!B) return DRR_OK;
     DevSwitch ds(B->ctx->device);
-    if (B->launched) (void)hipEventSynchronize(B->ev2);
+    // its tables go back to the pool: no launch, on whatever stream, may still read them
+    if (B->launched) (void)hipDeviceSynchronize();
     batch_free(B);
     return DRR_OK;
 }
@@ -537,8 +538,6 @@ int scratch_address(int device, unsigned char **out) {
     *out = g_scratch_ptr[device];
     return DRR_OK;
 }
-
-constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 }  // namespace
 
 extern "C" int drr_project_jobs_noalloc(drr_ctx *ctx, const drr_volume *const *vols, int n_vols,

@@ -17,15 +17,129 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <memory>
+#include <mutex>
 #include <string>
+#include <utility>
+#include <vector>
 
 #include "../../include/deepdrr_amd.h"
+
+// Small device buffers (job tables, keys, flags) of a context's calls, kept from
+// call to call: hipMalloc and hipFree cost about 20 us each and hipFree waits for
+// the whole device, where a call over a few small views takes a millisecond.  A
+// buffer is put back only after the GPU work that uses it has ended, so any
+// thread or stream may take it next.  At most 32 buffers and 64 MB of up to 16 MB
+// each are kept, and one of up to 2 GB: a volume's cells, which a fit makes anew
+// for every density (freeing 87 MB takes 0.3 ms).  They are freed with the
+// context, or when memory runs out; those that outlive it by their owner.
+class DevPool {
+  public:
+    ~DevPool() {
+        for (auto &b : free_) (void)hipFree(b.second);
+    }
+    // Contents undefined; `size` is what has to be given back with the buffer.
+    hipError_t take(size_t bytes, void **p, size_t *size) {
+        const size_t unit = bytes > ((size_t)1 << 20) ? (size_t)1 << 20 : 4096;
+        const size_t n = (bytes + unit - 1) / unit * unit;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            size_t best = free_.size();  // the smallest that fits and is not over twice as large
+            for (size_t i = 0; i < free_.size(); i++)
+                if (free_[i].first >= n && free_[i].first <= 2 * n &&
+                    (best == free_.size() || free_[i].first < free_[best].first))
+                    best = i;
+            if (best < free_.size()) {
+                *size = free_[best].first;
+                *p = free_[best].second;
+                if (*size <= BIG) held_ -= *size;
+                free_[best] = free_.back();
+                free_.pop_back();
+                return hipSuccess;
+            }
+        }
+        *size = n;
+        hipError_t e = hipMalloc(p, n);
+        if (e == hipErrorOutOfMemory && drop()) {
+            (void)hipGetLastError();
+            e = hipMalloc(p, n);
+        }
+        return e;
+    }
+    void put(void *p, size_t size) {
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            bool keep;
+            if (size > BIG) {
+                keep = size <= ((size_t)2 << 30);
+                for (auto &b : free_) keep &= b.first <= BIG;
+            } else {
+                keep = free_.size() < 32 && held_ + size <= ((size_t)64 << 20);
+            }
+            if (keep) {
+                free_.emplace_back(size, p);
+                if (size <= BIG) held_ += size;
+                return;
+            }
+        }
+        (void)hipFree(p);
+    }
+
+  private:
+    static constexpr size_t BIG = (size_t)16 << 20;
+    bool drop() {  // free what is kept
+        std::vector<std::pair<size_t, void *>> all;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            all.swap(free_);
+            held_ = 0;
+        }
+        for (auto &b : all) (void)hipFree(b.second);
+        return !all.empty();
+    }
+    std::mutex mu_;
+    std::vector<std::pair<size_t, void *>> free_;
+    size_t held_ = 0;
+};
+
+// A buffer of a pool, given back when its owner drops it.
+class PoolBuf {
+  public:
+    PoolBuf() = default;
+    PoolBuf(const PoolBuf &) = delete;
+    PoolBuf &operator=(const PoolBuf &) = delete;
+    ~PoolBuf() { reset(); }
+    hipError_t take(const std::shared_ptr<DevPool> &pool, size_t bytes) {
+        reset();
+        const hipError_t e = pool->take(bytes, &p_, &size_);
+        if (e == hipSuccess)
+            pool_ = pool;
+        else
+            p_ = nullptr;
+        return e;
+    }
+    void reset() {
+        if (p_) pool_->put(p_, size_);
+        p_ = nullptr;
+        pool_.reset();
+    }
+    template <typename T>
+    T *as(size_t byte_offset = 0) const {
+        return reinterpret_cast<T *>(static_cast<char *>(p_) + byte_offset);
+    }
+
+  private:
+    std::shared_ptr<DevPool> pool_;
+    void *p_ = nullptr;
+    size_t size_ = 0;
+};
 
 struct drr_volume_s {
     drr_ctx *ctx = nullptr;
     int device = 0;  // HIP device of the allocation (outlives the context)
     int nx = 0, ny = 0, nz = 0;
     int64_t n_cells = 0;
+    PoolBuf cell_buf;
     uint32_t *cells = nullptr;  // DRR_CELL_WORDS 32-bit words per cell
     // voxel-order records [nz][ny][nx] of (density bits, label), made on first
     // use by the Monte-Carlo path: a nearest-voxel lookup is one 8-byte load
@@ -37,6 +151,11 @@ struct drr_volume_s {
 struct drr_ctx_s {
     int device = 0;
     int n_cus = 0;  // compute units
+    std::shared_ptr<DevPool> pool = std::make_shared<DevPool>();
+    // The stream that plans are captured on (nothing runs on it), one for all:
+    // making a stream takes up to a millisecond.
+    std::mutex cap_mu;
+    hipStream_t cap = nullptr;
     drr_scene_t scene{0.1f, 0, 0, 0, DRR_MARCH_EXACT};
     bool have_scene = false;
     bool single_sums = false;  // the fast march adds every sample singly (drr_ctx_set_single_sums)
@@ -213,5 +332,6 @@ int drr_check_view_finite(const drr_view_t *view);
 int drr_volume_ensure_linear(drr_volume *vol);
 
 // Launchers implemented in forward.hip (used by batch/adjoint code).
-int drr_launch_expand(const float *density, const uint8_t *labels, int nx, int ny, int nz,
+// bad (may be NULL) becomes nonzero if a label is not below n_labels.
+int drr_launch_expand(const float *density, const uint8_t *labels, int n_labels, uint32_t *bad, int nx, int ny, int nz,
                       uint32_t *cells, hipStream_t st);

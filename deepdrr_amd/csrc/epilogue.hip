@@ -118,19 +118,17 @@ extern "C" int drr_neglog(drr_ctx *ctx, const float *in, float *out, int n_image
     if (n_images < 1 || npix < 1 || n_images > 65535)
         return drr_set_error(DRR_ERR_INVALID, "drr_neglog: need 1..65535 images of >= 1 pixel");
     hipStream_t st = (hipStream_t)stream;
-    ImgSeg *segs = nullptr;
-    unsigned int *keys = nullptr;
+    PoolBuf buf;  // the images, then their keys
     std::vector<ImgSeg> h(n_images);
     for (int i = 0; i < n_images; i++) h[i] = ImgSeg{(int64_t)i * npix, npix};
     int rc = DRR_OK;
-    hipError_t e = hipMalloc(&segs, sizeof(ImgSeg) * n_images);
-    if (e == hipSuccess) e = hipMalloc(&keys, sizeof(unsigned int) * 4 * n_images);
+    hipError_t e = buf.take(ctx->pool, (sizeof(ImgSeg) + 4 * sizeof(unsigned int)) * n_images);
+    ImgSeg *segs = buf.as<ImgSeg>();
+    unsigned int *keys = buf.as<unsigned int>(sizeof(ImgSeg) * n_images);
     if (e == hipSuccess) e = hipMemcpyAsync(segs, h.data(), sizeof(ImgSeg) * n_images, hipMemcpyHostToDevice, st);
     if (e != hipSuccess) rc = drr_hip_error(e, "drr_neglog setup");
     if (rc == DRR_OK) rc = drr_enqueue_neglog(in, out, segs, n_images, npix, keys, epsilon, st);
     e = hipStreamSynchronize(st);
     if (rc == DRR_OK && e != hipSuccess) rc = drr_hip_error(e, "drr_neglog");
-    (void)hipFree(segs);
-    (void)hipFree(keys);
     return rc;
 }

@@ -18,8 +18,9 @@ using namespace drr;
 // stores.  Consecutive threads write consecutive records, so the stores are
 // fully coalesced.
 __global__ __launch_bounds__(256) void k_expand(const float *__restrict__ density,
-                                                const uint8_t *__restrict__ labels, int nx, int ny,
-                                                int nz, uint32_t *__restrict__ cells) {
+                                                const uint8_t *__restrict__ labels, uint32_t n_labels,
+                                                uint32_t *__restrict__ bad, int nx, int ny, int nz,
+                                                uint32_t *__restrict__ cells) {
     const int64_t ncx = nx + 1, ncy = ny + 1, ncz = nz + 1;
     const int64_t ncell = ncx * ncy * ncz;
     for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < ncell;
@@ -40,11 +41,14 @@ __global__ __launch_bounds__(256) void k_expand(const float *__restrict__ densit
         }
         uint32_t packed = 0;
         bool same = true;
+        uint32_t top = 0;
 #pragma unroll
         for (int q = 0; q < 8; q++) {
+            top = max(top, l[q]);
             packed |= l[q] << (4 * q);
             same = same && (l[q] == l[0]);
         }
+        if (top >= n_labels && bad) atomicOr(bad, 1u);
         uint2 *rec = reinterpret_cast<uint2 *>(cells + DRR_CELL_WORDS * c);  // 8-byte aligned
 #pragma unroll
         for (int q = 0; q < 4; q++) rec[q] = make_uint2(__float_as_uint(d[2 * q]), __float_as_uint(d[2 * q + 1]));
@@ -52,12 +56,15 @@ __global__ __launch_bounds__(256) void k_expand(const float *__restrict__ densit
     }
 }
 
-int drr_launch_expand(const float *density, const uint8_t *labels, int nx, int ny, int nz,
+__global__ void k_zero(uint32_t *p) { *p = 0; }
+
+int drr_launch_expand(const float *density, const uint8_t *labels, int n_labels, uint32_t *bad, int nx, int ny, int nz,
                       uint32_t *cells, hipStream_t st) {
     const int64_t ncell = (int64_t)(nx + 1) * (ny + 1) * (nz + 1);
     int64_t blocks = (ncell + 255) / 256;
     if (blocks > 65536) blocks = 65536;
-    k_expand<<<(unsigned)blocks, 256, 0, st>>>(density, labels, nx, ny, nz, cells);
+    if (bad) k_zero<<<1, 1, 0, st>>>(bad);
+    k_expand<<<(unsigned)blocks, 256, 0, st>>>(density, labels, (uint32_t)n_labels, bad, nx, ny, nz, cells);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return drr_hip_error(e, "k_expand launch");
     return DRR_OK;

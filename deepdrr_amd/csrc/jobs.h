@@ -34,6 +34,8 @@ struct JobMultiDev {
 };
 
 struct JobTable {
+    PoolBuf buf;  // every table below, and the caller's extra bytes
+    void *d_extra = nullptr;
     int n_jobs = 0, n_vols = 0;
     JobDev *d_jobs = nullptr;   // single-volume jobs (entries of multi-volume jobs unused)
     VolDev *d_vols = nullptr;
@@ -56,8 +58,10 @@ struct JobTable {
 // 16x16 workgroup tiles) and single-volume jobs only.
 int drr_jobs_build(drr_ctx *ctx, const drr_volume *const *vols, int n_vols, const drr_job_t *jobs,
                    int n_jobs, const drr_batch_tuning_t &tune, JobTable &t);
+// extra (may be NULL): extra_bytes of the caller's, copied along to d_extra.
 int drr_jobs_build_tiles(drr_ctx *ctx, const drr_volume *const *vols, int n_vols, const drr_job_t *jobs,
-                         int n_jobs, const drr_batch_tuning_t &tune, JobTable &t);
+                         int n_jobs, const drr_batch_tuning_t &tune, JobTable &t, const void *extra,
+                         size_t extra_bytes);
 void drr_jobs_free(JobTable &t);
 
 __global__ void k_jobs_reset(int *counters);

@@ -138,8 +138,9 @@ extern "C" int drr_add_noise(drr_ctx *ctx, const float *intensity, const float *
     (void)hipGetDevice(&prev);
     if (prev != ctx->device) DRR_HIP_CHECK(hipSetDevice(ctx->device));
     const int64_t total = (int64_t)n_images * height * width;
-    float *shot = nullptr;
-    DRR_HIP_CHECK(hipMalloc(&shot, sizeof(float) * total));
+    PoolBuf buf;
+    DRR_HIP_CHECK(buf.take(ctx->pool, sizeof(float) * total));
+    float *shot = buf.as<float>();
     hipStream_t st = (hipStream_t)stream;
     int64_t blocks = (total + 255) / 256;
     if (blocks > 16384) blocks = 16384;
@@ -148,7 +149,6 @@ extern "C" int drr_add_noise(drr_ctx *ctx, const float *intensity, const float *
     k_correlate<<<(unsigned)blocks, 256, 0, st>>>(intensity, shot, out, n_images, height, width);
     hipError_t e = hipGetLastError();
     hipError_t e2 = hipStreamSynchronize(st);
-    (void)hipFree(shot);
     if (prev >= 0 && prev != ctx->device) (void)hipSetDevice(prev);
     if (e != hipSuccess) return drr_hip_error(e, "drr_add_noise launch");
     if (e2 != hipSuccess) return drr_hip_error(e2, "drr_add_noise");

@@ -102,6 +102,7 @@ int drr_ctx_destroy(drr_ctx *ctx) {
     (void)hipFree(ctx->d_mu);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
+    if (ctx->cap) (void)hipStreamDestroy(ctx->cap);
     delete ctx;
     return DRR_OK;
 }
@@ -166,14 +167,6 @@ int drr_ctx_last_kernel_ms(drr_ctx *ctx, float *ms) {
 
 // ---- volumes --------------------------------------------------------------
 
-__global__ void k_label_max(const uint8_t *labels, int64_t n, unsigned int *out) {
-    unsigned int m = 0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        m = max(m, (unsigned int)labels[i]);
-    atomicMax(out, m);
-}
-
 __global__ void k_hu_ingest(const int16_t *hu, int64_t n, int n_classes, const float *upper,
                             const uint8_t *label_of_class, float *density, uint8_t *labels) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
@@ -203,9 +196,9 @@ static int volume_alloc(drr_ctx *ctx, int nx, int ny, int nz, drr_volume **out) 
     v->ny = ny;
     v->nz = nz;
     v->n_cells = (int64_t)(nx + 1) * (ny + 1) * (nz + 1);
-    hipError_t e = hipMalloc(&v->cells, sizeof(uint32_t) * DRR_CELL_WORDS * v->n_cells);
+    hipError_t e = v->cell_buf.take(ctx->pool, sizeof(uint32_t) * DRR_CELL_WORDS * v->n_cells);
+    v->cells = v->cell_buf.as<uint32_t>();
     if (e != hipSuccess) {
-        (void)hipFree(v->cells);
         delete v;
         return drr_set_error(DRR_ERR_ALLOC, std::string("drr_volume: device allocation failed: ") +
                                                 hipGetErrorString(e));
@@ -238,7 +231,8 @@ int drr_volume_create(drr_ctx *ctx, const float *density, const uint8_t *labels,
     const int M = ctx->scene.n_materials;
     const float *d_den = density;
     const uint8_t *d_lab = labels;
-    DevBuf tmp_den, tmp_lab, d_max;
+    DevBuf tmp_den, tmp_lab;
+    PoolBuf bad;
     if (!on_device) {
         for (int64_t i = 0; i < n; i++)
             if (labels[i] >= M)
@@ -254,21 +248,20 @@ int drr_volume_create(drr_ctx *ctx, const float *density, const uint8_t *labels,
         // device inputs may come from any stream of the caller: wait for all
         // queued work before reading them
         DRR_HIP_CHECK(hipDeviceSynchronize());
-        DRR_HIP_CHECK(d_max.alloc(sizeof(unsigned int)));
-        DRR_HIP_CHECK(hipMemset(d_max.p, 0, sizeof(unsigned int)));
-        k_label_max<<<1024, 256, 0, 0>>>(labels, n, d_max.as<unsigned int>());
-        DRR_HIP_CHECK(hipGetLastError());
-        unsigned int mx = 0;
-        DRR_HIP_CHECK(hipMemcpy(&mx, d_max.p, sizeof(unsigned int), hipMemcpyDeviceToHost));
-        if ((int)mx >= M)
-            return drr_set_error(DRR_ERR_INVALID, "drr_volume_create: label >= n_materials");
+        DRR_HIP_CHECK(bad.take(ctx->pool, sizeof(uint32_t)));
     }
     drr_volume *v = nullptr;
     rc = volume_alloc(ctx, nx, ny, nz, &v);
-    if (rc == DRR_OK) rc = drr_launch_expand(d_den, d_lab, nx, ny, nz, v->cells, 0);
+    // (labels on the host are checked above; on the device by the expansion)
+    uint32_t *d_bad = on_device ? bad.as<uint32_t>() : nullptr, h_bad = 0;
+    if (rc == DRR_OK) rc = drr_launch_expand(d_den, d_lab, M, d_bad, nx, ny, nz, v->cells, 0);
     if (rc == DRR_OK) {
-        hipError_t e = hipDeviceSynchronize();
-        if (e != hipSuccess) rc = drr_hip_error(e, "drr_volume_create: expand");
+        // either waits for the expansion
+        hipError_t e = on_device ? hipMemcpy(&h_bad, d_bad, sizeof(h_bad), hipMemcpyDeviceToHost) : hipDeviceSynchronize();
+        if (e != hipSuccess)
+            rc = drr_hip_error(e, "drr_volume_create: expand");
+        else if (h_bad)
+            rc = drr_set_error(DRR_ERR_INVALID, "drr_volume_create: label >= n_materials");
     }
     if (rc != DRR_OK) {
         if (v) drr_volume_destroy(v);
@@ -315,7 +308,7 @@ int drr_volume_create_from_hu(drr_ctx *ctx, const int16_t *hu, int nx, int ny, i
     DRR_HIP_CHECK(hipGetLastError());
     drr_volume *v = nullptr;
     rc = volume_alloc(ctx, nx, ny, nz, &v);
-    if (rc == DRR_OK) rc = drr_launch_expand(d_den.as<float>(), d_lab.as<uint8_t>(), nx, ny, nz, v->cells, 0);
+    if (rc == DRR_OK) rc = drr_launch_expand(d_den.as<float>(), d_lab.as<uint8_t>(), DRR_MAX_MATERIALS, nullptr, nx, ny, nz, v->cells, 0);
     if (rc == DRR_OK) {
         hipError_t e = hipDeviceSynchronize();
         if (e != hipSuccess) rc = drr_hip_error(e, "drr_volume_create_from_hu");
@@ -331,7 +324,8 @@ int drr_volume_create_from_hu(drr_ctx *ctx, const int16_t *hu, int nx, int ny, i
 int drr_volume_destroy(drr_volume *vol) {
     if (!vol) return DRR_OK;
     DeviceGuard g(vol->device);
-    (void)hipFree(vol->cells);
+    // the cells go back to the pool: no launch may still read them
+    (void)hipDeviceSynchronize();
     (void)hipFree(vol->lin_vox);
     delete vol;
     return DRR_OK;

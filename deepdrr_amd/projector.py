@@ -48,12 +48,14 @@ def to_host(t) -> np.ndarray:
 
 def volume_view_params(vol: Volume, proj: geo.CameraProjection, priority: int) -> dict:
     """Per-volume uniforms of one view (projector.py:802-831, 1626-1637)."""
-    ijk_from_world = np.asarray(vol.IJK_from_world.toarray())
-    source_ijk = np.array(vol.IJK_from_world @ proj.center_in_world).astype(np.float32)
+    return _volume_params(vol, vol.IJK_from_world, proj.center_in_world, priority)
+
+
+def _volume_params(vol: Volume, ijk_from_world: geo.FrameTransform, center: geo.Point3D, priority: int) -> dict:
     shape = vol.shape
     return dict(
-        ijk_from_world=ijk_from_world[:3, :].astype(np.float32).reshape(12),
-        source_ijk=source_ijk,
+        ijk_from_world=np.asarray(ijk_from_world.toarray())[:3, :].astype(np.float32).reshape(12),
+        source_ijk=np.array(ijk_from_world @ center).astype(np.float32),
         bounds_lo=np.full(3, -0.5, np.float32),
         bounds_hi=np.array([shape[0] - 0.5, shape[1] - 0.5, shape[2] - 0.5], np.float32),
         priority=int(priority),
@@ -68,11 +70,44 @@ def world_from_index_rows(proj: geo.CameraProjection, sdd: float) -> np.ndarray:
     return w.astype(np.float32)
 
 
+def cameras(projections: Sequence[geo.CameraProjection], sdd: float):
+    """``world_from_index_rows`` and the camera centre in world [3] of each
+    projection, with one call for all the inverses (they take most of a view's
+    preparation: 64 views 1.5 ms one by one, 0.5 ms so)."""
+    k_inv = np.linalg.inv(np.stack([p.intrinsic.data for p in projections]))
+    known = [p.extrinsic._inv for p in projections]
+    open_ = [i for i, m in enumerate(known) if m is None]
+    if open_:
+        for i, m in zip(open_, np.linalg.inv(np.stack([projections[i].extrinsic.data for i in open_]))):
+            known[i] = m
+    rows, centers = [], []
+    for m, k in zip(known, k_inv):
+        w = m[:3, :3] @ k
+        if geo.RAY_SCALE == "source_to_pixel":
+            w = w * sdd
+        rows.append(w.astype(np.float32))
+        centers.append(m[:3, 3].copy())
+    return rows, centers
+
+
+def build_views(volumes: Sequence[Volume], priorities: Sequence[int], projections: Sequence[geo.CameraProjection],
+                max_ray_length: float, sdd: float = 1.0, allow_empty: bool = False, which=None):
+    """One view per projection, over all the volumes or (``which``) over one each."""
+    if not projections:
+        return []
+    ijk = [v.IJK_from_world for v in volumes]
+    views = []
+    for i, (proj, rows, center) in enumerate(zip(projections, *cameras(projections, sdd))):
+        w, h = proj.intrinsic.sensor_size
+        chosen = range(len(volumes)) if which is None else (which[i],)
+        vols = [_volume_params(volumes[k], ijk[k], geo.point(center), priorities[k]) for k in chosen]
+        views.append(make_view(rows, w, h, max_ray_length, vols, allow_empty=allow_empty))
+    return views
+
+
 def build_view(volumes: Sequence[Volume], priorities: Sequence[int], proj: geo.CameraProjection,
                max_ray_length: float, sdd: float = 1.0, allow_empty: bool = False):
-    w, h = proj.intrinsic.sensor_size
-    vols = [volume_view_params(v, proj, p) for v, p in zip(volumes, priorities)]
-    return make_view(world_from_index_rows(proj, sdd), w, h, max_ray_length, vols, allow_empty=allow_empty)
+    return build_views(volumes, priorities, [proj], max_ray_length, sdd, allow_empty)[0]
 
 
 def volume_arrays(vol: Volume, all_materials: List[str]):
