@@ -14,9 +14,8 @@
 // handed over when it leaves, and accumulates the pose gradient from
 //   dL/dp_t = wt_t [ (sum_d w_d h_d) grad(rho) + rho grad(sum_d h_d w_d) ]
 // (the second term vanishes in a cell whose labels agree).  Nothing is stored
-// per sample; in a cell whose labels agree, pass 2 forms the corner sums over
-// the cell's samples at once, in closed form (AdjRay::cell_sums, equal to the
-// per-sample sums up to rounding).  drr_adjoint scatters with
+// per sample; pass 2 forms the sums over a cell's samples at once, in closed
+// form (AdjRay::cell_sums, equal to the per-sample sums up to rounding).  drr_adjoint scatters with
 // global float atomics; drr_adjoint_jobs runs many views in one persistent
 // launch whose workgroups gather the scatter of their 16x16-ray tile in LDS,
 // slab by slab along the beam, and add it to the gradient volume once per
@@ -27,22 +26,11 @@
 #include <vector>
 
 #include "drr_internal.h"
+#include "fast_march.h"
 #include "jobs.h"
 #include "march.h"
 
 using namespace drr;
-
-// d/d(fx, fy, fz) of sum_d v_d w_d for corner values v (corner d = dx + 2dy + 4dz).
-__device__ __forceinline__ void grad_trilinear(const float v[8], float fx, float fy, float fz,
-                                               float out[3]) {
-    const float gx = 1.0f - fx, gy = 1.0f - fy, gz = 1.0f - fz;
-    out[0] = (v[1] - v[0]) * (gy * gz) + (v[3] - v[2]) * (fy * gz) + (v[5] - v[4]) * (gy * fz) +
-             (v[7] - v[6]) * (fy * fz);
-    out[1] = (v[2] - v[0]) * (gx * gz) + (v[3] - v[1]) * (fx * gz) + (v[6] - v[4]) * (gx * fz) +
-             (v[7] - v[5]) * (fx * fz);
-    out[2] = (v[4] - v[0]) * (gx * gy) + (v[5] - v[1]) * (fx * gy) + (v[6] - v[2]) * (gx * fy) +
-             (v[7] - v[3]) * (fx * fy);
-}
 
 // ---- where the per-cell corner sums go ----------------------------------------
 
@@ -95,14 +83,16 @@ struct NullDep {
 };
 
 // Into a workgroup's LDS box [o, o + L) (voxels, per axis); corners outside it
-// go to the gradient volume directly, so the box only changes the speed.
+// go to the gradient volume directly, so the box only changes the speed.  The
+// box is FP64 because ds_add_f64 is the fast one: a wave's add to 64 different
+// words takes 4 to 7 ns of a CU, ds_add_f32 80 (64 views of 256^2, density
+// alone: 20.5 ms with an FP32 box, its adds busy 89 % of the cycles; 12.2).
 struct BoxDep {
     static constexpr bool kDensity = true;
-    float *box;
+    double *box;
     int ox, oy, oz, Lx, Ly, Lz;
     float *gD;
     // some of the 8 corners: those with a zero sum are skipped lane by lane
-    // (an LDS atomic costs per active lane)
     __device__ __forceinline__ void part(const VolDev &vol, float bx, float by, float bz, const float (&v)[8]) {
         float a[8];
 #pragma unroll
@@ -126,7 +116,7 @@ struct BoxDep {
                                 (iz[1] * Ly + iy[1]) * Lx};
 #pragma unroll
             for (int d = 0; d < 8; d++)
-                if (!SKIP_ZERO || acc[d] != 0.0f) atomicAdd(box + (row[d >> 1] + ix[d & 1]), acc[d]);
+                if (!SKIP_ZERO || acc[d] != 0.0f) atomicAdd(box + (row[d >> 1] + ix[d & 1]), (double)acc[d]);
         } else {
             const uint32_t nx = vol.nx, ny = vol.ny;
 #pragma unroll
@@ -136,7 +126,7 @@ struct BoxDep {
                 const bool in = ((uint32_t)ix[a] < (uint32_t)Lx) & ((uint32_t)iy[b] < (uint32_t)Ly) &
                                 ((uint32_t)iz[c] < (uint32_t)Lz);
                 if (in) {
-                    atomicAdd(box + ((iz[c] * Ly + iy[b]) * Lx + ix[a]), acc[d]);
+                    atomicAdd(box + ((iz[c] * Ly + iy[b]) * Lx + ix[a]), (double)acc[d]);
                 } else {
                     const uint32_t x = a ? k.x1 : k.x0, y = b ? k.y1 : k.y0, z = c ? k.z1 : k.z0;
                     unsafeAtomicAdd(gD + ((z * ny + y) * nx + x), acc[d]);
@@ -176,28 +166,24 @@ template <int M, bool POSE>
 struct AdjRay {
     RayV1 r;
     Cell c;
+    Cell next;  // that of the sample at alpha
     float alpha;
     int t;
     bool live;
     float graw[M];
-    float acc[8];   // sum over the cell's samples of G w_d: density gradient of corner d
-    float acc1[8];  // sum of (alpha - aref) G w_d (pose only)
+    // sum over samples of G w_d, the density gradient of corner d: the open cell's
+    // and those carried into it through the face it was entered by
+    float acc[8];
     float aref;     // the ray's volume entry: alpha-weighted sums are taken about it
-    // (pose kernel) density sums carried into the open cell through the face
-    // it was entered by, held apart from acc so the pose term sees the cell's
-    // own sums
-    float carry[8];
     float hu;       // dL/d(ad_raw) of the material of a cell whose labels agree
     // Pose sums S0 = sum_t dL/dp_t, S1 = sum_t (alpha_t - aref) dL/dp_t, in FP64
     // (thousands of terms of both signs), in registers.  Within a cell, dL/dp_t =
     // G_t grad(rho)(p_t) [+ wt rho_t grad(h)(p_t) if the labels differ, h_d =
-    // dL/d(ad_raw) of corner d's material], and grad(rho) along x is
-    // sum_yz (D[1yz] - D[0yz]) w_yz, so sum_t G_t grad_x(rho) =
-    // sum_yz (D[1yz] - D[0yz]) (acc[0yz] + acc[1yz]) (w_0yz + w_1yz = w_yz):
-    // the G term needs no per-sample gradient.  All of this is linear in the
-    // sums, so a cell may be flushed in parts.  (They were per-thread LDS
-    // slots while the pose kernel ran at 4 waves per SIMD; at 3 the registers
-    // are there, and the FP64 adds leave the LDS to the box atomics.)
+    // dL/d(ad_raw) of corner d's material].  In a one-label cell grad(rho) along
+    // an axis is bilinear in the other two, a quadratic along the ray, which
+    // cell_sums adds in closed form; elsewhere, along x, it is sum_yz (D[1yz] -
+    // D[0yz]) w_yz, so sum_t G_t grad_x(rho) = sum_yz (D[1yz] - D[0yz]) (a[0yz] +
+    // a[1yz]) with a = sum_t G_t w (w_0yz + w_1yz = w_yz).
     double S[6];
 
     __device__ __forceinline__ void add_S(int k, double v) { S[k] += v; }
@@ -221,8 +207,6 @@ struct AdjRay {
 #pragma unroll
         for (int d = 0; d < 8; d++) {
             acc[d] = 0.0f;
-            acc1[d] = 0.0f;
-            carry[d] = 0.0f;
         }
         hu = 0.0f;
         if (POSE)
@@ -249,43 +233,31 @@ struct AdjRay {
             ++t;
         }
         if (c.have) set_h();
+        next.load(vol, floorf(sample_pos(sx, alpha, rix)), floorf(sample_pos(sy, alpha, riy)),
+                  floorf(sample_pos(sz, alpha, riz)));
     }
 
-    __device__ __forceinline__ void flush_pose() {
-        const float D[8] = {c.d0.x, c.d0.y, c.d0.z, c.d0.w, c.d1.x, c.d1.y, c.d1.z, c.d1.w};
-        float g0[3] = {0.f, 0.f, 0.f}, g1[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            const int b = 1 << k;
-#pragma unroll
-            for (int d = 0; d < 8; d++) {
-                if (d & b) continue;
-                const float dD = D[d | b] - D[d];
-                g0[k] = fmaf(dD, acc[d] + acc[d | b], g0[k]);
-                g1[k] = fmaf(dD, acc1[d] + acc1[d | b], g1[k]);
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            add_S(k, (double)g0[k]);
-            add_S(k + 3, (double)g1[k]);
-        }
-#pragma unroll
-        for (int d = 0; d < 8; d++) acc1[d] = 0.0f;
+    // Adds to S[k] and, weighted with alpha - aref, S[k + 3] the sums over a run of
+    // samples (cell_sums) of G times the bilinear interpolant of q00, q10 (first
+    // axis up), q01, q11, a quadratic in v; (y, ry), (z, rz): fractions at the run's
+    // middle and rates along the ray, A[j] = sum G v^j.
+    __device__ __forceinline__ static void bilinear(float amid, const float (&A)[4], float q00, float q10, float q01,
+                                                    float q11, float y, float ry, float z, float rz, float &s0,
+                                                    float &s1) {
+        const float y0 = q10 - q00, y1 = q11 - q01;
+        const float e0 = fmaf(y, y0, q00), e1 = fmaf(y, y1, q01), f0 = ry * y0, f1 = ry * y1;
+        const float ez = e1 - e0, fz = f1 - f0;
+        const float p0 = fmaf(z, ez, e0), p1 = fmaf(rz, ez, fmaf(z, fz, f0)), p2 = rz * fz;
+        const float a0 = fmaf(p2, A[2], fmaf(p1, A[1], p0 * A[0]));
+        const float a1 = fmaf(p2, A[3], fmaf(p1, A[2], p0 * A[1]));
+        s0 += a0;
+        s1 += fmaf(amid, a0, a1);
     }
 
     // Hand the open cell's sums to `dep` (the cell stays cached).
     template <class Dep>
     __device__ __forceinline__ void flush(const VolDev &vol, Dep &dep) {
         if (!c.have) return;
-        if (POSE) {
-            flush_pose();
-#pragma unroll
-            for (int d = 0; d < 8; d++) {
-                acc[d] += carry[d];
-                carry[d] = 0.0f;
-            }
-        }
         dep(vol, c.bx, c.by, c.bz, acc);
     }
 
@@ -294,20 +266,13 @@ struct AdjRay {
     // on that face are corners of the next cell too: their sums stay in
     // registers (moved to the next cell's corner slots) and only the 4 corners
     // left behind are handed to `dep`, lane by lane, so a face crossing costs
-    // half the LDS atomic lanes of a full flush.  The density-only kernel
-    // carries them in acc itself; the pose kernel, whose pose term needs the
-    // cell's own sums, flushes its pose term first and carries them in carry.
+    // half the LDS atomic lanes of a full flush.
     template <class Dep>
     __device__ __forceinline__ void leave_through_face(const VolDev &vol, Dep &dep, int k, int s) {
         const int f = s < 0 ? 1 : 0;  // bit along k of the corners left behind
         // (masks and products instead of selects between array elements, which
         // the compiler would turn into indexed loads from scratch memory)
         const float m0 = k == 0 ? 1.0f : 0.0f, m1 = k == 1 ? 1.0f : 0.0f, m2 = k == 2 ? 1.0f : 0.0f;
-        if (POSE) {
-            flush_pose();
-#pragma unroll
-            for (int d = 0; d < 8; d++) acc[d] += carry[d];
-        }
         float leave[8], nacc[8];
 #pragma unroll
         for (int d = 0; d < 8; d++) {
@@ -319,76 +284,100 @@ struct AdjRay {
         }
         dep.part(vol, c.bx, c.by, c.bz, leave);
 #pragma unroll
-        for (int d = 0; d < 8; d++) {
+        for (int d = 0; d < 8; d++) acc[d] = nacc[d];
+    }
+
+    // Sums of a cell's n samples of weight wt (1, or n = 1) in closed form.  The samples sit at
+    // u_k = k h (k < n) from the entry sample, whose fractions against the cell
+    // are f.  About the run's midpoint u_m = h (n - 1) / 2, with v = u - u_m,
+    // corner d = (a, b, c)'s weight is X_a(v) Y_b(v) Z_c(v), X_1 = x_1 + r_x v
+    // with x_1 = f_x + r_x u_m and X_0 = 1 - X_1 (so x_0' = -r_x, x_1' = r_x),
+    // and likewise along y and z.  The odd central sums of v vanish; the even
+    // ones are C2 = h^2 n (n^2 - 1) / 12, C4 = h^4 n (n^2 - 1) (3 n^2 - 7) / 240 and
+    // C6 = h^6 n (n^2 - 1) (3 n^4 - 18 n^2 + 31) / 1344.
+    //   In a one-label cell G is hu (the material's dL/d(ad_raw), times the weights'
+    // sum, 1 to rounding); elsewhere it is
+    // the trilinear interpolant of the corners' h, a cubic g_0..g_3 in v.  With
+    //   A_0 = n g_0 + C2 g_2, A_1 = C2 g_1 + C4 g_3, A_2 = C2 g_0 + C4 g_2, A_3 = C4 g_1 + C6 g_3
+    // (A_j = sum G v^j) the sum of G times a polynomial w_0..w_3 is sum w_j A_j:
+    // Y_b Z_c = (yz, y'z + yz', y'z') and the weight of corner (1, b, c) is that
+    // times x_1 + r_x v; (0, b, c)'s sum is the difference.  The pose adds G
+    // grad(rho) and, where the labels differ, rho grad(h) (bilinear).
+    template <bool DENSITY>
+    __device__ __forceinline__ void cell_sums(int n, float wt, float h, float am, float fx, float fy, float fz, float rx,
+                                              float ry, float rz) {
+        const float n2 = (float)n * (float)n, nf = wt * (float)n;
+        const float um = 0.5f * h * ((float)n - 1.0f);
+        const float x1 = fmaf(rx, um, fx), y1 = fmaf(ry, um, fy), z1 = fmaf(rz, um, fz);
+        const float h2 = h * h;
+        const float C2 = h2 * nf * (n2 - 1.0f) * (1.0f / 12.0f);
+        const float amid = (am - aref) + um;
+        const float D[8] = {c.d0.x, c.d0.y, c.d0.z, c.d0.w, c.d1.x, c.d1.y, c.d1.z, c.d1.w};
+        float A[4] = {nf * hu, 0.0f, C2 * hu, 0.0f};
+        float s0[3] = {0.f, 0.f, 0.f}, s1[3] = {0.f, 0.f, 0.f};
+        if (!c.uni) {
+            const float C4 = C2 * h2 * fmaf(3.0f, n2, -7.0f) * (1.0f / 20.0f);
+            const float C6 = C2 * h2 * h2 * fmaf(fmaf(3.0f, n2, -18.0f), n2, 31.0f) * (1.0f / 112.0f);
+            float hc[8];
+            corner_h(hc);
+            const Cubic g = cell_cubic(hc[0], hc[1] - hc[0], hc[2], hc[3] - hc[2], hc[4], hc[5] - hc[4], hc[6],
+                                       hc[7] - hc[6], x1, y1, z1, rx, ry, rz);
+            A[0] = fmaf(C2, g.c2, nf * g.c0);
+            A[1] = fmaf(C4, g.c3, C2 * g.c1);
+            A[2] = fmaf(C4, g.c2, C2 * g.c0);
+            A[3] = fmaf(C6, g.c3, C4 * g.c1);
             if (POSE) {
-                carry[d] = nacc[d];
-                acc[d] = 0.0f;
-            } else {
-                acc[d] = nacc[d];
+                const Cubic r = cell_cubic(D[0], D[1] - D[0], D[2], D[3] - D[2], D[4], D[5] - D[4], D[6], D[7] - D[6],
+                                           x1, y1, z1, rx, ry, rz);
+                const float R[4] = {fmaf(C2, r.c2, nf * r.c0), fmaf(C4, r.c3, C2 * r.c1), fmaf(C4, r.c2, C2 * r.c0),
+                                    fmaf(C6, r.c3, C4 * r.c1)};
+                pose_gradients(amid, R, hc, x1, rx, y1, ry, z1, rz, s0, s1);
+            }
+        }
+        if (DENSITY) {
+            const float Y[2] = {1.0f - y1, y1}, Z[2] = {1.0f - z1, z1};
+            const float Yd[2] = {-ry, ry}, Zd[2] = {-rz, rz};
+#pragma unroll
+            for (int bc = 0; bc < 4; bc++) {
+                const int b = bc & 1, c3 = bc >> 1;
+                const float yz = Y[b] * Z[c3], t1 = fmaf(Yd[b], Z[c3], Y[b] * Zd[c3]), qq = Yd[b] * Zd[c3];
+                const float Wyz = fmaf(qq, A[2], fmaf(t1, A[1], yz * A[0]));
+                const float W1 = fmaf(rx * qq, A[3], fmaf(fmaf(rx, t1, x1 * qq), A[2],
+                                                          fmaf(fmaf(rx, yz, x1 * t1), A[1], x1 * yz * A[0])));
+                acc[2 * bc] += Wyz - W1;
+                acc[2 * bc + 1] += W1;
+            }
+        }
+        if (POSE) {
+            pose_gradients(amid, A, D, x1, rx, y1, ry, z1, rz, s0, s1);
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                add_S(k, (double)s0[k]);
+                add_S(k + 3, (double)s1[k]);
             }
         }
     }
 
-    // Sums of a one-label cell's n samples of weight 1 in closed form.  The
-    // samples sit at u_k = k h (k < n) from the entry sample, whose fractions
-    // against the cell are f.  About the run's midpoint u_m = h (n - 1) / 2,
-    // with v = u - u_m, corner d = (a, b, c)'s weight is X_a(v) Y_b(v) Z_c(v),
-    // X_1 = x_1 + r_x v with x_1 = f_x + r_x u_m and X_0 = 1 - X_1 (so
-    // x_0' = -r_x, x_1' = r_x), and likewise along y and z.  The odd central
-    // sums of v vanish, so with C2 = sum v^2 = h^2 n (n^2 - 1) / 12 and
-    // C4 = sum v^4 = h^4 n (n^2 - 1) (3 n^2 - 7) / 240:
-    //   sum_k w_d = n xyz + C2 (x'y'z + x'yz' + xy'z'),
-    //   sum_k alpha_k w_d = alpha_m sum_k w_d + C2 (x'yz + xy'z + xyz') + C4 x'y'z',
-    // with alpha_m the midpoint's alpha (taken about aref, as acc1 is).  Both are added times hu (the
-    // material's dL/d(ad_raw)), as the per-sample loop adds G w_d with G = hu
-    // times the weights' sum, which is 1 to rounding.
-    __device__ __forceinline__ void cell_sums(int n, float h, float am, float fx, float fy, float fz, float rx,
-                                              float ry, float rz) {
-        const float nf = (float)n;
-        const float um = 0.5f * h * (nf - 1.0f);
-        const float x1 = fmaf(rx, um, fx), y1 = fmaf(ry, um, fy), z1 = fmaf(rz, um, fz);
-        const float X[2] = {1.0f - x1, x1}, Y[2] = {1.0f - y1, y1}, Z[2] = {1.0f - z1, z1};
-        const float Xd[2] = {-rx, rx}, Yd[2] = {-ry, ry}, Zd[2] = {-rz, rz};
-        const float h2 = h * h, q = fmaf(nf, nf, -1.0f);
-        const float C2 = h2 * nf * q * (1.0f / 12.0f);
-        const float C4 = h2 * h2 * nf * q * fmaf(3.0f * nf, nf, -7.0f) * (1.0f / 240.0f);
-        const float amid = (am - aref) + um;
-        // per (b, c) pair: yz, y'z + yz', y'z'; then each corner (a, b, c)
-#pragma unroll
-        for (int bc = 0; bc < 4; bc++) {
-            const int b = bc & 1, c3 = bc >> 1;
-            const float yz = Y[b] * Z[c3], s1 = fmaf(Yd[b], Z[c3], Y[b] * Zd[c3]), qq = Yd[b] * Zd[c3];
-#pragma unroll
-            for (int a = 0; a < 2; a++) {
-                const int d = a + 2 * bc;
-                const float t2 = fmaf(Xd[a], s1, X[a] * qq);  // x'(y'z + yz') + x y'z'
-                const float W = fmaf(C2, t2, nf * (X[a] * yz));
-                acc[d] = fmaf(hu, W, acc[d]);
-                if (POSE) {
-                    const float t3 = fmaf(X[a], s1, Xd[a] * yz);  // x'yz + x(y'z + yz')
-                    const float A = fmaf(amid, W, fmaf(C2, t3, C4 * (Xd[a] * qq)));
-                    acc1[d] = fmaf(hu, A, acc1[d]);
-                }
-            }
-        }
+    // sum of A's factor times the gradient of the trilinear interpolant of V
+    __device__ __forceinline__ static void pose_gradients(float amid, const float (&A)[4], const float (&V)[8], float x,
+                                                          float rx, float y, float ry, float z, float rz,
+                                                          float (&s0)[3], float (&s1)[3]) {
+        bilinear(amid, A, V[1] - V[0], V[3] - V[2], V[5] - V[4], V[7] - V[6], y, ry, z, rz, s0[0], s1[0]);
+        bilinear(amid, A, V[2] - V[0], V[3] - V[1], V[6] - V[4], V[7] - V[5], x, rx, z, rz, s0[1], s1[1]);
+        bilinear(amid, A, V[4] - V[0], V[5] - V[1], V[6] - V[2], V[7] - V[3], x, rx, y, ry, s0[2], s1[2]);
     }
 
     // March on while the floor of the sample position along `axis` of each
     // newly entered cell satisfies go(floor).  The open cell's sums are handed
     // over when the ray leaves it or ends.
     //
-    // Cell by cell: every lane still marching hands over its open cell and
-    // loads the cell of its current sample together (one execution of that
-    // long block for the whole wave), then the wave runs the samples of those
-    // cells until every lane's next sample lies outside its own.  Lanes whose
-    // cells end early idle for the rest of that inner loop, which costs less
-    // than running the hand-over once for each group of lanes that leave
-    // together.  Membership is the exact march's: fractions p - b in [0, 1).
-    // Loop tests are wave votes and per-lane choices in the inner loop are
-    // 0/1 factors (an idle lane's fractions are taken as 0, so its terms are
-    // exact zeros): per-lane branches and loop exits cost scalar instructions.
-    // Each lane's samples, sums and hand-overs are those of a plain per-sample
-    // march.
+    // Cell by cell: every lane still marching hands over its open cell, takes the
+    // cell of its current sample and sums that cell's samples together (one
+    // execution of that long block for the whole wave).  The next cell's record
+    // is loaded before the present one is summed.  VALU issue bounds it (0.94 of
+    // the cycles; one label 250 instructions, several 400 more).  64 views of 256^2
+    // through 192^3: 28.6 ms with the samples of several labels one by one (91
+    // instructions each), 22.5 in closed form, 16.9 with the box in FP64.
     template <class Dep, class Go>
     __device__ __forceinline__ void run(const Geo1 &g, const VolDev &vol, float step, int axis, Dep &dep, Go go) {
         const int N = r.N;
@@ -404,6 +393,7 @@ struct AdjRay {
         const float hy = riy == 0.0f ? INFINITY : (riy < 0.0f ? 0.0f : jy);
         const float hz = riz == 0.0f ? INFINITY : (riz < 0.0f ? 0.0f : jz);
         bool act = live;
+        bool single = false;  // the open cell's samples are taken one by one
         while (__ballot(act) != 0) {
             // the lane's current sample and its cell
             const float px = sample_pos(sx, alpha, rix), py = sample_pos(sy, alpha, riy),
@@ -426,85 +416,57 @@ struct AdjRay {
                 } else {
                     flush(vol, dep);
                 }
-                c.load(vol, bx, by, bz);
+                c = next;
+                c.bx = bx;
+                c.by = by;
+                c.bz = bz;
                 set_h();
+                single = false;
             }
-            // (ex, ey, ez): the fractions of the lane's next sample against the
-            // open cell
-            float ex = px - c.bx, ey = py - c.by, ez = pz - c.bz;
-            // A one-label cell whose samples all have weight 1 and over which
+            // The cell's samples from this one on that all have weight 1 and over which
             // the FP32 alpha sequence is linear (its first two increments agree,
-            // so no tie alternates, and it stays in one binade) takes its samples
-            // at once (cell_sums).  The sample count comes from the exit distance,
-            // so a sample within rounding of a face may fall to either cell (the
-            // weights on the shared face agree); the last sample is kept for
-            // the loop below when the ray ends in the cell.
-            bool cf = false;
-            if (act && c.uni && t >= 1) {
+            // so no tie alternates, and it stays in one binade).  Their number
+            // comes from the exit distance, so a sample within rounding of a face
+            // may fall to either cell (the weights on the shared face agree).
+            // Where that is not so, the cell's samples are taken singly.
+            if (act) {
+                const float ex = px - c.bx, ey = py - c.by, ez = pz - c.bz;
                 const float a1 = alpha + step, s1 = a1 - alpha, s2 = (a1 + step) - a1;
                 // the samples before the exit face at the actual increment s1 (a
                 // far source moves alpha by up to a quarter step more, or not at all)
                 const float nex = fminf(fmaf(-ex, jx, hx), fminf(fmaf(-ey, jy, hy), fmaf(-ez, jz, hz))) *
                                   (s1 > 0.0f ? step / s1 : INFINITY);
-                const int n = min(max((int)ceilf(nex), 1), N - 1 - t);
-                const float an = fmaf((float)n, s1, alpha);  // alpha after the n samples
-                if (n >= 1 && s1 == s2 && (__float_as_uint(an) ^ __float_as_uint(alpha)) < 0x00800000u &&
-                    an - s1 <= r.mxv) {
-                    cell_sums(n, s1, alpha, ex, ey, ez, rix, riy, riz);
-                    alpha = an;
-                    t += n;
-                    cf = true;
+                int n = min(max((int)ceilf(nex), 1), N - 1 - t);
+                float an = fmaf((float)n, s1, alpha);  // alpha after the n samples
+                single = single || !(t >= 1 && n >= 1 && s1 == s2 &&
+                                     (__float_as_uint(an) ^ __float_as_uint(alpha)) < 0x00800000u && an - s1 <= r.mxv);
+                if (single) {
+                    n = 1;
+                    an = a1;
                 }
-            }
-            // the other lanes' samples of the cell, one by one
-            bool in = act & !cf;
-            if (__ballot(in) == 0) continue;
-            do {
-                const float gm = in ? 1.0f : 0.0f;
-                const float fx = in ? ex : 0.0f, fy = in ? ey : 0.0f, fz = in ? ez : 0.0f;
-                float w[8];
-                weights8(fx, fy, fz, w);
+                // Where the labels differ the pose sums jump at the faces (rho grad(h)),
+                // and samples on a face come in numbers (a voxel of so many steps):
+                // those that are in the cell, by their FP32 positions.
+                if (POSE && !c.uni && n > 1) {
+                    auto inside = [&](float al) {
+                        const float qx = sample_pos(sx, al, rix) - c.bx, qy = sample_pos(sy, al, riy) - c.by,
+                                    qz = sample_pos(sz, al, riz) - c.bz;
+                        return max(max(__float_as_uint(qx), __float_as_uint(qy)), __float_as_uint(qz)) < 0x3f800000u;
+                    };
+                    // (several off where a ray runs along a face)
+                    for (; n > 1 && !inside(an - s1); --n) an -= s1;
+                    for (; n < N - 1 - t && an <= r.mxv && inside(an) &&
+                           (__float_as_uint(an + s1) ^ __float_as_uint(alpha)) < 0x00800000u; ++n)
+                        an += s1;
+                }
                 // t == 0 or t == N-1 (t < N), as one unsigned comparison
                 const float wt = ((uint32_t)(t - 1) >= (uint32_t)(N - 2)) ? 0.5f : 1.0f;
-                float sw;
-                if (c.uni) {
-                    const float ssum = ((((((w[0] + w[1]) + w[2]) + w[3]) + w[4]) + w[5]) + w[6]) + w[7];
-                    sw = hu * ssum;
-                } else {
-                    float h[8];
-                    corner_h(h);
-                    sw = 0.0f;
-#pragma unroll
-                    for (int d = 0; d < 8; d++) sw = fmaf(w[d], h[d], sw);
-                    if (POSE && in) {
-                        // label-gradient term of a cell whose labels differ (rare)
-                        const float rho = trilerp(c.d0, c.d1, w);
-                        float gh[3];
-                        grad_trilinear(h, fx, fy, fz, gh);
-                        const float wr = wt * rho;
-#pragma unroll
-                        for (int k = 0; k < 3; k++) {
-                            add_S(k, (double)(wr * gh[k]));
-                            add_S(k + 3, (double)((alpha - aref) * wr * gh[k]));
-                        }
-                    }
-                }
-                const float G = gm * (wt * sw);
-#pragma unroll
-                for (int d = 0; d < 8; d++) acc[d] = fmaf(G, w[d], acc[d]);
-                if (POSE) {
-                    const float aG = (alpha - aref) * G;
-#pragma unroll
-                    for (int d = 0; d < 8; d++) acc1[d] = fmaf(aG, w[d], acc1[d]);
-                }
-                alpha = fmaf(gm, step, alpha);
-                t += in ? 1 : 0;
-                ex = sample_pos(sx, alpha, rix) - c.bx;
-                ey = sample_pos(sy, alpha, riy) - c.by;
-                ez = sample_pos(sz, alpha, riz) - c.bz;
-                in = in & (max(max(__float_as_uint(ex), __float_as_uint(ey)), __float_as_uint(ez)) < 0x3f800000u) &
-                     (t < N) & (alpha <= r.mxv);
-            } while (__ballot(in) != 0);
+                next.load(vol, floorf(sample_pos(sx, an, rix)), floorf(sample_pos(sy, an, riy)),
+                          floorf(sample_pos(sz, an, riz)));
+                cell_sums<Dep::kDensity>(n, wt, s1, alpha, ex, ey, ez, rix, riy, riz);
+                alpha = an;
+                t += n;
+            }
         }
         if (live && !(t < N && alpha <= r.mxv)) {
             flush(vol, dep);
@@ -638,13 +600,14 @@ __global__ void k_pose_finish(const double *acc, float *gPose) {
 // along the axis its central ray advances fastest on, and all rays march one
 // slab at a time.  Corner sums go into an LDS box covering the slab
 // (ADJ_SLAB + 1 voxel planes along that axis, ADJ_BOX voxels across, centred
-// on the central ray) with LDS atomics; after each slab the box is added to
+// on the central ray; slabs of 11: 11.9 ms for the density alone, 7: 12.4, 15:
+// 14.2, where only 3 boxes fit a CU) with LDS atomics; after each slab the box is added to
 // the gradient volume once per touched voxel.  Corners outside the box (a
 // beam wider than the box, a ray against the slab order) go to the gradient
 // volume directly, so results do not depend on the geometry, only the
 // number of global atomics does.
 constexpr int ADJ_TILE = 16;
-constexpr int ADJ_SLAB = 15;
+constexpr int ADJ_SLAB = 11;
 constexpr int ADJ_BOX = 20;
 constexpr int ADJ_BOX_CELLS = (ADJ_SLAB + 1) * ADJ_BOX * ADJ_BOX;
 
@@ -655,23 +618,24 @@ __device__ __forceinline__ void ray_through(const float *W, float fu, float fv, 
     r[2] = fu * W[6] + fv * W[7] + W[8];
 }
 
-// Occupancy targets that fit without (or, for more materials, with a few)
-// register spills: 5 waves per SIMD for the density gradient alone, 3 with
-// the pose sums (density, pose moments and the carried face: 4 waves spill in
-// the cell loop and ran 4 % slower).
+// Occupancy targets: waves per SIMD, also the blocks per CU that the launch keeps
+// resident.  64 views of 256^2 through 192^3: density alone 12.2 ms at 4 (122
+// registers; 5 spill 14), with the pose 16.9 ms at 3 (4 spill 39).  The
+// pose alone: 6.9 ms at 3, 7.7 at 4.
 template <int POSE>
 struct AdjOcc {
-    static constexpr int waves = POSE ? 3 : 5;
+    static constexpr int waves = POSE ? 3 : 4;
 };
+constexpr int ADJ_POSE_WAVES = 3;
 
 template <int M, bool ATTEN, bool POSE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AdjOcc<POSE>::waves))) void k_adjoint_jobs(const JobDev *__restrict__ jobs, const int2 *__restrict__ items,
                                                       const int *__restrict__ seg, int *counters,
                                                       const float *__restrict__ sw_jobs, VolDev vol, SpectrumDev sp,
                                                       float step, int air, AdjArgs a, double *pose64) {
-    __shared__ float box[ADJ_BOX_CELLS];
+    __shared__ double box[ADJ_BOX_CELLS];
     __shared__ double s_pose[4][6];
-    for (int i = threadIdx.x; i < ADJ_BOX_CELLS; i += blockDim.x) box[i] = 0.0f;
+    for (int i = threadIdx.x; i < ADJ_BOX_CELLS; i += blockDim.x) box[i] = 0.0;
     __syncthreads();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for_each_block_item(jobs, items, seg, counters, [&](int j, const JobDev &J, int tile) __attribute__((always_inline)) {
@@ -746,16 +710,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AdjOcc<POSE
             const float inv_x = 1.0f / (float)len[0], inv_y = 1.0f / (float)len[1];
             const uint32_t nx = vol.nx, ny = vol.ny;
             for (int i = threadIdx.x; i < ADJ_BOX_CELLS; i += blockDim.x) {
-                const float v = box[i];
-                if (v != 0.0f) {
+                const double v = box[i];
+                if (v != 0.0) {
                     const int iyz = (int)(((float)i + 0.5f) * inv_x);
                     const int ix = i - iyz * len[0];
                     const int iz = (int)(((float)iyz + 0.5f) * inv_y);
                     const int iy = iyz - iz * len[1];
                     const int x = org[0] + ix, y = org[1] + iy, z = org[2] + iz;
                     if (x >= 0 && x < vol.nx && y >= 0 && y < vol.ny && z >= 0 && z < vol.nz)
-                        unsafeAtomicAdd(a.gD + (((uint32_t)z * ny + (uint32_t)y) * nx + (uint32_t)x), v);
-                    box[i] = 0.0f;
+                        unsafeAtomicAdd(a.gD + (((uint32_t)z * ny + (uint32_t)y) * nx + (uint32_t)x), (float)v);
+                    box[i] = 0.0;
                 }
             }
             __syncthreads();
@@ -788,7 +752,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AdjOcc<POSE
 // pose sums as k_adjoint_jobs<..., true>, without any density scatter, so no
 // slabs or LDS box.
 template <int M, bool ATTEN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_adjoint_pose_jobs(const JobDev *__restrict__ jobs,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ADJ_POSE_WAVES))) void k_adjoint_pose_jobs(const JobDev *__restrict__ jobs,
                                                            const int2 *__restrict__ items,
                                                            const int *__restrict__ seg, int *counters,
                                                            const float *__restrict__ sw_jobs, VolDev vol,
@@ -954,7 +918,7 @@ extern "C" int drr_adjoint_jobs(drr_ctx *ctx, const drr_volume *vol, const drr_j
     // 16x16-pixel workgroup tiles, 4 waves per workgroup; as many persistent
     // workgroups per CU as the kernel's occupancy target holds (LDS allows it)
     const bool pose = grad_pose != nullptr;
-    const int blocks_per_cu = pose ? AdjOcc<1>::waves : AdjOcc<0>::waves;  // pose only: 4, as with density
+    const int blocks_per_cu = !grad_density ? ADJ_POSE_WAVES : pose ? AdjOcc<1>::waves : AdjOcc<0>::waves;
     const drr_batch_tuning_t tune{ADJ_TILE, ADJ_TILE, 4, blocks_per_cu};
     // beside the tables: FP64 pose accumulator [6], then the job sources [3 * n_jobs]
     std::vector<char> extra(sizeof(double) * 6 + sizeof(float) * 3 * n_jobs, 0);
