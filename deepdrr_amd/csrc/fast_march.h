@@ -31,8 +31,12 @@
 // * A cell with three or more labels takes the exact filter's formulas.
 //
 // Every lane enters its next cell together with the others (one execution of
-// the entry block for the wave); lanes that add one by one do so in loops of
-// their own afterwards.  The materials' sums live in LDS, one word per lane and
+// the entry block for the wave), and each kind of cell runs its block and its
+// loop over the samples for its own lanes.  (With the loops after all blocks, wave
+// votes as their tests and 0/1 factors as the lanes' choices, for the scalar
+// instructions that lanes' own branches take, a sample cost 7 vector
+// instructions in place of 5, one of two labels 39 in place of 30 for every lane
+// of the wave: 16 clinical views 85.5 ms, 73.3 now; 48 mixed 17.6, 16.5.)  The materials' sums live in LDS, one word per lane and
 // material: an entry reads and writes the words its labels name, which in
 // registers takes a compare and a select per material and holds the
 // materials' registers and lane masks through the loop.  The record of the
@@ -51,12 +55,12 @@ namespace drr {
 
 // Running sum (density x step, mm g/cm^3) up to which cells are summed at once:
 // images of clinical views are then within 7.8e-6 of the exact march's (6.4e-6
-// with every sample added singly, 1.2e-5 at 128, 1.6e-5 at 204.8), at 17.5 ms
-// for 48 mixed views against 24.2 singly.
+// with every sample added singly, 1.2e-5 at 128, 1.6e-5 at 204.8), at 16.5 ms
+// for 48 mixed views (when singly took 24.2, this took 17.5).
 constexpr float FAST_CLOSED_SUM = 102.4f;
-// Waves per SIMD of the kernels that march fast: 96 registers hold the entry
-// block and the record on its way (6 waves spill 16: 7.4 ms against 5.7 on the
-// clinical view; 4 waves: 5.7).
+// Waves per SIMD of the kernels that march fast: 87 registers hold the entry
+// block and the record on its way (with 9 more, 6 waves spilled 16: 7.4 ms
+// against 5.7 on the clinical view; 4 waves: 5.7).
 constexpr int FAST_WAVES = 5;
 
 // A trilinear interpolant along the ray p(u) = p_m + u r as a cubic in u:
@@ -105,12 +109,6 @@ __device__ __forceinline__ float mean_rounding(float cur, float lo, float hi) {
     // (el - eh is d where the ends round to the same value)
     return fabsf(d) > 9.5367432e-7f * fabsf(hi) ? s * ((el - eh) * __builtin_amdgcn_rcpf(d)) : s;
 }
-
-// Two-label cells: the corners' indicators of the second label as lerps along x
-// (first corners vYZ, differences xYZ), 0 or 1 and 0 or +-1.
-struct Second {
-    float v00, v10, v01, v11, x00, x10, x01, x11;
-};
 
 // One sample of weight wt by the exact filter's formulas, added to the sums.
 template <int M>
@@ -176,133 +174,101 @@ __device__ __forceinline__ void fast_run(const VolDev &vol, float *acc, float sx
         // sum of u^2 over the samples
         const float S2 = inc2_12 * (nf * __builtin_fmaf(nf, nf, -1.0f));
         const uint32_t l0 = c.l0, la = l0 & 0xfu;
-        float *pa = acc + LDS_LANES * la, *pb = acc;  // sums of the first and second label
-        float cur = *pa, sq = 0.0f;
-        Cubic fc = cell_cubic(c.d0.x, c.d0.y - c.d0.x, c.d0.z, c.d0.w - c.d0.z, c.d1.x, c.d1.y - c.d1.x, c.d1.z,
-                              c.d1.w - c.d1.z, mx, my, mz, rix, riy, riz);
-        const float h = 0.5f * inc * nf, h2 = h * h;  // the samples' extent is [-h, h]
-        bool one = true;  // the samples are to be added one by one
-        bool tw = false, ex = false;  // two labels; three or more
-        Second e;
+        float *pa = acc + LDS_LANES * la;
         if (c.uni) {
+            float cur = *pa;
+            const Cubic fc = cell_cubic(c.d0.x, c.d0.y - c.d0.x, c.d0.z, c.d0.w - c.d0.z, c.d1.x, c.d1.y - c.d1.x,
+                                        c.d1.z, c.d1.w - c.d1.z, mx, my, mz, rix, riy, riz);
+            const float h = 0.5f * inc * nf, h2 = h * h;  // the samples' extent is [-h, h]
             const float ev = __builtin_fmaf(fc.c2, h2, fc.c0), od = h * __builtin_fmaf(fc.c3, h2, fc.c1);
             const bool flat = (fc.c1 == 0.0f) & (fc.c2 == 0.0f);
-            one = !(flat | (cur < acut));
-            if (!one) *pa = cur + __builtin_fmaf(fc.c2, S2, nf * (fc.c0 + mean_rounding(cur, ev - od, ev + od)));
-        } else {
-            const uint32_t xa = l0 ^ (la * 0x11111111u);  // nonzero nibbles: corners not la
-            const uint32_t lb = (l0 >> (__builtin_ctz(xa) & ~3u)) & 0xfu;
-            const uint32_t xb = l0 ^ (lb * 0x11111111u);
-            const uint32_t na = nz_nibbles(xa), nb = nz_nibbles(xb);  // nb bit set: corner not lb
-            tw = (na & nb) == 0u;
-            ex = !tw;
-            pb = acc + LDS_LANES * lb;
-            sq = *pb;
-            e.v00 = (nb & 0x8u) ? 0.f : 1.f;
-            e.v10 = (nb & 0x800u) ? 0.f : 1.f;
-            e.v01 = (nb & 0x80000u) ? 0.f : 1.f;
-            e.v11 = (nb & 0x8000000u) ? 0.f : 1.f;
-            e.x00 = ((nb & 0x80u) ? 0.f : 1.f) - e.v00;
-            e.x10 = ((nb & 0x8000u) ? 0.f : 1.f) - e.v10;
-            e.x01 = ((nb & 0x800000u) ? 0.f : 1.f) - e.v01;
-            e.x11 = ((nb & 0x80000000u) ? 0.f : 1.f) - e.v11;
-            if (tw & (fmaxf(cur, sq) < acut)) {
-                // The middle's fractions as the mean of the samples' FP32
-                // positions: the exact filter's positions round with the same
-                // sign over many samples, which along a boundary adds up (with
-                // the entry's alone, oblique clinical views came to 2e-5 of the
-                // exact march's, with three samples' to 1.2e-5).
-                float qx = 0.0f, qy = 0.0f, qz = 0.0f, al = alpha0;
-                for (int k = 0;; k += 2) {
-                    const bool in = k < n;
-                    if (__ballot(in) == 0) break;
-                    const float g = in ? 1.0f : 0.0f, g1 = k + 1 < n ? 1.0f : 0.0f, al1 = al + inc;
-                    qx = __builtin_fmaf(g, __builtin_fmaf(al, rix, sx) - (bx + 1.0f), qx);
-                    qy = __builtin_fmaf(g, __builtin_fmaf(al, riy, sy) - (by + 1.0f), qy);
-                    qz = __builtin_fmaf(g, __builtin_fmaf(al, riz, sz) - (bz + 1.0f), qz);
-                    qx = __builtin_fmaf(g1, __builtin_fmaf(al1, rix, sx) - (bx + 1.0f), qx);
-                    qy = __builtin_fmaf(g1, __builtin_fmaf(al1, riy, sy) - (by + 1.0f), qy);
-                    qz = __builtin_fmaf(g1, __builtin_fmaf(al1, riz, sz) - (bz + 1.0f), qz);
-                    al = al1 + inc;
+            if (flat | (cur < acut)) {
+                cur += __builtin_fmaf(fc.c2, S2, nf * (fc.c0 + mean_rounding(cur, ev - od, ev + od)));
+            } else {
+                float u = -um;
+                for (int k = 0; k < n; ++k) {
+                    cur += __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(fc.c3, u, fc.c2), u, fc.c1), u, fc.c0);
+                    u += inc;
                 }
-                const float rn = __builtin_amdgcn_rcpf(nf);
-                qx *= rn;
-                qy *= rn;
-                qz *= rn;
-                const Cubic g = cell_cubic(e.v00, e.x00, e.v10, e.x10, e.v01, e.x01, e.v11, e.x11, qx, qy, qz, rix,
-                                           riy, riz);
-                fc = cell_cubic(c.d0.x, c.d0.y - c.d0.x, c.d0.z, c.d0.w - c.d0.z, c.d1.x, c.d1.y - c.d1.x, c.d1.z,
-                                c.d1.w - c.d1.z, qx, qy, qz, rix, riy, riz);
-                const float S4 = S2 * (inc2_12 * 0.6f) * __builtin_fmaf(3.0f * nf, nf, -7.0f);
-                const float S6 = S2 * (inc2_12 * inc2_12 * (9.0f / 7.0f)) *
-                                 __builtin_fmaf(nf * nf, __builtin_fmaf(3.0f * nf, nf, -18.0f), 31.0f);
-                const float p2 = __builtin_fmaf(fc.c0, g.c2, __builtin_fmaf(fc.c1, g.c1, fc.c2 * g.c0));
-                const float p4 = __builtin_fmaf(fc.c1, g.c3, __builtin_fmaf(fc.c2, g.c2, fc.c3 * g.c1));
-                const float sum_q = __builtin_fmaf(
-                    nf, fc.c0 * g.c0, __builtin_fmaf(S2, p2, __builtin_fmaf(S4, p4, S6 * (fc.c3 * g.c3))));
-                *pb = sq + sum_q;
-                *pa = cur + (__builtin_fmaf(fc.c2, S2, nf * fc.c0) - sum_q);
-                one = false;
             }
+            *pa = cur;
+            continue;
         }
-        if (__ballot(one) == 0) continue;
-        if (!one) n = 0;
-        tw = tw & one;
-        if (ex) fc = Cubic{0.0f, 0.0f, 0.0f, 0.0f};
-        // the samples that are added one by one.  The loops' tests are wave votes
-        // and their per-lane choices 0/1 factors: per-lane branches cost scalar
-        // instructions, enough to become the limit in loops this short.
-        if (__ballot(tw) != 0) {
-            // two labels: density and second fraction at the sample's FP32
-            // position, each by nested lerps; the other lanes' cubics beside them
-            float al = alpha0, u = -um;
-            for (int k = 0;; ++k) {
-                const bool in = k < n;
-                if (__ballot(in) == 0) break;
-                const float g = in ? 1.0f : 0.0f;
-                float rho = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(fc.c3, u, fc.c2), u, fc.c1), u, fc.c0);
-                const float fx = __builtin_fmaf(al, rix, sx) - (c.bx + 1.0f);
-                const float fy = __builtin_fmaf(al, riy, sy) - (c.by + 1.0f);
-                const float fz = __builtin_fmaf(al, riz, sz) - (c.bz + 1.0f);
-                const float a00 = __builtin_fmaf(fx, c.d0.y - c.d0.x, c.d0.x);
-                const float a10 = __builtin_fmaf(fx, c.d0.w - c.d0.z, c.d0.z);
-                const float a01 = __builtin_fmaf(fx, c.d1.y - c.d1.x, c.d1.x);
-                const float a11 = __builtin_fmaf(fx, c.d1.w - c.d1.z, c.d1.z);
-                const float b0 = __builtin_fmaf(fy, a10 - a00, a00), b1 = __builtin_fmaf(fy, a11 - a01, a01);
-                const float x = __builtin_fmaf(fz, b1 - b0, b0);
-                const float i00 = __builtin_fmaf(fx, e.x00, e.v00), i10 = __builtin_fmaf(fx, e.x10, e.v10);
-                const float i01 = __builtin_fmaf(fx, e.x01, e.v01), i11 = __builtin_fmaf(fx, e.x11, e.v11);
-                const float j0 = __builtin_fmaf(fy, i10 - i00, i00), j1 = __builtin_fmaf(fy, i11 - i01, i01);
-                const float fq = __builtin_fmaf(fz, j1 - j0, j0);
-                const float xq = x * fq;
-                sq = __builtin_fmaf(g, tw ? xq : 0.0f, sq);
-                rho = tw ? x - xq : rho;
-                cur = __builtin_fmaf(g, rho, cur);
-                al = __builtin_fmaf(g, step, al);
-                u += inc;
+        const uint32_t xa = l0 ^ (la * 0x11111111u);  // nonzero nibbles: corners not la
+        const uint32_t lb = (l0 >> (__builtin_ctz(xa) & ~3u)) & 0xfu;
+        const uint32_t xb = l0 ^ (lb * 0x11111111u);
+        const uint32_t na = nz_nibbles(xa), nb = nz_nibbles(xb);  // nb bit set: corner not lb
+        float al = alpha0;
+        if ((na & nb) != 0u) {  // three or more labels
+            for (int k = 0; k < n; ++k) {
+                fast_sample<M>(c, acc, __builtin_fmaf(al, rix, sx) - (bx + 1.0f),
+                               __builtin_fmaf(al, riy, sy) - (by + 1.0f), __builtin_fmaf(al, riz, sz) - (bz + 1.0f),
+                               1.0f);
+                al += step;
             }
-            if (tw) *pb = sq;
+            continue;
+        }
+        float *pb = acc + LDS_LANES * lb;
+        float cur = *pa, sq = *pb;
+        // the second label's indicators of the corners as lerps along x: 0 or 1,
+        // 0 or +-1
+        const float v00 = (nb & 0x8u) ? 0.f : 1.f, x00 = ((nb & 0x80u) ? 0.f : 1.f) - v00;
+        const float v10 = (nb & 0x800u) ? 0.f : 1.f, x10 = ((nb & 0x8000u) ? 0.f : 1.f) - v10;
+        const float v01 = (nb & 0x80000u) ? 0.f : 1.f, x01 = ((nb & 0x800000u) ? 0.f : 1.f) - v01;
+        const float v11 = (nb & 0x8000000u) ? 0.f : 1.f, x11 = ((nb & 0x80000000u) ? 0.f : 1.f) - v11;
+        if (fmaxf(cur, sq) < acut) {
+            // The middle's fractions as the mean of the samples' FP32
+            // positions: the exact filter's positions round with the same
+            // sign over many samples, which along a boundary adds up (with
+            // the entry's alone, oblique clinical views came to 2e-5 of the
+            // exact march's, with three samples' to 1.2e-5).
+            float qx = 0.0f, qy = 0.0f, qz = 0.0f;
+            for (int k = 0; k < n; ++k) {
+                qx += __builtin_fmaf(al, rix, sx) - (bx + 1.0f);
+                qy += __builtin_fmaf(al, riy, sy) - (by + 1.0f);
+                qz += __builtin_fmaf(al, riz, sz) - (bz + 1.0f);
+                al += inc;
+            }
+            const float rn = __builtin_amdgcn_rcpf(nf);
+            qx *= rn;
+            qy *= rn;
+            qz *= rn;
+            const Cubic g = cell_cubic(v00, x00, v10, x10, v01, x01, v11, x11, qx, qy, qz, rix, riy, riz);
+            const Cubic fc = cell_cubic(c.d0.x, c.d0.y - c.d0.x, c.d0.z, c.d0.w - c.d0.z, c.d1.x, c.d1.y - c.d1.x,
+                                        c.d1.z, c.d1.w - c.d1.z, qx, qy, qz, rix, riy, riz);
+            const float S4 = S2 * (inc2_12 * 0.6f) * __builtin_fmaf(3.0f * nf, nf, -7.0f);
+            const float S6 = S2 * (inc2_12 * inc2_12 * (9.0f / 7.0f)) *
+                             __builtin_fmaf(nf * nf, __builtin_fmaf(3.0f * nf, nf, -18.0f), 31.0f);
+            const float p2 = __builtin_fmaf(fc.c0, g.c2, __builtin_fmaf(fc.c1, g.c1, fc.c2 * g.c0));
+            const float p4 = __builtin_fmaf(fc.c1, g.c3, __builtin_fmaf(fc.c2, g.c2, fc.c3 * g.c1));
+            const float sum_q = __builtin_fmaf(
+                nf, fc.c0 * g.c0, __builtin_fmaf(S2, p2, __builtin_fmaf(S4, p4, S6 * (fc.c3 * g.c3))));
+            sq += sum_q;
+            cur += __builtin_fmaf(fc.c2, S2, nf * fc.c0) - sum_q;
         } else {
-            float u = -um;
-            for (int k = 0;; ++k) {
-                const bool in = k < n;
-                if (__ballot(in) == 0) break;
-                const float rho = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(fc.c3, u, fc.c2), u, fc.c1), u, fc.c0);
-                cur = __builtin_fmaf(in ? 1.0f : 0.0f, rho, cur);
-                u += inc;
-            }
-        }
-        if (one & !ex) *pa = cur;
-        if (__ballot(ex) != 0) {
-            float al = alpha0;
-            for (int k = 0; __ballot((k < n) & ex) != 0; ++k) {
-                if ((k < n) & ex)
-                    fast_sample<M>(c, acc, __builtin_fmaf(al, rix, sx) - (c.bx + 1.0f),
-                                   __builtin_fmaf(al, riy, sy) - (c.by + 1.0f),
-                                   __builtin_fmaf(al, riz, sz) - (c.bz + 1.0f), 1.0f);
+            // density and second fraction at each sample's FP32 position, by
+            // nested lerps
+            for (int k = 0; k < n; ++k) {
+                const float gx = __builtin_fmaf(al, rix, sx) - (bx + 1.0f);
+                const float gy = __builtin_fmaf(al, riy, sy) - (by + 1.0f);
+                const float gz = __builtin_fmaf(al, riz, sz) - (bz + 1.0f);
+                const float a00 = __builtin_fmaf(gx, c.d0.y - c.d0.x, c.d0.x);
+                const float a10 = __builtin_fmaf(gx, c.d0.w - c.d0.z, c.d0.z);
+                const float a01 = __builtin_fmaf(gx, c.d1.y - c.d1.x, c.d1.x);
+                const float a11 = __builtin_fmaf(gx, c.d1.w - c.d1.z, c.d1.z);
+                const float b0 = __builtin_fmaf(gy, a10 - a00, a00), b1 = __builtin_fmaf(gy, a11 - a01, a01);
+                const float x = __builtin_fmaf(gz, b1 - b0, b0);
+                const float i00 = __builtin_fmaf(gx, x00, v00), i10 = __builtin_fmaf(gx, x10, v10);
+                const float i01 = __builtin_fmaf(gx, x01, v01), i11 = __builtin_fmaf(gx, x11, v11);
+                const float j0 = __builtin_fmaf(gy, i10 - i00, i00), j1 = __builtin_fmaf(gy, i11 - i01, i01);
+                const float xq = x * __builtin_fmaf(gz, j1 - j0, j0);
+                sq += xq;
+                cur += x - xq;
                 al += step;
             }
         }
+        *pb = sq;
+        *pa = cur;
     }
 }
 

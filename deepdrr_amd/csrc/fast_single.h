@@ -30,7 +30,7 @@
 // (in registers the entry block took a compare and a select per material, and
 // their lane masks spilled 95 scalar registers through the loop), and a
 // sample's distance from the cell's first is k inc, with no alpha to follow:
-// 8 views of 500 x 400 through 256 x 256 x 300 march in 4.06 ms, 4.60 before.  The
+// 8 views of 500 x 400 through 256 x 256 x 300 march in 3.88 ms, 4.60 before.  The
 // next cell's record is loaded before this one's samples, for the small
 // launches, which wait for it (fast_march.h): 4 views of 356 x 225 through
 // 150 x 172 x 79 take 0.85 ms, 0.95 without.
@@ -40,8 +40,8 @@
 
 namespace drr {
 
-// Waves per SIMD of the kernels that march so: 8 views of 500 x 400 take 4.06 ms at
-// 5 and 4.09 at 6 (with spills), 2 views of 299 x 102 0.87 and 0.91, 4 views of
+// Waves per SIMD of the kernels that march so: at an earlier stage 8 views of 500 x 400
+// took 4.06 ms at 5 and 4.09 at 6 (with spills), 2 views of 299 x 102 0.87 and 0.91, 4 views of
 // 356 x 225 0.85 and 0.94.
 constexpr int SINGLE_WAVES = 5;
 
@@ -110,18 +110,12 @@ __device__ __forceinline__ void single_run(const VolDev &vol, LdsAccum &a, bool 
                                            int tlim, float amax) {
     // Cell by cell: every lane still marching enters the cell of its current
     // sample together (one execution of the long cell-entry block for the whole
-    // wave), then the wave runs the samples of those cells until every lane has
-    // taken its own.  Lanes whose cells end early idle for the rest of that inner
-    // loop, which costs less than running the entry block once for each group
-    // of lanes that leave together.  A cell's sample count n is fixed on entry:
+    // wave), then runs that cell's samples.  A cell's sample count n is fixed on entry:
     // the samples at u = 0, step, 2 step, ... (for a far source, at the FP32
     // increment) before the exit distance (at least the entry sample, at
     // most the samples left before tlim); a sample within the FP32 alpha
     // sequence's drift of the face may so fall to either cell, where the
-    // density is continuous.  The inner loop's test is a wave vote and
-    // its per-lane choices are 0/1 factors: per-lane branches and loop exits cost
-    // scalar instructions (exec-mask bookkeeping), enough to become the limit in
-    // a loop this short.
+    // density is continuous.
     //
     // Materials: a cell whose labels agree adds each sample's density to the sum
     // of its material.  A cell with exactly two labels
@@ -133,10 +127,7 @@ __device__ __forceinline__ void single_run(const VolDev &vol, LdsAccum &a, bool 
     // rho (1 - f_q) goes to the sum of the first material and rho f_q to that of
     // q; the first is the one that the ray's last samples went to, if the cell
     // has it.  A cell with three or more labels takes the exact filter's
-    // formulas.  In a wave with no two-label
-    // cell the two-label formulas are skipped; a lane in a one-label cell
-    // selects its cubic's value and adds zero to sq, so its results do not
-    // depend on the other lanes.
+    // formulas.
     if (t >= tlim) return;
     // exit distances in steps (reciprocals to 1 ulp are plenty there), kept in
     // registers (an empty asm stops the compiler from forming them again on
@@ -234,27 +225,17 @@ __device__ __forceinline__ void single_run(const VolDev &vol, LdsAccum &a, bool 
         next.load(vol, floorf(px), floorf(py), floorf(pz));
         const bool even = alpha <= top;  // alpha - a0 is k inc at the cell's k-th sample, exactly
         const int ne = even & !ex ? n : 0;
-        // (with g = 1, fma(g, rho, cur) = cur + rho exactly; with 0 it stays)
-        if (__ballot(tw) != 0) {
-            float u = 0.0f, al = a0;
-            for (int k = 0;; ++k) {
-                const bool in = k < ne;
-                if (__ballot(in) == 0) break;
-                const float g = in ? 1.0f : 0.0f;
-                float rho = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(c3, u, c2), u, c1), u, c0);
-                const float xq = second_share(c, al, sx, sy, sz, rix, riy, riz, v00, v10, v01, v11, e00, e10, e01, e11, rho, tw);
-                sq = __builtin_fmaf(g, xq, sq);
-                cur = __builtin_fmaf(g, rho, cur);
-                u += inc;
+        float u = 0.0f, al = a0;
+        if (tw) {
+            for (int k = 0; k < ne; ++k) {
+                float rho;
+                sq += second_share(c, al, sx, sy, sz, rix, riy, riz, v00, v10, v01, v11, e00, e10, e01, e11, rho, true);
+                cur += rho;
                 al += inc;
             }
         } else {
-            float u = 0.0f;
-            for (int k = 0;; ++k) {
-                const bool in = k < ne;
-                if (__ballot(in) == 0) break;
-                const float rho = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(c3, u, c2), u, c1), u, c0);
-                cur = __builtin_fmaf(in ? 1.0f : 0.0f, rho, cur);
+            for (int k = 0; k < ne; ++k) {
+                cur += __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(c3, u, c2), u, c1), u, c0);
                 u += inc;
             }
         }
