@@ -480,7 +480,7 @@ def main():
                                      f"schedule ({PMC_SUMMARY})" if traffic is not None else None),
                   "valu": valu, "l2_hit_rate": l2_hit,
                   "kernel": f"k_batch_march<{len(materials)},false,{plan.tuning[0]},"
-                            f"{'true' if args.march == 'fast' else 'false'}>",
+                            f"{1 if args.march == 'fast' else 0}>",
                   "kernel_ms": kernel_ms, "samples_per_launch": samples_per_launch,
                   "samples_per_s": samples_per_launch / (kernel_ms * 1e-3),
                   "gather_equivalent": {

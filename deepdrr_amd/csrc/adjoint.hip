@@ -374,8 +374,8 @@ struct AdjRay {
     // Cell by cell: every lane still marching hands over its open cell, takes the
     // cell of its current sample and sums that cell's samples together (one
     // execution of that long block for the whole wave).  The next cell's record
-    // is loaded before the present one is summed.  VALU issue bounds it (0.94 of
-    // the cycles; one label 250 instructions, several 400 more).  64 views of 256^2
+    // is loaded before the present one is summed.  VALU issue bounds it (0.82 of
+    // the slots; one label 250 instructions, several 400 more).  64 views of 256^2
     // through 192^3: 28.6 ms with the samples of several labels one by one (91
     // instructions each), 22.5 in closed form, 16.9 with the box in FP64.
     template <class Dep, class Go>
