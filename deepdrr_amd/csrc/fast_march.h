@@ -99,17 +99,6 @@ __device__ __forceinline__ uint32_t nz_nibbles(uint32_t x) {
     return (((x & 0x77777777u) + 0x77777777u) | x) & 0x88888888u;
 }
 
-// What rounding to cur's precision adds to the mean of samples that are added to
-// cur one by one, where the samples run from lo to hi.  The rounding error of a
-// term x is a sawtooth in x, whose integral is its square, so over a ramp the
-// mean of the errors is (el^2 - eh^2) / (2 (hi - lo)) with those at the ends.
-__device__ __forceinline__ float mean_rounding(float cur, float lo, float hi) {
-    const float el = ((cur + lo) - cur) - lo, eh = ((cur + hi) - cur) - hi, d = hi - lo;
-    const float s = 0.5f * (el + eh);
-    // (el - eh is d where the ends round to the same value)
-    return fabsf(d) > 9.5367432e-7f * fabsf(hi) ? s * ((el - eh) * __builtin_amdgcn_rcpf(d)) : s;
-}
-
 // One sample of weight wt by the exact filter's formulas, added to the sums.
 template <int M>
 __device__ __forceinline__ void fast_sample(const Cell &c, float *acc, float fx, float fy, float fz, float wt) {

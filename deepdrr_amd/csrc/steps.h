@@ -1,6 +1,6 @@
 // steps.h -- the march's FP32 sequences `x += d` taken many steps at a time with
-// the results of the single additions.  Host code runs them too, to check them
-// against the plain loops.
+// the results of the single additions, and the mean of what such additions
+// round off.  Host code runs them too, to check them against the plain loops.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -93,6 +93,24 @@ __host__ __device__ __forceinline__ int stretch(float alpha, float step, float m
         k += 1.0f;
     const int n = (int)k + 1;
     return n < most ? n : most;
+}
+
+// What rounding to cur's precision adds to the mean of samples that are added to
+// cur one by one, where the samples run from lo to hi.  The rounding error of a
+// term x is a sawtooth in x, whose integral is its square, so over a ramp the
+// mean of the errors is (el^2 - eh^2) / (2 (hi - lo)) with those at the ends.
+__host__ __device__ __forceinline__ float mean_rounding(float cur, float lo, float hi) {
+    const float el = ((cur + lo) - cur) - lo, eh = ((cur + hi) - cur) - hi, d = hi - lo;
+    const float s = 0.5f * (el + eh);
+    // el - eh is d where the ends round to the same value.  A difference too
+    // small for its own rounding to leave anything of it, or for its reciprocal
+    // to be a number (smooth densities have subnormal tails), counts as none.
+#ifdef __HIP_DEVICE_COMPILE__
+    const float id = __builtin_amdgcn_rcpf(d);
+#else
+    const float id = 1.0f / d;
+#endif
+    return fabsf(d) > __builtin_fmaf(9.5367432e-7f, fabsf(hi), 1e-30f) ? s * ((el - eh) * id) : s;
 }
 
 }  // namespace drr
