@@ -142,7 +142,11 @@ int jobs_prepare(drr_ctx *ctx, const drr_volume *const *vols, int n_vols, const 
     t.n_mjobs = (int)h.mjobs.size();
     for (int q = 0; q <= 8; q++) h.seg[q] = (int)(t.n_items * q / 8);
     h.vols.resize(n_vols);
-    for (int v = 0; v < n_vols; v++) h.vols[v] = vol_to_dev(vols[v]);
+    t.n_labels = 0;
+    for (int v = 0; v < n_vols; v++) {
+        h.vols[v] = vol_to_dev(vols[v]);
+        t.n_labels = std::max(t.n_labels, vols[v]->n_labels);
+    }
     t.block = 64 * tune.waves_per_block;
     t.grid = ctx->n_cus * tune.blocks_per_cu;
     return DRR_OK;
@@ -246,11 +250,12 @@ template <int M, bool ATTEN, int MARCH>
 static void launch_march_tw(int tw, const JobTable &t, hipStream_t st, SpectrumDev sp, float step, int air,
                             float *I, float *P, float *AD) {
     dim3 g(t.grid), b(t.block);
+    const size_t lds = march_bytes(MARCH, M, t.n_labels);
     if (tw == 16)
-        k_batch_march<M, ATTEN, 16, MARCH><<<g, b, 0, st>>>(t.d_jobs, t.d_vols, t.d_items, t.d_seg, t.d_counters,
+        k_batch_march<M, ATTEN, 16, MARCH><<<g, b, lds, st>>>(t.d_jobs, t.d_vols, t.d_items, t.d_seg, t.d_counters,
                                                              sp, step, air, I, P, AD);
     else
-        k_batch_march<M, ATTEN, 8, MARCH><<<g, b, 0, st>>>(t.d_jobs, t.d_vols, t.d_items, t.d_seg, t.d_counters,
+        k_batch_march<M, ATTEN, 8, MARCH><<<g, b, lds, st>>>(t.d_jobs, t.d_vols, t.d_items, t.d_seg, t.d_counters,
                                                             sp, step, air, I, P, AD);
 }
 
@@ -301,8 +306,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI_WAVES
     lane_pixel(tile % J.tiles_x, tile / J.tiles_x, lane, udx, vdx);
     if (udx >= J.vd.width || vdx >= J.vd.height) return;
     float ad[M];
-    __shared__ float sums[M * LDS_LANES];  // each thread its own words
-    march_multi<V, M>(J.vd, udx, vdx, step, atten, air, sums + threadIdx.x, ad);
+    march_multi<V, M>(J.vd, udx, vdx, step, atten, air, thread_sums(), ad);
     float inten, pp;
     spectral<M>(sp, ad, inten, pp);
     const int64_t npix = (int64_t)J.vd.width * J.vd.height;
@@ -322,9 +326,10 @@ static void launch_multi_v(const JobTable &t, int M, hipStream_t st, SpectrumDev
     if (n <= 0) return;
     const dim3 g((unsigned)((n + 3) / 4)), b(256);
     const int2 *items = t.d_mitems + t.m_first[V];
+    const size_t lds = sums_bytes(M, t.n_labels);
     switch (M) {
 #define DRR_CASE(MM) \
-    case MM: k_batch_multi<V, MM><<<g, b, 0, st>>>(t.d_mjobs, items, n, sp, step, atten, air, I, P, AD); break;
+    case MM: k_batch_multi<V, MM><<<g, b, lds, st>>>(t.d_mjobs, items, n, sp, step, atten, air, I, P, AD); break;
         DRR_CASE(1) DRR_CASE(2) DRR_CASE(3) DRR_CASE(4) DRR_CASE(5) DRR_CASE(6) DRR_CASE(7) DRR_CASE(8) \
         DRR_CASE(9) DRR_CASE(10) DRR_CASE(11) DRR_CASE(12) DRR_CASE(13) DRR_CASE(14) DRR_CASE(15) DRR_CASE(16)
 #undef DRR_CASE

@@ -139,6 +139,7 @@ struct drr_volume_s {
     int device = 0;  // HIP device of the allocation (outlives the context)
     int nx = 0, ny = 0, nz = 0;
     int64_t n_cells = 0;
+    int n_labels = 0;  // every label is below it: the scene's materials when the volume was made
     PoolBuf cell_buf;
     uint32_t *cells = nullptr;  // DRR_CELL_WORDS 32-bit words per cell
     // voxel-order records [nz][ny][nx] of (density bits, label), made on first
@@ -183,7 +184,6 @@ int drr_hip_error(hipError_t e, const char *what);
 
 // One volume as the march sees it.
 struct VolDev {
-    const uint32_t *cells;
     int nx, ny, nz;
     // Cell index in FP32 arithmetic for clamped cell coordinates (cx, cy, cz)
     // (march.h, Cell::load): with e1 = cz * a1 + (cy * b1 + c1) and
@@ -194,7 +194,9 @@ struct VolDev {
     uint32_t s1;
     float cmax[3];  // nx - 1, ny - 1, nz - 1: the largest cell coordinate
     uint64_t cells_b;  // address of the record of index -0x4B000000
+    int n_labels;      // every label of the cells is below it
 };
+static_assert(sizeof(VolDev) == 64, "the fixed scratch of drr_project_jobs_noalloc holds as many volumes as ever");
 
 // Parameters of the FP32 cell index.  Form A ((nx+1)(ny+1) <= 2^23):
 // e1 = cz + 1, e2 = (cy+1)(nx+1) + (cx+1) + 2^23, s1 = (nx+1)(ny+1).  Form B
@@ -205,7 +207,6 @@ struct VolDev {
 // taken off the base addresses instead of each index.
 inline VolDev vol_index_params(const uint32_t *cells, int nx, int ny, int nz) {
     VolDev d{};
-    d.cells = cells;
     d.nx = nx;
     d.ny = ny;
     d.nz = nz;
@@ -297,7 +298,9 @@ __host__ __device__ __forceinline__ uint32_t cell_index_biased(const VolDev &v, 
 }
 
 inline VolDev vol_to_dev(const drr_volume *v) {
-    return vol_index_params(v->cells, v->nx, v->ny, v->nz);
+    VolDev d = vol_index_params(v->cells, v->nx, v->ny, v->nz);
+    d.n_labels = v->n_labels;
+    return d;
 }
 
 inline void view_to_dev(const drr_view_t &v, const drr_volume *const *vols, ViewDev &d) {

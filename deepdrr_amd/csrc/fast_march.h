@@ -269,7 +269,7 @@ __device__ __forceinline__ void march_fast(const Geo1 &g, const VolDev &vol, int
                                            float *acc, float (&ad)[M]) {
     RayV1 r;
     march_setup_v1(g, udx, vdx, step, r);
-    for (int m = 0; m < M; m++) acc[LDS_LANES * m] = 0.0f;
+    clear_sums<M>(acc, vol.n_labels);
     float air_sum = 0.0f;
     if (ATTEN) air_sum = (float)((double)air_sum + (double)(r.minA / step) * DRR_AIR_DENSITY);
     const int N = r.N;

@@ -275,7 +275,7 @@ __device__ __forceinline__ void march_fast_single(const Geo1 &g, const VolDev &v
                                                   float step, int air, float *sums, float (&ad)[M]) {
     RayV1 r;
     march_setup_v1(g, udx, vdx, step, r);
-    for (int m = 0; m < M; m++) sums[LDS_LANES * m] = 0.0f;
+    clear_sums<M>(sums, vol.n_labels);
     float acc = 0.0f;  // air accumulator while no volume is sampled
     if (ATTEN) acc = (float)((double)acc + (double)(r.minA / step) * DRR_AIR_DENSITY);
 
@@ -369,16 +369,20 @@ __device__ __forceinline__ void march_fast_single(const Geo1 &g, const VolDev &v
     for (int m = 0; m < M; m++) ad[m] /= 10.0f;
 }
 
+// LDS of a launch that marches so.
+inline size_t march_bytes(int march, int n_materials, int n_labels) {
+    return march == MARCH_V1_EXACT ? 0 : sums_bytes(n_materials, n_labels);
+}
+
 // The single-volume march of a thread of a block of at most LDS_LANES.
 template <int M, bool ATTEN, int MARCH>
 __device__ __forceinline__ void march_single_volume(const Geo1 &g, const VolDev &vol, int udx, int vdx, float step,
                                                     int air, float (&ad)[M]) {
     if constexpr (MARCH != MARCH_V1_EXACT) {
-        __shared__ float sums[M * LDS_LANES];  // each thread its own words
         if constexpr (MARCH == MARCH_V1_FAST)
-            march_fast<M, ATTEN>(g, vol, udx, vdx, step, air, sums + threadIdx.x, ad);
+            march_fast<M, ATTEN>(g, vol, udx, vdx, step, air, thread_sums(), ad);
         else
-            march_fast_single<M, ATTEN>(g, vol, udx, vdx, step, air, sums + threadIdx.x, ad);
+            march_fast_single<M, ATTEN>(g, vol, udx, vdx, step, air, thread_sums(), ad);
     } else {
         march_v1<M, ATTEN>(g, vol, udx, vdx, step, air, ad);
     }

@@ -131,8 +131,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI_WAVES
     lane_pixel(bx * 2 + (wave & 1), by * 2 + (wave >> 1), lane, udx, vdx);
     if (udx >= vd.width || vdx >= vd.height) return;
     float ad[M];
-    __shared__ float sums[M * LDS_LANES];  // each thread its own words
-    march_multi<V, M>(vd, udx, vdx, step, atten, air, sums + threadIdx.x, ad);
+    march_multi<V, M>(vd, udx, vdx, step, atten, air, thread_sums(), ad);
     float I, P;
     spectral<M>(sp, ad, I, P);
     const int64_t npix = (int64_t)vd.width * vd.height;
@@ -149,12 +148,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI_WAVES
 template <int M>
 static void launch_v1(bool atten, int march, dim3 g, dim3 b, hipStream_t st, const Geo1 &geo, const VolDev &vol,
                       const SpectrumDev &sp, float step, int air, const OutDev &o, int tx, int rows) {
-#define DRR_MARCH_CASE(MARCH)                                                                    \
-    case MARCH:                                                                                  \
-        if (atten)                                                                               \
-            k_project_v1<M, true, MARCH><<<g, b, 0, st>>>(geo, vol, sp, step, air, o, tx, rows);  \
-        else                                                                                     \
-            k_project_v1<M, false, MARCH><<<g, b, 0, st>>>(geo, vol, sp, step, air, o, tx, rows); \
+    const size_t lds = march_bytes(march, M, vol.n_labels);
+#define DRR_MARCH_CASE(MARCH)                                                                      \
+    case MARCH:                                                                                    \
+        if (atten)                                                                                 \
+            k_project_v1<M, true, MARCH><<<g, b, lds, st>>>(geo, vol, sp, step, air, o, tx, rows);  \
+        else                                                                                       \
+            k_project_v1<M, false, MARCH><<<g, b, lds, st>>>(geo, vol, sp, step, air, o, tx, rows); \
         break;
     switch (march) {
         DRR_MARCH_CASE(MARCH_V1_EXACT) DRR_MARCH_CASE(MARCH_V1_FAST) DRR_MARCH_CASE(MARCH_V1_SINGLE)
@@ -166,9 +166,10 @@ template <int V>
 static void launch_multi(int M, dim3 g, dim3 b, hipStream_t st, const ViewDev &vd,
                          const SpectrumDev &sp, float step, int atten, int air, const OutDev &o,
                          int tx) {
+    const size_t lds = sums_bytes(M, max_labels(vd, V));
     switch (M) {
 #define DRR_CASE(MM) \
-    case MM: k_project_multi<V, MM><<<g, b, 0, st>>>(vd, sp, step, atten, air, o, tx); break;
+    case MM: k_project_multi<V, MM><<<g, b, lds, st>>>(vd, sp, step, atten, air, o, tx); break;
         DRR_CASE(1) DRR_CASE(2) DRR_CASE(3) DRR_CASE(4) DRR_CASE(5) DRR_CASE(6) DRR_CASE(7) DRR_CASE(8) \
         DRR_CASE(9) DRR_CASE(10) DRR_CASE(11) DRR_CASE(12) DRR_CASE(13) DRR_CASE(14) DRR_CASE(15) DRR_CASE(16)
 #undef DRR_CASE

@@ -37,6 +37,7 @@ struct JobTable {
     PoolBuf buf;  // every table below, and the caller's extra bytes
     void *d_extra = nullptr;
     int n_jobs = 0, n_vols = 0;
+    int n_labels = 0;  // every label of the volumes is below it
     JobDev *d_jobs = nullptr;   // single-volume jobs (entries of multi-volume jobs unused)
     VolDev *d_vols = nullptr;
     int2 *d_items = nullptr;    // single-volume tiles (job, tile)

@@ -352,8 +352,33 @@ __device__ __forceinline__ void march_v1(const Geo1 &g, const VolDev &vol, int u
 // sums[LDS_LANES m] from the thread's first; consecutive lanes in consecutive
 // banks): an access by a label known only at run time is one LDS access, where
 // registers take a compare and a select per material and hold M registers and
-// their masks through the march.
+// their masks through the march.  There is a word for every label of the volumes
+// (sums_bytes): a scene may come to have fewer materials than the volumes were
+// made with, whose labels then go to no material, but have their words.
 constexpr int LDS_LANES = 256;  // threads per block of the kernels that use them
+
+inline int max_labels(const ViewDev &vd, int n_volumes) {
+    int n = 0;
+    for (int i = 0; i < n_volumes; i++) n = vd.vol[i].n_labels > n ? vd.vol[i].n_labels : n;
+    return n;
+}
+
+inline size_t sums_bytes(int n_materials, int n_labels) {
+    return sizeof(float) * LDS_LANES * (n_materials > n_labels ? n_materials : n_labels);
+}
+
+template <int M>
+__device__ __forceinline__ void clear_sums(float *sums, int n_labels) {
+#pragma unroll
+    for (int m = 0; m < M; m++) sums[LDS_LANES * m] = 0.0f;
+    for (int m = M; m < n_labels; m++) sums[LDS_LANES * m] = 0.0f;
+}
+
+// This thread's words, of the LDS that the launch asked for with sums_bytes.
+__device__ __forceinline__ float *thread_sums() {
+    extern __shared__ float lane_sums[];
+    return lane_sums + threadIdx.x;
+}
 
 // Running sum of the current one-label material of such sums.
 struct LdsAccum {
@@ -476,7 +501,10 @@ __device__ __forceinline__ void march_multi(const ViewDev &vd, int udx, int vdx,
     float rx, ry, rz, L;
     ray_dir(vd.W, udx, vdx, rx, ry, rz, L);
     float minA = L, maxA = 0.0f;
-    for (int m = 0; m < M; m++) sums[LDS_LANES * m] = 0.0f;
+    int n_labels = 0;
+#pragma unroll
+    for (int i = 0; i < V; i++) n_labels = max(n_labels, vd.vol[i].n_labels);
+    clear_sums<M>(sums, n_labels);
     constexpr int VA = V > 0 ? V : 1;  // array extent (V = 0: meshes only)
     float ri[VA][3], mnv[VA], mxv[VA];
     float first = INFINITY, last = -INFINITY;  // the ray's part inside any volume

@@ -642,8 +642,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI_WAVES
                0.0f,               0.0f,        false};
     mr.next();
     float ad[M];
-    __shared__ float sums[M * LDS_LANES];  // each thread its own words
-    march_multi<V, M, MeshRay>(vd, udx, vdx, step, atten, air, sums + threadIdx.x, ad, mr);
+    march_multi<V, M, MeshRay>(vd, udx, vdx, step, atten, air, thread_sums(), ad, mr);
     float I, P;
     spectral<M>(sp, ad, I, P);
     out.intensity[idx] = I;
@@ -658,9 +657,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI_WAVES
 template <int V>
 void launch_mesh_march(int M, dim3 g, dim3 b, hipStream_t st, const ViewDev &vd, const SpectrumDev &sp, float step,
                        int atten, int air, const MeshTerms &mt, const OutMesh &o, int tx) {
+    const size_t lds = sums_bytes(M, max_labels(vd, V));
     switch (M) {
 #define DRR_CASE(MM) \
-    case MM: k_project_mesh<V, MM><<<g, b, 0, st>>>(vd, sp, step, atten, air, mt, o, tx); break;
+    case MM: k_project_mesh<V, MM><<<g, b, lds, st>>>(vd, sp, step, atten, air, mt, o, tx); break;
         DRR_CASE(1) DRR_CASE(2) DRR_CASE(3) DRR_CASE(4) DRR_CASE(5) DRR_CASE(6) DRR_CASE(7) DRR_CASE(8) \
         DRR_CASE(9) DRR_CASE(10) DRR_CASE(11) DRR_CASE(12) DRR_CASE(13) DRR_CASE(14) DRR_CASE(15) DRR_CASE(16)
 #undef DRR_CASE

@@ -196,6 +196,7 @@ static int volume_alloc(drr_ctx *ctx, int nx, int ny, int nz, drr_volume **out) 
     v->ny = ny;
     v->nz = nz;
     v->n_cells = (int64_t)(nx + 1) * (ny + 1) * (nz + 1);
+    v->n_labels = ctx->scene.n_materials;
     hipError_t e = v->cell_buf.take(ctx->pool, sizeof(uint32_t) * DRR_CELL_WORDS * v->n_cells);
     v->cells = v->cell_buf.as<uint32_t>();
     if (e != hipSuccess) {
