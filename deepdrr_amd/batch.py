@@ -174,7 +174,8 @@ class PendingFetch:
 def plan_for_projector(projector, projections: Sequence[geo.CameraProjection],
                        volume_indices: Optional[Sequence[int]] = None, neglog: Optional[bool] = None,
                        tuning=None) -> BatchPlan:
-    """Batch plan over an initialised ``Projector``'s volumes."""
+    """Batch plan over an initialised ``Projector``'s volumes, marched as its
+    ``project`` does now (with ``add_noise``: every sample added singly)."""
     from .projector import build_views
 
     if not projector.initialized:
@@ -187,12 +188,15 @@ def plan_for_projector(projector, projections: Sequence[geo.CameraProjection],
     if volume_indices is None:
         # every view over all the projector's volumes, as project() renders it
         volume_indices = [0] * len(projections)
+    # before the plan, and before the schedules that are timed for it
+    projector._set_sums()
     key = None
     if tuning == "auto":
         from . import autotune
 
+        march = projector.march + (", single sums" if projector.march == "fast" and projector.add_noise else "")
         key = autotune.workload_key(views, volume_indices, [v.shape for v in projector.volumes],
-                                    len(projector.all_materials), march=projector.march)
+                                    len(projector.all_materials), march=march)
     return BatchPlan(projector._ctx, projector._vols, views, volume_indices,
                      neglog=projector.neglog if neglog is None else neglog, tuning=tuning,
                      device=projector._torch_device, tune_key=key)

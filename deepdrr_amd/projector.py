@@ -439,7 +439,8 @@ class Projector:
         return self._mesh
 
     def _set_sums(self):
-        # noise drawn for a seed follows the photon probabilities' roundings
+        # noise drawn for a seed follows the photon probabilities' roundings; set
+        # before every launch and every plan, since add_noise may change
         _abi.call("drr_ctx_set_single_sums", self._ctx, 1 if self.add_noise else 0)
 
     def _launch_view(self, proj: geo.CameraProjection, intensity, photon_prob, area_density, solid_angle, stream):
@@ -525,7 +526,6 @@ class Projector:
                         and self.intensity_upper_bound is None)
         host_epilogue = (self.add_noise and not device_noise) or self.intensity_upper_bound is not None \
             or self.mc_scatter_histories > 0
-        self._set_sums()
         plan = plan_for_projector(self, camera_projections, volume_indices,
                                   neglog=self.neglog and not host_epilogue and not device_noise, tuning=tuning)
         try:
