@@ -65,8 +65,7 @@ class PoseGeometry:
         w_from_ijk = T @ self.world_from_ijk
         ijk_from_w = np.linalg.inv(w_from_ijk)
         out = []
-        if not projections:
-            return out
+        projections = list(projections)
         for proj, rows, src in zip(projections, *cameras(projections, 1.0)):
             s_ijk = (ijk_from_w @ np.append(src, 1.0))[:3]
             w, h = proj.intrinsic.sensor_size
