@@ -73,23 +73,28 @@ def world_from_index_rows(proj: geo.CameraProjection, sdd: float) -> np.ndarray:
 def cameras(projections: Sequence[geo.CameraProjection], sdd: float):
     """``world_from_index_rows`` and the camera centre in world [3] of each
     projection, with one call for all the inverses (they take most of a view's
-    preparation: 64 views 1.5 ms one by one, 0.5 ms so)."""
-    if not projections:
-        return [], []
-    k_inv = np.linalg.inv(np.stack([p.intrinsic.data for p in projections]))
-    known = [p.extrinsic._inv for p in projections]
-    open_ = [i for i, m in enumerate(known) if m is None]
-    if open_:
-        for i, m in zip(open_, np.linalg.inv(np.stack([projections[i].extrinsic.data for i in open_]))):
-            known[i] = m
-    rows, centers = [], []
-    for m, k in zip(known, k_inv):
-        w = m[:3, :3] @ k
-        if geo.RAY_SCALE == "source_to_pixel":
-            w = w * sdd
-        rows.append(w.astype(np.float32))
-        centers.append(m[:3, 3].copy())
-    return rows, centers
+    preparation: 64 views 1.5 ms one by one, 0.5 ms so).  Only plain
+    ``CameraProjection`` of plain poses are taken together; any other camera is
+    asked for its own properties."""
+    out = [None] * len(projections)
+    plain = [i for i, p in enumerate(projections)
+             if type(p) is geo.CameraProjection and type(p.extrinsic) is geo.FrameTransform]
+    if plain:
+        k_inv = np.linalg.inv(np.stack([projections[i].intrinsic.data for i in plain]))
+        known = [projections[i].extrinsic._inv for i in plain]
+        open_ = [j for j, m in enumerate(known) if m is None]
+        if open_:
+            for j, m in zip(open_, np.linalg.inv(np.stack([projections[plain[j]].extrinsic.data for j in open_]))):
+                known[j] = m
+        for i, m, k in zip(plain, known, k_inv):
+            w = m[:3, :3] @ k
+            if geo.RAY_SCALE == "source_to_pixel":
+                w = w * sdd
+            out[i] = w.astype(np.float32), m[:3, 3].copy()
+    for i, p in enumerate(projections):
+        if out[i] is None:
+            out[i] = world_from_index_rows(p, sdd), np.array(p.center_in_world)
+    return [r for r, _ in out], [c for _, c in out]
 
 
 def build_views(volumes: Sequence[Volume], priorities: Sequence[int], projections: Sequence[geo.CameraProjection],
