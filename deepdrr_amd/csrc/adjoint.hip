@@ -287,6 +287,18 @@ struct AdjRay {
         for (int d = 0; d < 8; d++) acc[d] = nacc[d];
     }
 
+    // Fraction of the position s + alpha r - 1 against its cell's base b, to the
+    // precision of a fraction (s - (b + 1) as a rounded difference and its
+    // rounding error).  The difference of the FP32 position and b has the position's
+    // precision, and a closed sum takes it for all samples of the cell, where it
+    // does not average out: gradients through random labels were 3.2e-7 (density)
+    // and 4.8e-7 (pose) from 64 bits, 1.6e-7 and 2.6e-7 with the samples one by one, and are
+    // 1.2e-7 and 2.2e-7.  64 views of 256^2 through 192^3 take 17.2 ms for 16.9.
+    __device__ __forceinline__ static float fraction(float s, float alpha, float r, float b) {
+        const float c = b + 1.0f, hi = s - c, bb = hi - s;
+        return __builtin_fmaf(alpha, r, hi) + ((s - (hi - bb)) - (c + bb));
+    }
+
     // Sums of a cell's n samples of weight wt (1, or n = 1) in closed form.  The samples sit at
     // u_k = k h (k < n) from the entry sample, whose fractions against the cell
     // are f.  About the run's midpoint u_m = h (n - 1) / 2, with v = u - u_m,
@@ -463,7 +475,8 @@ struct AdjRay {
                 const float wt = ((uint32_t)(t - 1) >= (uint32_t)(N - 2)) ? 0.5f : 1.0f;
                 next.load(vol, floorf(sample_pos(sx, an, rix)), floorf(sample_pos(sy, an, riy)),
                           floorf(sample_pos(sz, an, riz)));
-                cell_sums<Dep::kDensity>(n, wt, s1, alpha, ex, ey, ez, rix, riy, riz);
+                cell_sums<Dep::kDensity>(n, wt, s1, alpha, fraction(sx, alpha, rix, c.bx), fraction(sy, alpha, riy, c.by),
+                                         fraction(sz, alpha, riz, c.bz), rix, riy, riz);
                 alpha = an;
                 t += n;
             }
