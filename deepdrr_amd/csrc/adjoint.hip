@@ -970,6 +970,7 @@ extern "C" int drr_adjoint_jobs(drr_ctx *ctx, const drr_volume *vol, const drr_j
     (void)hipEventRecord(ctx->ev1, st);
     ctx->timed = true;
     hipError_t e2 = hipStreamSynchronize(st);
+    if (e2 != hipSuccess) t.buf.discard();
     drr_jobs_free(t);
     if (prev >= 0 && prev != ctx->device) (void)hipSetDevice(prev);
     if (e != hipSuccess) return drr_hip_error(e, "drr_adjoint_jobs launch");

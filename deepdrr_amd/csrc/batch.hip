@@ -469,7 +469,10 @@ extern "C" int drr_batch_destroy(drr_batch *B) {
     if (!B) return DRR_OK;
     DevSwitch ds(B->ctx->device);
     // its tables go back to the pool: no launch, on whatever stream, may still read them
-    if (B->launched) (void)hipDeviceSynchronize();
+    if (B->launched && hipDeviceSynchronize() != hipSuccess) {
+        B->t.buf.discard();
+        B->imgs_keys.discard();
+    }
     batch_free(B);
     return DRR_OK;
 }
@@ -498,6 +501,7 @@ extern "C" int drr_project_jobs_march(drr_ctx *ctx, const drr_volume *const *vol
     (void)hipEventRecord(ctx->ev1, st);
     ctx->timed = true;
     hipError_t e2 = hipStreamSynchronize(st);
+    if (e2 != hipSuccess) t.buf.discard();
     drr_jobs_free(t);
     if (e != hipSuccess) return drr_hip_error(e, "drr_project_jobs launch");
     if (e2 != hipSuccess) return drr_hip_error(e2, "drr_project_jobs");

@@ -20,8 +20,6 @@
 #include <memory>
 #include <mutex>
 #include <string>
-#include <utility>
-#include <vector>
 
 #include "../../include/deepdrr_amd.h"
 
@@ -31,76 +29,136 @@
 // buffer is put back only after the GPU work that uses it has ended, so any
 // thread or stream may take it next.  At most 32 buffers and 64 MB of up to 16 MB
 // each are kept, and one of up to 2 GB: a volume's cells, which a fit makes anew
-// for every density (freeing 87 MB takes 0.3 ms).  They are freed with the
-// context, or when memory runs out; those that outlive it by their owner.
+// for every density (freeing 87 MB takes 0.3 ms); it serves that size alone and
+// is freed when another is asked for.  All are freed with the context, those that
+// outlive it by their owner, and every context's when an allocation of the library
+// (drr_device_malloc) finds no memory.
 class DevPool {
   public:
+    DevPool() {
+        std::lock_guard<std::mutex> lk(all_mu_);
+        next_ = all_;
+        all_ = this;
+    }
     ~DevPool() {
-        for (auto &b : free_) (void)hipFree(b.second);
-    }
-    // Contents undefined; `size` is what has to be given back with the buffer.
-    hipError_t take(size_t bytes, void **p, size_t *size) {
-        const size_t unit = bytes > ((size_t)1 << 20) ? (size_t)1 << 20 : 4096;
-        const size_t n = (bytes + unit - 1) / unit * unit;
         {
-            std::lock_guard<std::mutex> lk(mu_);
-            size_t best = free_.size();  // the smallest that fits and is not over twice as large
-            for (size_t i = 0; i < free_.size(); i++)
-                if (free_[i].first >= n && free_[i].first <= 2 * n &&
-                    (best == free_.size() || free_[i].first < free_[best].first))
-                    best = i;
-            if (best < free_.size()) {
-                *size = free_[best].first;
-                *p = free_[best].second;
-                if (*size <= BIG) held_ -= *size;
-                free_[best] = free_.back();
-                free_.pop_back();
-                return hipSuccess;
-            }
+            std::lock_guard<std::mutex> lk(all_mu_);
+            DevPool **at = &all_;
+            while (*at != this) at = &(*at)->next_;
+            *at = next_;
         }
-        *size = n;
-        hipError_t e = hipMalloc(p, n);
-        if (e == hipErrorOutOfMemory && drop()) {
-            (void)hipGetLastError();
-            e = hipMalloc(p, n);
-        }
-        return e;
+        (void)drop();
     }
+    DevPool(const DevPool &) = delete;
+    DevPool &operator=(const DevPool &) = delete;
+
+    // Contents undefined; `size` is what has to be given back with the buffer.
+    hipError_t take(size_t bytes, void **p, size_t *size);
+
     void put(void *p, size_t size) {
         {
             std::lock_guard<std::mutex> lk(mu_);
-            bool keep;
             if (size > BIG) {
-                keep = size <= ((size_t)2 << 30);
-                for (auto &b : free_) keep &= b.first <= BIG;
-            } else {
-                keep = free_.size() < 32 && held_ + size <= ((size_t)64 << 20);
-            }
-            if (keep) {
-                free_.emplace_back(size, p);
-                if (size <= BIG) held_ += size;
+                if (size <= ((size_t)2 << 30) && !big_.p) {
+                    big_ = Buf{size, p};
+                    return;
+                }
+            } else if (n_ < MOST && held_ + size <= ((size_t)64 << 20)) {
+                free_[n_++] = Buf{size, p};
+                held_ += size;
                 return;
             }
         }
         (void)hipFree(p);
     }
 
+    // Free what every context keeps; whether there was anything.
+    static bool drop_all() {
+        std::lock_guard<std::mutex> lk(all_mu_);
+        bool any = false;
+        for (DevPool *q = all_; q; q = q->next_) any |= q->drop();
+        return any;
+    }
+
   private:
+    struct Buf {
+        size_t size;
+        void *p;
+    };
     static constexpr size_t BIG = (size_t)16 << 20;
-    bool drop() {  // free what is kept
-        std::vector<std::pair<size_t, void *>> all;
+    static constexpr int MOST = 32;
+    bool drop() {
+        Buf all[MOST + 1];
+        int n;
         {
             std::lock_guard<std::mutex> lk(mu_);
-            all.swap(free_);
+            n = n_;
+            for (int i = 0; i < n; i++) all[i] = free_[i];
+            if (big_.p) all[n++] = big_;
+            n_ = 0;
             held_ = 0;
+            big_ = Buf{0, nullptr};
         }
-        for (auto &b : all) (void)hipFree(b.second);
-        return !all.empty();
+        for (int i = 0; i < n; i++) (void)hipFree(all[i].p);
+        return n > 0;
     }
     std::mutex mu_;
-    std::vector<std::pair<size_t, void *>> free_;
-    size_t held_ = 0;
+    Buf free_[MOST];
+    Buf big_{0, nullptr};
+    int n_ = 0;
+    size_t held_ = 0;  // bytes in free_
+    DevPool *next_ = nullptr;
+    static inline std::mutex all_mu_;
+    static inline DevPool *all_ = nullptr;
 };
+
+// hipMalloc that has the contexts give back what they keep before it fails.
+inline hipError_t drr_device_malloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && DevPool::drop_all()) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+template <typename T>
+inline hipError_t drr_device_malloc(T **p, size_t bytes) {
+    return drr_device_malloc(reinterpret_cast<void **>(p), bytes);
+}
+
+inline hipError_t DevPool::take(size_t bytes, void **p, size_t *size) {
+    const size_t unit = bytes > ((size_t)1 << 20) ? (size_t)1 << 20 : 4096;
+    const size_t n = (bytes + unit - 1) / unit * unit;
+    void *stale = nullptr;
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        if (n > BIG) {
+            const Buf b = big_;
+            big_ = Buf{0, nullptr};
+            if (b.p && b.size == n) {
+                *size = n;
+                *p = b.p;
+                return hipSuccess;
+            }
+            stale = b.p;
+        } else {
+            int best = n_;  // the smallest that fits and is not over twice as large
+            for (int i = 0; i < n_; i++)
+                if (free_[i].size >= n && free_[i].size <= 2 * n && (best == n_ || free_[i].size < free_[best].size))
+                    best = i;
+            if (best < n_) {
+                *size = free_[best].size;
+                *p = free_[best].p;
+                held_ -= *size;
+                free_[best] = free_[--n_];
+                return hipSuccess;
+            }
+        }
+    }
+    if (stale) (void)hipFree(stale);
+    *size = n;
+    return drr_device_malloc(p, n);
+}
 
 // A buffer of a pool, given back when its owner drops it.
 class PoolBuf {
@@ -120,6 +178,12 @@ class PoolBuf {
     }
     void reset() {
         if (p_) pool_->put(p_, size_);
+        p_ = nullptr;
+        pool_.reset();
+    }
+    // Where the wait for the buffer's work failed: nobody gets it, and hipFree waits.
+    void discard() {
+        if (p_) (void)hipFree(p_);
         p_ = nullptr;
         pool_.reset();
     }

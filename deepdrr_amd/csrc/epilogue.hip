@@ -129,6 +129,7 @@ extern "C" int drr_neglog(drr_ctx *ctx, const float *in, float *out, int n_image
     if (e != hipSuccess) rc = drr_hip_error(e, "drr_neglog setup");
     if (rc == DRR_OK) rc = drr_enqueue_neglog(in, out, segs, n_images, npix, keys, epsilon, st);
     e = hipStreamSynchronize(st);
+    if (e != hipSuccess) buf.discard();
     if (rc == DRR_OK && e != hipSuccess) rc = drr_hip_error(e, "drr_neglog");
     return rc;
 }

@@ -492,6 +492,10 @@ extern "C" int drr_mc_scatter(drr_ctx *ctx, const drr_volume *vol, const drr_mc_
     const int64_t n_bricks = (int64_t)bk.nb[0] * bk.nb[1] * bk.nb[2];
     float4 *maj = nullptr;
     hipError_t e = hipMallocAsync((void **)&maj, sizeof(float4) * n_bricks, st);
+    if (e == hipErrorOutOfMemory && DevPool::drop_all()) {
+        (void)hipGetLastError();
+        e = hipMallocAsync((void **)&maj, sizeof(float4) * n_bricks, st);
+    }
     if (e != hipSuccess) {
         if (prev >= 0 && prev != ctx->device) (void)hipSetDevice(prev);
         return drr_hip_error(e, "hipMallocAsync(brick majorants)");

@@ -328,13 +328,13 @@ extern "C" int drr_mesh_create(drr_ctx *ctx, const float *vertices, int n_vertic
         }                                 \
     } while (0)
     if (m->n_nodes > 0) {
-        MCHK(hipMalloc(&m->d_nodes, sizeof(BvhNode) * nodes.size()));
-        MCHK(hipMalloc(&m->d_tris, sizeof(TriDev) * tris_sorted.size()));
+        MCHK(drr_device_malloc(&m->d_nodes, sizeof(BvhNode) * nodes.size()));
+        MCHK(drr_device_malloc(&m->d_tris, sizeof(TriDev) * tris_sorted.size()));
         MCHK(hipMemcpy(m->d_nodes, nodes.data(), sizeof(BvhNode) * nodes.size(), hipMemcpyHostToDevice));
         MCHK(hipMemcpy(m->d_tris, tris_sorted.data(), sizeof(TriDev) * tris_sorted.size(), hipMemcpyHostToDevice));
     }
     if (n_prims > 0) {
-        MCHK(hipMalloc(&m->d_prims, sizeof(PrimDev) * n_prims));
+        MCHK(drr_device_malloc(&m->d_prims, sizeof(PrimDev) * n_prims));
         MCHK(hipMemcpy(m->d_prims, pd.data(), sizeof(PrimDev) * n_prims, hipMemcpyHostToDevice));
     }
 #undef MCHK
@@ -754,9 +754,9 @@ extern "C" int drr_project_meshes(drr_ctx *ctx, const drr_volume *const *vols, c
         mesh->d_cnt = nullptr;
         mesh->d_add = nullptr;
         mesh->cap_pix = 0;
-        hipError_t e1 = hipMalloc(&mesh->d_iv, sizeof(float2) * (size_t)K * npix);
-        hipError_t e2 = hipMalloc(&mesh->d_cnt, sizeof(int32_t) * npix);
-        hipError_t e3 = classes ? hipMalloc(&mesh->d_add, sizeof(float) * (size_t)classes * npix) : hipSuccess;
+        hipError_t e1 = drr_device_malloc(&mesh->d_iv, sizeof(float2) * (size_t)K * npix);
+        hipError_t e2 = drr_device_malloc(&mesh->d_cnt, sizeof(int32_t) * npix);
+        hipError_t e3 = classes ? drr_device_malloc(&mesh->d_add, sizeof(float) * (size_t)classes * npix) : hipSuccess;
         if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) {
             (void)hipFree(mesh->d_iv);
             (void)hipFree(mesh->d_cnt);

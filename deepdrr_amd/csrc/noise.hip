@@ -149,6 +149,7 @@ extern "C" int drr_add_noise(drr_ctx *ctx, const float *intensity, const float *
     k_correlate<<<(unsigned)blocks, 256, 0, st>>>(intensity, shot, out, n_images, height, width);
     hipError_t e = hipGetLastError();
     hipError_t e2 = hipStreamSynchronize(st);
+    if (e2 != hipSuccess) buf.discard();
     if (prev >= 0 && prev != ctx->device) (void)hipSetDevice(prev);
     if (e != hipSuccess) return drr_hip_error(e, "drr_add_noise launch");
     if (e2 != hipSuccess) return drr_hip_error(e2, "drr_add_noise");

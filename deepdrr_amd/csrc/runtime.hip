@@ -55,7 +55,7 @@ struct DevBuf {
     T *as() const {
         return static_cast<T *>(p);
     }
-    hipError_t alloc(size_t bytes) { return hipMalloc(&p, bytes); }
+    hipError_t alloc(size_t bytes) { return drr_device_malloc(&p, bytes); }
 };
 
 }  // namespace
@@ -146,9 +146,9 @@ int drr_ctx_set_spectrum(drr_ctx *ctx, int n_bins, const float *energies_keV, co
     (void)hipFree(ctx->d_mu);
     ctx->d_energies = ctx->d_pdf = ctx->d_mu = nullptr;
     ctx->n_bins = 0;
-    DRR_HIP_CHECK(hipMalloc(&ctx->d_energies, sizeof(float) * n_bins));
-    DRR_HIP_CHECK(hipMalloc(&ctx->d_pdf, sizeof(float) * n_bins));
-    DRR_HIP_CHECK(hipMalloc(&ctx->d_mu, sizeof(float) * n_bins * M));
+    DRR_HIP_CHECK(drr_device_malloc(&ctx->d_energies, sizeof(float) * n_bins));
+    DRR_HIP_CHECK(drr_device_malloc(&ctx->d_pdf, sizeof(float) * n_bins));
+    DRR_HIP_CHECK(drr_device_malloc(&ctx->d_mu, sizeof(float) * n_bins * M));
     DRR_HIP_CHECK(hipMemcpy(ctx->d_energies, energies_keV, sizeof(float) * n_bins, hipMemcpyHostToDevice));
     DRR_HIP_CHECK(hipMemcpy(ctx->d_pdf, pdf, sizeof(float) * n_bins, hipMemcpyHostToDevice));
     DRR_HIP_CHECK(hipMemcpy(ctx->d_mu, mu_over_rho, sizeof(float) * n_bins * M, hipMemcpyHostToDevice));
@@ -259,10 +259,12 @@ int drr_volume_create(drr_ctx *ctx, const float *density, const uint8_t *labels,
     if (rc == DRR_OK) {
         // either waits for the expansion
         hipError_t e = on_device ? hipMemcpy(&h_bad, d_bad, sizeof(h_bad), hipMemcpyDeviceToHost) : hipDeviceSynchronize();
-        if (e != hipSuccess)
+        if (e != hipSuccess) {
+            bad.discard();
             rc = drr_hip_error(e, "drr_volume_create: expand");
-        else if (h_bad)
+        } else if (h_bad) {
             rc = drr_set_error(DRR_ERR_INVALID, "drr_volume_create: label >= n_materials");
+        }
     }
     if (rc != DRR_OK) {
         if (v) drr_volume_destroy(v);
@@ -326,7 +328,7 @@ int drr_volume_destroy(drr_volume *vol) {
     if (!vol) return DRR_OK;
     DeviceGuard g(vol->device);
     // the cells go back to the pool: no launch may still read them
-    (void)hipDeviceSynchronize();
+    if (hipDeviceSynchronize() != hipSuccess) vol->cell_buf.discard();
     (void)hipFree(vol->lin_vox);
     delete vol;
     return DRR_OK;
@@ -372,8 +374,8 @@ int drr_volume_ensure_linear(drr_volume *vol) {
     const int64_t n = (int64_t)vol->nx * vol->ny * vol->nz;
     uint2 *vox = nullptr;
     unsigned int *d_max = nullptr;
-    hipError_t e = hipMalloc(&vox, sizeof(uint2) * n);
-    if (e == hipSuccess) e = hipMalloc(&d_max, sizeof(unsigned int));
+    hipError_t e = drr_device_malloc(&vox, sizeof(uint2) * n);
+    if (e == hipSuccess) e = drr_device_malloc(&d_max, sizeof(unsigned int));
     if (e == hipSuccess) e = hipMemset(d_max, 0, sizeof(unsigned int));
     if (e == hipSuccess) {
         k_voxels<<<2048, 256, 0, 0>>>(vol->cells, vol->nx, vol->ny, vol->nz, vox, d_max);

@@ -132,6 +132,10 @@ int drr_volume_create_from_hu(drr_ctx *ctx, const int16_t *hu, int nx, int ny, i
                               int on_device, int n_classes, const float *upper_hu,
                               const uint8_t *label_of_class, drr_volume **out);
 
+/* Waits for the device.  One destroyed volume's cells of up to 2 GB stay with the
+ * context for its next volume of that size; they are freed with the context, when
+ * a volume of another size is made, or when an allocation of this library finds no
+ * memory (other allocators of the process do not get them). */
 int drr_volume_destroy(drr_volume *vol);
 
 /* Copy the volume's float32 density and uint8 labels back ([nz][ny][nx], host). */
