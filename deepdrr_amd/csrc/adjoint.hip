@@ -157,7 +157,7 @@ struct UpToSlab {
 // ---- pass 2 of one ray as a resumable state -------------------------------------
 
 // The second march of one ray: the same samples as march_v1 (same alpha
-// sequence, same label cache), scattering G_t w_d(p_t) into the cell's 8
+// sequence, labels of the sample's cell), scattering G_t w_d(p_t) into the cell's 8
 // corner sums, handed to a deposit target whenever the ray leaves a cell
 // (and on request), and accumulating the pose sums S0, S1.  `run` stops
 // before the first sample whose cell fails a predicate on its coordinate
@@ -179,11 +179,9 @@ struct AdjRay {
     // Pose sums S0 = sum_t dL/dp_t, S1 = sum_t (alpha_t - aref) dL/dp_t, in FP64
     // (thousands of terms of both signs), in registers.  Within a cell, dL/dp_t =
     // G_t grad(rho)(p_t) [+ wt rho_t grad(h)(p_t) if the labels differ, h_d =
-    // dL/d(ad_raw) of corner d's material].  In a one-label cell grad(rho) along
-    // an axis is bilinear in the other two, a quadratic along the ray, which
-    // cell_sums adds in closed form; elsewhere, along x, it is sum_yz (D[1yz] -
-    // D[0yz]) w_yz, so sum_t G_t grad_x(rho) = sum_yz (D[1yz] - D[0yz]) (a[0yz] +
-    // a[1yz]) with a = sum_t G_t w (w_0yz + w_1yz = w_yz).
+    // dL/d(ad_raw) of corner d's material].  Along an axis grad(rho), and grad(h),
+    // is bilinear in the other two, a quadratic along the ray, which cell_sums adds
+    // in closed form: in FP32 over a cell's samples, then to these.
     double S[6];
 
     __device__ __forceinline__ void add_S(int k, double v) { S[k] += v; }
@@ -198,8 +196,8 @@ struct AdjRay {
         for (int d = 0; d < 8; d++) h[d] = get_m<M>(graw, (int)corner_label(c.l0, c.l1, d));
     }
 
-    // Ray setup and the steps before the volume (skip, then the window that
-    // re-establishes the label cache), exactly as march_v1.
+    // Ray setup and the steps before the volume: march_v1's, except that those of
+    // the last voxel before it open the cells they pass (which sum nothing there).
     __device__ __forceinline__ void begin(const Geo1 &g, const VolDev &vol, int udx, int vdx, float step,
                                           const float (&gr)[M]) {
 #pragma unroll
@@ -228,7 +226,7 @@ struct AdjRay {
             const float py = sample_pos(sy, alpha, riy);
             const float pz = sample_pos(sz, alpha, riz);
             const float bx = floorf(px), by = floorf(py), bz = floorf(pz);
-            if (!c.have || bx != c.bx || by != c.by || bz != c.bz) c.load(vol, px, py, pz, bx, by, bz);
+            if (!c.have || bx != c.bx || by != c.by || bz != c.bz) c.load(vol, bx, by, bz);
             alpha += step;
             ++t;
         }

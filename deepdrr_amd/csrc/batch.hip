@@ -288,8 +288,8 @@ static void launch_march(const JobTable &t, int M, bool atten, int march, int tw
     }
 }
 
-// Jobs over 2..4 volumes: one 8x8-pixel tile per wave, the literal
-// multi-volume march (march_multi, as drr_project runs such a view).
+// Jobs over 2..4 volumes: one 8x8-pixel tile per wave, the multi-volume march
+// (march_multi, as drr_project runs such a view).
 template <int V, int M>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI_WAVES))) void k_batch_multi(const JobMultiDev *__restrict__ jobs, const int2 *__restrict__ items,
                                                      int64_t n_items, SpectrumDev sp, float step, int atten, int air,

@@ -52,30 +52,6 @@ inline int march_v1_mode(const drr_ctx *ctx, int march) {
     return ctx->single_sums ? MARCH_V1_SINGLE : MARCH_V1_FAST;
 }
 inline int march_v1_mode(const drr_ctx *ctx) { return march_v1_mode(ctx, ctx->scene.march); }
-// Coefficients of the trilinear interpolant of corner values (v0 = corners
-// 0..3, v1 = 4..7, corner d = dx + 2 dy + 4 dz) along the ray p(u) = p0 + u r
-// from fractions f = p0 - b: value(u) = ((k3 u + k2) u + k1) u + k0.
-__device__ __forceinline__ void cell_cubic(const float4 &v0, const float4 &v1, float fx, float fy, float fz,
-                                           float rx, float ry, float rz, float &k0, float &k1, float &k2,
-                                           float &k3) {
-    // x: e_yz(u) = A_yz + B_yz u, the lerp of corners (0yz, 1yz)
-    const float X00 = v0.y - v0.x, X10 = v0.w - v0.z, X01 = v1.y - v1.x, X11 = v1.w - v1.z;
-    const float A00 = __builtin_fmaf(fx, X00, v0.x), A10 = __builtin_fmaf(fx, X10, v0.z);
-    const float A01 = __builtin_fmaf(fx, X01, v1.x), A11 = __builtin_fmaf(fx, X11, v1.z);
-    const float B00 = rx * X00, B10 = rx * X10, B01 = rx * X01, B11 = rx * X11;
-    // y: g_z(u) = G_z0 + G_z1 u + G_z2 u^2
-    const float P0 = A10 - A00, Q0 = B10 - B00, P1 = A11 - A01, Q1 = B11 - B01;
-    const float G00 = __builtin_fmaf(fy, P0, A00), G01 = __builtin_fmaf(fy, Q0, __builtin_fmaf(ry, P0, B00));
-    const float G02 = ry * Q0;
-    const float G10 = __builtin_fmaf(fy, P1, A01), G11 = __builtin_fmaf(fy, Q1, __builtin_fmaf(ry, P1, B01));
-    const float G12 = ry * Q1;
-    // z: the cubic
-    const float D0 = G10 - G00, D1 = G11 - G01, D2 = G12 - G02;
-    k0 = __builtin_fmaf(fz, D0, G00);
-    k1 = __builtin_fmaf(fz, D1, __builtin_fmaf(rz, D0, G01));
-    k2 = __builtin_fmaf(fz, D2, __builtin_fmaf(rz, D1, G02));
-    k3 = rz * D2;
-}
 
 // Of a two-label cell (tw): the second label's share of the density at the sample
 // at al, at its FP32 position (that of the exact filter), by nested lerps of the
@@ -177,8 +153,8 @@ __device__ __forceinline__ void single_run(const VolDev &vol, LdsAccum &a, bool 
         uni = c.uni;
         const float fx = px - bx, fy = py - by, fz = pz - bz;
         // density = ((c3 u + c2) u + c1) u + c0
-        float c0, c1, c2, c3;
-        cell_cubic(c.d0, c.d1, fx, fy, fz, rix, riy, riz, c0, c1, c2, c3);
+        const Cubic fc = cell_cubic(c.d0.x, c.d0.y - c.d0.x, c.d0.z, c.d0.w - c.d0.z, c.d1.x, c.d1.y - c.d1.x,
+                                    c.d1.z, c.d1.w - c.d1.z, fx, fy, fz, rix, riy, riz);
         // per axis, the exit face is reached after fma(-f, j, h) steps with
         // j = 1 / (r step) and h = j going up, 0 going down (j = 0, h = +inf
         // where r = 0)
@@ -235,7 +211,7 @@ __device__ __forceinline__ void single_run(const VolDev &vol, LdsAccum &a, bool 
             }
         } else {
             for (int k = 0; k < ne; ++k) {
-                cur += __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(c3, u, c2), u, c1), u, c0);
+                cur += __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(fc.c3, u, fc.c2), u, fc.c1), u, fc.c0);
                 u += inc;
             }
         }
@@ -243,7 +219,7 @@ __device__ __forceinline__ void single_run(const VolDev &vol, LdsAccum &a, bool 
             alpha = a0;
             for (int k = 0; k < n; ++k) {
                 const float u = alpha - a0;
-                float rho = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(c3, u, c2), u, c1), u, c0);
+                float rho = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(fc.c3, u, fc.c2), u, fc.c1), u, fc.c0);
                 const float xq = second_share(c, alpha, sx, sy, sz, rix, riy, riz, v00, v10, v01, v11, e00, e10, e01, e11, rho, tw);
                 sq += xq;
                 cur += rho;
@@ -290,7 +266,8 @@ __device__ __forceinline__ void march_fast_single(const Geo1 &g, const VolDev &v
         const float lim = r.mnv - (1.0f / rdom + 2.0f * step);
         skip_steps(N, lim, step, alpha, t);
         if (ATTEN) air_steps(t, acc);
-        // Phase 2: approach window, label cache tracked as the reference does.
+        // Phase 2: the cells of the last voxel before the volume, from the last of
+        // which the first cell inside takes its first material (single_run).
         Cell c;
         while (t < N && alpha < r.mnv) {
             const float px = sample_pos(sx, alpha, rix);

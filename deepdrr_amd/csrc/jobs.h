@@ -24,7 +24,7 @@ struct JobDev {
     int64_t out_offset;
 };
 
-// A job over 2..4 volumes: the literal multi-volume march (priorities, the
+// A job over 2..4 volumes: the multi-volume march (march_multi: priorities, the
 // shared label cache) of the whole view, on 8x8-pixel wave tiles.
 struct JobMultiDev {
     ViewDev vd;

@@ -175,9 +175,6 @@ struct Cell {
         bz = z;
         have = true;
     }
-    __device__ __forceinline__ void load(const VolDev &vol, float, float, float, float x, float y, float z) {
-        load(vol, x, y, z);
-    }
 };
 
 // Running area density of the current uniform material: ad[cm] lives in
