@@ -384,8 +384,8 @@ struct AdjRay {
     // Cell by cell: every lane still marching hands over its open cell, takes the
     // cell of its current sample and sums that cell's samples together (one
     // execution of that long block for the whole wave).  The next cell's record
-    // is loaded before the present one is summed.  VALU issue bounds it (0.82 of
-    // the slots; one label 250 instructions, several 400 more).  64 views of 256^2
+    // is loaded before the present one is summed.  VALU issue bounds it (0.84 of
+    // the slots; one label 260 instructions, several 400 more).  64 views of 256^2
     // through 192^3: 28.6 ms with the samples of several labels one by one (91
     // instructions each), 22.5 in closed form, 16.9 with the box in FP64.
     template <class Dep, class Go>
@@ -631,7 +631,7 @@ __device__ __forceinline__ void ray_through(const float *W, float fu, float fv, 
 
 // Occupancy targets: waves per SIMD, also the blocks per CU that the launch keeps
 // resident.  64 views of 256^2 through 192^3: density alone 12.2 ms at 4 (122
-// registers; 5 spill 14), with the pose 16.9 ms at 3 (4 spill 39).  The
+// registers; 5 spill 14), with the pose 16.9 ms at 3 (which spill 20; 4 spill 39).  The
 // pose alone: 6.9 ms at 3, 7.7 at 4.
 template <int POSE>
 struct AdjOcc {

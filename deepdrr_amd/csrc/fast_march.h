@@ -37,8 +37,9 @@
 // votes as their tests and 0/1 factors as the lanes' choices, for the scalar
 // instructions that lanes' own branches take, a sample cost 7 vector
 // instructions in place of 5, one of two labels 39 in place of 30 for every lane
-// of the wave: 16 clinical views 85.5 ms, 73.3 now; 48 mixed 17.6, 16.5.)  The materials' sums live in LDS, one word per lane and
-// material: an entry reads and writes the words its labels name, which in
+// of the wave: 16 clinical views 85.5 ms, 73.3 after it (launches apart; back to
+// back 80 to 84); 48 mixed 17.6, 16.5.)  The materials' sums live in LDS, one word per lane and
+// label: an entry reads and writes the words its labels name, which in
 // registers takes a compare and a select per material and holds the
 // materials' registers and lane masks through the loop.  The record of the
 // cell after is loaded before the present one is summed: the wait for it was
@@ -69,7 +70,7 @@ constexpr float FAST_CLOSED_UNITS = 1024.0f;
 // bound where a cell has many (voxels of 20 mm at a step of 0.1: 9.4e-6 without,
 // 6.7e-6 with; of up to 6 mm it changes nothing).
 constexpr int FAST_CLOSED_SAMPLES = 64;
-// Waves per SIMD of the kernels that march fast: 87 registers hold the entry
+// Waves per SIMD of the kernels that march fast: 89 registers hold the entry
 // block and the record on its way (with 9 more, 6 waves spilled 16: 7.4 ms
 // against 5.7 on the clinical view; 4 waves: 5.7).
 constexpr int FAST_WAVES = 5;

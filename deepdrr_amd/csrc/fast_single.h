@@ -26,7 +26,7 @@
 // filter's formulas.  The sums stay within about 1e-7 relative of the exact
 // march's; nothing depends on the launch or on other lanes.
 //
-// VALU issue bounds it.  The sums live in LDS, one word per lane and material
+// VALU issue bounds it.  The sums live in LDS, one word per lane and label
 // (in registers the entry block took a compare and a select per material, and
 // their lane masks spilled 95 scalar registers through the loop), and a
 // sample's distance from the cell's first is k inc, with no alpha to follow:
